@@ -151,10 +151,12 @@ typedef i32x4 acc_t;
 #define TILES_N ((N + BN - 1) / BN)
 /* KP = K rounded up to a multiple of 64 (host checks KP % BK == 0); chunks
  * beyond K are zero-filled by the load predicate. When K is no multiple of 16
- * the rows of A and B are not 16-byte aligned and the last chunk of a row is
- * partly beyond it (those bytes are the next row's, not zeros): the chunk is
- * then put together from dword loads (K % 4 == 0) or byte loads, each with its
- * own predicate. Register-staged pipelines only. */
+ * the rows of A and B are not 16-byte aligned: a buffer load of 16 bytes needs
+ * dword alignment only, which is enough for K % 4 == 0; otherwise a chunk is cut
+ * out of the five dwords it lies in (one 128-bit and one 32-bit load, four
+ * byte-aligning shifts). The last chunk of a row is partly beyond it (those
+ * bytes are the next row's): they are zeroed in A on the way into LDS.
+ * Register-staged pipelines only. */
 #define KT (KP / BK / (SPLITK * WAVES_K))      /* tiles of one k-group (host checks divisibility) */
 #if EARLYST && (SPLITK > 1 || WAVES_K > 1)
 #error "early stores write finished sums: no K division"
@@ -285,48 +287,88 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
 
     /* raw buffer loads: an element that must read as zero (edge tile, idle
      * lane, K tail) gets an offset beyond the buffer and loads 0 */
+#if K % 4 == 0
+#define SHIFTED(p) (p)
+#define A_SPAN (M * K)
+#define B_SPAN (N * K)
+#else
+    /* Rows begin at any byte. The descriptors start at the dword the operand begins in, a chunk is
+     * loaded from the dword its first byte lies in, and the byte inside that dword (the same for every
+     * k tile, BK being a multiple of 4) becomes the shift. The spans are whole dwords: the last
+     * one may hold bytes behind the operand, which share its page and are never used. */
+#define SHIFTED(p) (const_cast<signed char*>(p) - ((unsigned long long)(p) & 3))
+#define A_SPAN ((int)(((unsigned)(M * K) + (unsigned)a_lsb + 3u) & ~3u))
+#define B_SPAN ((int)(((unsigned)(N * K) + (unsigned)b_lsb + 3u) & ~3u))
+    const int a_lsb = __builtin_amdgcn_readfirstlane((int)((unsigned long long)A & 3));
+    const int b_lsb = __builtin_amdgcn_readfirstlane((int)((unsigned long long)B & 3));
+#endif
     const __amdgpu_buffer_rsrc_t rsrc_a =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(A), 0, M * K, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(SHIFTED(A)), 0, A_SPAN, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(B), 0, N * K, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(SHIFTED(B)), 0, B_SPAN, 0x00020000);
     unsigned a_voff[EA], b_voff[EB];
+#if K % 4 == 0
+#define A_SHIFT(e) 0
+#define B_SHIFT(e) 0
+#else
+    int a_sh[EA], b_sh[EB];
+#define A_SHIFT(e) a_sh[e]
+#define B_SHIFT(e) b_sh[e]
+#endif
 #pragma unroll
     for (int e = 0; e < EA; ++e) {
         const int m = m0 + a_row[e];
         bool ok = (A_CHUNKS % NT == 0) || (tid + e * NT < A_CHUNKS);
         if (M % BM != 0) ok = ok && (m < M);
-        a_voff[e] = ok ? (unsigned)(m * K + a_col[e]) : OOB;
+#if K % 4 == 0
+        const unsigned off = (unsigned)(m * K + a_col[e]);
+#else
+        const unsigned byte = (unsigned)(m * K + a_col[e] + a_lsb), off = byte & ~3u;
+        a_sh[e] = (int)(byte & 3u);
+#endif
+        a_voff[e] = ok ? off : OOB;
     }
 #pragma unroll
     for (int e = 0; e < EB; ++e) {
         const int n = n0 + b_row[e];
         bool ok = (B_CHUNKS % NT == 0) || (tid + e * NT < B_CHUNKS);
         if (N % BN != 0) ok = ok && (n < N);
-        b_voff[e] = ok ? (unsigned)(n * K + b_col[e]) : OOB;
+#if K % 4 == 0
+        const unsigned off = (unsigned)(n * K + b_col[e]);
+#else
+        const unsigned byte = (unsigned)(n * K + b_col[e] + b_lsb), off = byte & ~3u;
+        b_sh[e] = (int)(byte & 3u);
+#endif
+        b_voff[e] = ok ? off : OOB;
     }
 
-    i32x4 areg[PD][EA], breg[PD][EB];
-
-    /* the 16 bytes k0 + col .. k0 + col + 15 of the row whose chunk offset is vo */
-    auto load_chunk = [&](__amdgpu_buffer_rsrc_t rsrc, unsigned vo, int k0, int col) -> i32x4 {
-#if K % 16 == 0
-        return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)vo, k0, 0));
-#elif K % 4 == 0
-        i32x4 v;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const unsigned o = (vo != OOB && k0 + col + 4 * d < K) ? vo + 4 * d : OOB;
-            v[d] = (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)o, k0, 0);
-        }
-        return v;
+    /* what a lane holds of a chunk between its load and its store to LDS */
+#if K % 4 == 0
+    typedef i32x4 chunk_t;
 #else
-        i32x4 v = (i32x4)(0);
-#pragma unroll
-        for (int b = 0; b < 16; ++b) {
-            const unsigned o = (vo != OOB && k0 + col + b < K) ? vo + b : OOB;
-            const unsigned byte = (unsigned)__builtin_amdgcn_raw_buffer_load_b8(rsrc, (int)o, k0, 0) & 0xffu;
-            v[b / 4] |= (int)(byte << (8 * (b % 4)));
-        }
+    struct chunk_t { i32x4 lo; int hi; };     /* the five dwords its 16 bytes lie in */
+#endif
+    chunk_t areg[PD][EA], breg[PD][EB];
+
+    auto load_chunk = [&](__amdgpu_buffer_rsrc_t rsrc, unsigned vo, int k0) -> chunk_t {
+        const i32x4 lo = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)vo, k0, 0));
+#if K % 4 == 0
+        return lo;
+#else
+        return {lo, (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)vo, k0 + 16, 0)};
+#endif
+    };
+    /* the chunk's 16 bytes; sh = byte the chunk begins at inside its first dword */
+    auto chunk_bytes = [&](const chunk_t& c, int sh) -> i32x4 {
+#if K % 4 == 0
+        (void)sh;
+        return c;
+#else
+        i32x4 v;
+        v[0] = (int)__builtin_amdgcn_alignbyte((unsigned)c.lo[1], (unsigned)c.lo[0], (unsigned)sh);
+        v[1] = (int)__builtin_amdgcn_alignbyte((unsigned)c.lo[2], (unsigned)c.lo[1], (unsigned)sh);
+        v[2] = (int)__builtin_amdgcn_alignbyte((unsigned)c.lo[3], (unsigned)c.lo[2], (unsigned)sh);
+        v[3] = (int)__builtin_amdgcn_alignbyte((unsigned)c.hi, (unsigned)c.lo[3], (unsigned)sh);
         return v;
 #endif
     };
@@ -337,25 +379,42 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
         for (int e = 0; e < EA; ++e) {
             unsigned vo = a_voff[e];
             if (KP != K) vo = (k0 + a_col[e] < K) ? vo : OOB;
-            areg[set][e] = load_chunk(rsrc_a, vo, k0, a_col[e]);
+            areg[set][e] = load_chunk(rsrc_a, vo, k0);
         }
 #pragma unroll
         for (int e = 0; e < EB; ++e) {
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_col[e] < K) ? vo : OOB;
-            breg[set][e] = load_chunk(rsrc_b, vo, k0, b_col[e]);
+            breg[set][e] = load_chunk(rsrc_b, vo, k0);
         }
     };
 
-    auto store_lds = [&](int buf, int set) {
+    /* tile kt, which register set `set` holds, to LDS buffer buf */
+    auto store_lds = [&](int kt, int buf, int set) {
+        const int k0 = kbase + kt * BK;
 #pragma unroll
         for (int e = 0; e < EA; ++e)
-            if ((A_CHUNKS % NT == 0) || (tid + e * NT < A_CHUNKS))
-                *reinterpret_cast<i32x4*>(&As[buf][a_row[e] * SROW + PCOL(a_row[e], a_col[e])]) = areg[set][e];
+            if ((A_CHUNKS % NT == 0) || (tid + e * NT < A_CHUNKS)) {
+                i32x4 v = chunk_bytes(areg[set][e], A_SHIFT(e));
+#if K % 16 != 0
+                /* the last chunk of a row runs into the next row: those bytes of A become zeros, and
+                 * whatever B holds there does not count */
+                if (k0 + BK > K) {
+                    const int valid = K - k0 - a_col[e];         /* bytes of the chunk inside the row */
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const int nb = valid - 4 * d;
+                        v[d] = nb >= 4 ? v[d] : (nb <= 0 ? 0 : v[d] & ((1 << (8 * nb)) - 1));
+                    }
+                }
+#endif
+                *reinterpret_cast<i32x4*>(&As[buf][a_row[e] * SROW + PCOL(a_row[e], a_col[e])]) = v;
+            }
 #pragma unroll
         for (int e = 0; e < EB; ++e)
             if ((B_CHUNKS % NT == 0) || (tid + e * NT < B_CHUNKS))
-                *reinterpret_cast<i32x4*>(&Bs[buf][b_row[e] * SROW + PCOL(b_row[e], b_col[e])]) = breg[set][e];
+                *reinterpret_cast<i32x4*>(&Bs[buf][b_row[e] * SROW + PCOL(b_row[e], b_col[e])]) =
+                    chunk_bytes(breg[set][e], B_SHIFT(e));
     };
 
     acc_t acc[REP_M][REP_N];
@@ -677,14 +736,14 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
         };
         i32x4 fa[REP_M], fb[REP_N];
         load_global(0, 0);
-        store_lds(0, 0);
+        store_lds(0, 0, 0);
         if (KT > 1) load_global(1, 0);
         __syncthreads();
         load_frags(0, 0, fa, fb);
         for (int kt = 0; kt < KT; ++kt) {
             const int cur = kt & 1;
             if (kt + 1 < KT) {
-                store_lds(cur ^ 1, 0);                 /* tile kt+1, loaded during iteration kt-1 */
+                store_lds(kt + 1, cur ^ 1, 0);         /* tile kt+1, loaded during iteration kt-1 */
                 __builtin_amdgcn_sched_barrier(0);
                 if (kt + 2 < KT) load_global(kt + 2, 0);
                 __builtin_amdgcn_sched_barrier(0);
@@ -718,7 +777,7 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
 #pragma unroll
     for (int p = 0; p < PD; ++p)
         if (p < KT) load_global(p, p);
-    store_lds(0, 0);
+    store_lds(0, 0, 0);
     __syncthreads();
     for (int kt0 = 0; kt0 < KT; kt0 += PD) {
 #pragma unroll
@@ -732,7 +791,7 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
                 __builtin_amdgcn_sched_barrier(0);
                 compute(cur);
                 if (STAGES == 1) __syncthreads();
-                if (kt + 1 < KT) store_lds((STAGES == 2) ? (cur ^ 1) : 0, (u + 1) % PD);
+                if (kt + 1 < KT) store_lds(kt + 1, (STAGES == 2) ? (cur ^ 1) : 0, (u + 1) % PD);
                 __syncthreads();
             }
         }
