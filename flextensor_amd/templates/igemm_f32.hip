@@ -336,6 +336,14 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 #endif
 
+/* Rows along K whose length is no multiple of 4: 16-byte loads need dword alignment only, so the vectors
+ * stay, but the last one of a row runs into the next row (or, behind the last row, beyond the buffer,
+ * where each dword reads as zero by itself). Those elements are zeroed: a product with the zeros of
+ * the other operand would not be zero for an infinity or a NaN. Vectors along M or N that run beyond a row
+ * only feed results that are not stored. */
+#define A_TAIL (!TA && AV == 4 && K % 4 != 0)
+#define B_TAIL (MODE == 2 && BV == 4 && K % 4 != 0)
+
 #if AV == 4
 typedef f32x4 avec_t;
 #elif AV == 1
@@ -802,6 +810,31 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
         dma_tile_a(kt, buf, part, nparts);
         dma_tile_b(kt, buf, part, nparts);
     };
+    /* zeroes what the loads of tile kt fetched from beyond the rows' ends. Every lane mends the chunks it
+     * requested itself, so its wavefront's wait for the loads goes before and the barrier behind. */
+    auto mend_tail = [&](int kt, int buf) {
+#if A_TAIL || B_TAIL
+        const int k0 = kbase + kt * BK;
+        if (k0 + BK > K) {
+#if A_TAIL
+#pragma unroll
+            for (int e = 0; e < EA; ++e)
+#pragma unroll
+                for (int i = 1; i < 4; ++i)
+                    if (k0 + a_col[e] < K && k0 + a_col[e] + i >= K && ((A_CHUNKS % NT == 0) || (tid + e * NT < A_CHUNKS)))
+                        As[buf][(e * NT + tid) * 4 + i] = 0.0f;
+#endif
+#if B_TAIL
+#pragma unroll
+            for (int e = 0; e < EB; ++e)
+#pragma unroll
+                for (int i = 1; i < 4; ++i)
+                    if (k0 + b_col[e] < K && k0 + b_col[e] + i >= K && ((B_CHUNKS % NT == 0) || (tid + e * NT < B_CHUNKS)))
+                        Bs[buf][(e * NT + tid) * 4 + i] = 0.0f;
+#endif
+        }
+#endif
+    };
 #endif
     /* Every offset below is computed for all lanes and then chosen against the out-of-range
      * constant: a select of two values, never "compute it if in range". The second form becomes a
@@ -933,7 +966,26 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
         }
     };
 
-    auto store_lds = [&](int buf, int set) {
+    auto store_lds = [&](int kt, int buf, int set) {
+#if A_TAIL || B_TAIL
+        const int k0 = kbase + kt * BK;
+        if (k0 + BK > K) {            /* the chunks that run beyond their row's end */
+#if A_TAIL
+#pragma unroll
+            for (int e = 0; e < EA; ++e)
+#pragma unroll
+                for (int i = 1; i < 4; ++i)
+                    if (k0 + a_col[e] + i >= K) areg[set][e][i] = 0.0f;
+#endif
+#if B_TAIL
+#pragma unroll
+            for (int e = 0; e < EB; ++e)
+#pragma unroll
+                for (int i = 1; i < 4; ++i)
+                    if (k0 + b_col[e] + i >= K) breg[set][e][i] = 0.0f;
+#endif
+        }
+#endif
 #pragma unroll
         for (int e = 0; e < EA; ++e) {
             if ((A_CHUNKS % NT == 0) || (tid + e * NT < A_CHUNKS)) {
@@ -1075,11 +1127,12 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #if DTL
     /* tile 0 was requested above, as early as its addresses were known */
     __builtin_amdgcn_s_waitcnt(0x0F70);      /* vmcnt(0): this wavefront's part of tile 0 is in LDS */
+    mend_tail(0, 0);
 #else
 #pragma unroll
     for (int p = 0; p < PD; ++p)
         if (p < nk) load_global(p, p);
-    store_lds(0, 0);
+    store_lds(0, 0, 0);
 #endif
 #if SK_PER > 0
     /* The arrival for the slot written at the end of the previous segment is
@@ -1118,6 +1171,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
             else if (behind == 1) VMCNT(DMA_PER_TILE);
 #endif
             else VMCNT(0);
+            if (kt + 1 < nk) mend_tail(kt + 1, cur + 1 == STAGES ? 0 : cur + 1);
             __syncthreads();
             cur = (cur + 1 == STAGES) ? 0 : cur + 1;
             nxt = (nxt + 1 == STAGES) ? 0 : nxt + 1;
@@ -1147,6 +1201,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
                 if (blk + 1 < BK / KBLK) read_block(cur, (blk + 1) * KBLK, a[(blk + 1) & 1], b[(blk + 1) & 1]);
                 if (blk == BK / KBLK - 1) {
                     __builtin_amdgcn_s_waitcnt(0x0070);      /* vmcnt(0), lgkmcnt(0) */
+                    if (kt + 1 < nk) mend_tail(kt + 1, cur ^ 1);
                     __syncthreads();
                     /* after the last tile this reads stale data that nothing uses */
                     read_block(cur ^ 1, 0, na, nb);
@@ -1172,6 +1227,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
         if (kt + 1 < nk) dma_tile(kt + 1, cur ^ 1);      /* lands while tile kt is multiplied */
         compute(cur);
         __builtin_amdgcn_s_waitcnt(0x0F70);
+        if (kt + 1 < nk) mend_tail(kt + 1, cur ^ 1);
         __syncthreads();
     }
 #else
@@ -1187,7 +1243,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
                 __builtin_amdgcn_sched_barrier(0);
                 compute(cur);
                 if (STAGES == 1) __syncthreads();
-                if (kt + 1 < nk) store_lds((STAGES == 2) ? (cur ^ 1) : 0, (u + 1) % PD);
+                if (kt + 1 < nk) store_lds(kt + 1, (STAGES == 2) ? (cur ^ 1) : 0, (u + 1) % PD);
                 __syncthreads();
             }
         }

@@ -16,6 +16,39 @@ def build_default(func, category, args):
     return build_plan(s, bufs, "rocm"), bufs
 
 
+def gemm_of(trans_b, batch=0):
+    """fp32 GEMM task function (M, K, N) -> (ops, bufs), B stored [N][K] with ``trans_b``."""
+    def func(m, k, n):
+        from flextensor_amd import nn
+        from flextensor_amd.te import placeholder
+        lead = (batch,) if batch else ()
+        a, b = placeholder(lead + (m, k), name="A"), placeholder(lead + ((n, k) if trans_b else (k, n)), name="B")
+        c = (nn.batch_gemm if batch else nn.gemm)(a, b, transposeB=trans_b)
+        return [c.op], [a, b, c]
+    return func
+
+
+def build_config(func, args, config):
+    from flextensor_amd.plan import build as build_plan
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.utils import Config
+    ops, bufs = func(*args)
+    s, bufs = schedule_with_config_ops(ops, bufs, Config([config] if config else [], None))
+    return build_plan(s, bufs, "rocm"), bufs
+
+
+def gemm_config(m, k, n, wm, wn, rep, mfma, bk, depth, groups=1):
+    cd = lambda a, b: -(-a // b)
+    return dict(spatial=[[cd(m, wm * rep * mfma), wm, rep, mfma], [cd(n, wn * rep * mfma), wn, rep, mfma]],
+                reduce=[[groups, cd(k, groups * bk), bk]], unroll=[[depth, 1]], fuse=[[4]],
+                reorder=[[1, 1 if groups > 1 else 0, 0]], inline=[], merge=[], special=[])
+
+
+def close(got, want):
+    """The fp32 bound of the product's own gate: max|diff| / max|ref| <= 1e-5."""
+    return float(np.max(np.abs(got - want)) / np.max(np.abs(want))) <= 1e-5
+
+
 def placed(array, offset=0):
     """A contiguous device tensor of ``array`` that begins ``offset`` elements behind an allocation's start."""
     import torch
@@ -42,3 +75,56 @@ def test_int8_rows_at_any_byte(oracle, m, k, n):
         c = torch.full((m, n), -7, dtype=torch.int32, device="cuda")
         f(placed(a, oa), placed(b, ob), c)
         assert np.array_equal(c.cpu().numpy(), want), (oa, ob)
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("m,k,n", [
+    (1, 1, 1), (5, 3, 2), (3, 5, 4), (17, 33, 19), (64, 30, 65), (33, 17, 70), (130, 130, 258), (127, 129, 126),
+    (30, 999, 611), (201, 77, 131), (513, 67, 259), (1030, 35, 1027)])
+def test_fp32_rows_of_any_length(oracle, m, k, n, trans_b):
+    """Default plans at extents that are no multiples of a vector, a tile or a k block."""
+    import torch
+    rng = np.random.default_rng(m + 3 * k + 7 * n)
+    a, b = [rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n))]
+    f, _ = build_config(gemm_of(trans_b), (m, k, n), None)
+    c = torch.full((m, n), -7.0, device="cuda")
+    f(placed(a, 1), placed(np.ascontiguousarray(b.T) if trans_b else b, 3), c)
+    assert close(c.cpu().numpy(), oracle.gemm_f32_c(a, b))
+
+
+@pytest.mark.parametrize("depth,bk,mfma,groups", [(1, 16, 16, 1), (2, 16, 32, 2), (3, 32, 16, 1), (4, 16, 16, 1), (5, 32, 16, 1),
+                                                  (5, 32, 32, 2), (6, 32, 16, 1), (7, 32, 16, 1), (8, 32, 16, 1), (8, 32, 32, 1)])
+@pytest.mark.parametrize("k", [61, 62, 63, 109, 127])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_what_a_row_takes_from_the_next_one_does_not_count(depth, bk, mfma, groups, k, trans_b):
+    """The last vector of a row along K runs into the next row on every pipeline: an infinity or a NaN that
+    begins that row must not reach the row before it (0 * inf is not 0)."""
+    import torch
+    m, n = 70, 66
+    rng = np.random.default_rng(k)
+    a, b = [rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n))]
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    a[5, :3] = [np.inf, np.nan, np.inf]
+    f, _ = build_config(gemm_of(trans_b), (m, k, n), gemm_config(m, k, n, 2, 2, 1, mfma, bk, depth, groups))
+    for spoil_b in (False, True) if trans_b else (False,):
+        bb = b.copy()
+        if spoil_b:
+            bb[:3, 9] = [np.nan, np.inf, np.inf]
+        c = torch.full((m, n), -7.0, device="cuda")
+        f(placed(a), placed(np.ascontiguousarray(bb.T) if trans_b else bb), c)
+        got = c.cpu().numpy()
+        rows, cols = np.arange(m) != 5, np.arange(n) != (9 if spoil_b else -1)
+        assert not np.isfinite(got[5]).any()
+        assert close(got[rows][:, cols], want[rows][:, cols]), (depth, k, spoil_b)
+
+
+@pytest.mark.parametrize("b,m,k,n,trans_b", [(3, 49, 33, 50, True), (5, 17, 31, 18, False), (70, 197, 64, 31, True),
+                                             (9, 128, 129, 127, False)])
+def test_batched_products_of_odd_extents(b, m, k, n, trans_b):
+    import torch
+    rng = np.random.default_rng(b + m)
+    x, y = [rng.uniform(-1, 1, s).astype(np.float32) for s in ((b, m, k), (b, k, n))]
+    f, _ = build_config(gemm_of(trans_b, batch=b), (m, k, n), None)
+    c = torch.full((b, m, n), -7.0, device="cuda")
+    f(placed(x), placed(np.ascontiguousarray(y.transpose(0, 2, 1)) if trans_b else y), c)
+    assert close(c.cpu().numpy(), np.matmul(x.astype(np.float64), y.astype(np.float64)))
