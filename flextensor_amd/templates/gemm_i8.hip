@@ -158,6 +158,14 @@ typedef i32x4 acc_t;
  * bytes are the next row's): they are zeroed in A on the way into LDS.
  * Register-staged pipelines only. */
 #define KT (KP / BK / (SPLITK * WAVES_K))      /* tiles of one k-group (host checks divisibility) */
+/* K offset of a tile that goes into the scalar offset of its loads. The range check of a buffer load compares
+ * the lane's offset with (bytes - scalar offset): a scalar offset beyond the buffer would wrap that difference
+ * and let every lane pass. A tile wholly behind K (its lanes are all out of range) therefore takes 0. */
+#if KP - K >= BK
+#define K_AT(k0) ((k0) < K ? (k0) : 0)
+#else
+#define K_AT(k0) (k0)
+#endif
 #if EARLYST && (SPLITK > 1 || WAVES_K > 1)
 #error "early stores write finished sums: no K division"
 #endif
@@ -351,11 +359,11 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
     chunk_t areg[PD][EA], breg[PD][EB];
 
     auto load_chunk = [&](__amdgpu_buffer_rsrc_t rsrc, unsigned vo, int k0) -> chunk_t {
-        const i32x4 lo = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)vo, k0, 0));
+        const i32x4 lo = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)vo, K_AT(k0), 0));
 #if K % 4 == 0
         return lo;
 #else
-        return {lo, (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)vo, k0 + 16, 0)};
+        return {lo, (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(vo + 16u), K_AT(k0), 0)};
 #endif
     };
     /* the chunk's 16 bytes; sh = byte the chunk begins at inside its first dword */
@@ -535,13 +543,13 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
             for (int e = 0; e < EA; ++e) {
                 unsigned vo = a_voff[e];
                 if (KP != K) vo = (k0 + a_col[e] < K) ? vo : OOB;
-                dma16(ra, &As[buf][(e * NT + wv * 64) * 16], vo, k0);
+                dma16(ra, &As[buf][(e * NT + wv * 64) * 16], vo, K_AT(k0));
             }
 #pragma unroll
             for (int e = 0; e < EB; ++e) {
                 unsigned vo = b_voff[e];
                 if (KP != K) vo = (k0 + b_col[e] < K) ? vo : OOB;
-                dma16(rb, &Bs[buf][(e * NT + wv * 64) * 16], vo, k0);
+                dma16(rb, &Bs[buf][(e * NT + wv * 64) * 16], vo, K_AT(k0));
             }
         };
         dma_tile(0, 0);
@@ -578,11 +586,11 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
             if (e < EA) {
                 unsigned vo = a_voff[e];
                 if (KP != K) vo = (k0 + a_col[e] < K) ? vo : OOB;
-                dma16(ra, &As[buf][(e * NT + wv * 64) * 16], vo, k0);
+                dma16(ra, &As[buf][(e * NT + wv * 64) * 16], vo, K_AT(k0));
             } else {
                 unsigned vo = b_voff[e - EA];
                 if (KP != K) vo = (k0 + b_col[e - EA] < K) ? vo : OOB;
-                dma16(rb, &Bs[buf][((e - EA) * NT + wv * 64) * 16], vo, k0);
+                dma16(rb, &Bs[buf][((e - EA) * NT + wv * 64) * 16], vo, K_AT(k0));
             }
         };
         /* one tile; NEXT: tile kt+1 exists (its fragments are fetched), NEXT2: tile kt+2 exists */

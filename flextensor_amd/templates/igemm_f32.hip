@@ -235,6 +235,14 @@ typedef f32x4 acc_t;
 #define KSPLIT_LEN (KP / SPLITK)
 #define KGROUP_LEN (KSPLIT_LEN / WAVES_K)
 #define KT (KGROUP_LEN / BK)
+/* K offset of a tile that goes into the scalar offset of its loads. The range check of a buffer load compares
+ * the lane's offset with (bytes - scalar offset): a scalar offset beyond the buffer would wrap that difference
+ * and let every lane pass. A tile wholly behind K (its lanes are all out of range) therefore takes 0. */
+#if KP - K >= BK
+#define K_AT(k0) ((k0) < K ? (k0) : 0)
+#else
+#define K_AT(k0) (k0)
+#endif
 
 #if BK % KBLK != 0
 #error "BK must be a multiple of 4*(64/MFMA)"
@@ -754,11 +762,11 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #if TA
             if (KP != K) vo = (k0 + a_row[e] < K) ? vo : OOB;
             if ((A_CHUNKS % NT == 0) || (e * NT + wv * 64 < A_CHUNKS))
-                dma16(desc_a, &As[buf][(e * NT + wv * 64) * 4], vo, k0 * (M * 4));
+                dma16(desc_a, &As[buf][(e * NT + wv * 64) * 4], vo, K_AT(k0) * (M * 4));
 #else
             if (KP != K) vo = (k0 + a_col[e] < K) ? vo : OOB;
             if ((A_CHUNKS % NT == 0) || (e * NT + wv * 64 < A_CHUNKS))     /* whole wavefronts only */
-                dma16(desc_a, &As[buf][(e * NT + wv * 64) * 4], vo, k0 * 4);
+                dma16(desc_a, &As[buf][(e * NT + wv * 64) * 4], vo, K_AT(k0) * 4);
 #endif
         }
     };
@@ -769,7 +777,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #if MODE == 2
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_col[e] < K) ? vo : OOB;
-            dma16(desc_b, &Bs[buf][(e * NT + wv * 64) * 4], vo, k0 * 4);
+            dma16(desc_b, &Bs[buf][(e * NT + wv * 64) * 4], vo, K_AT(k0) * 4);
 #else
             /* the wavefront's 64 lanes are 64 consecutive columns of one k row */
             const int q0 = e * NT + wv * 64;
@@ -777,15 +785,15 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #if MODE == 0 && defined(BSWZ)
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_row[e] < K) ? vo : OOB;
-            dma16(desc_b, &Bs[buf][(e * NT + wv * 64) * 4], vo, k0 * (N * 4));
+            dma16(desc_b, &Bs[buf][(e * NT + wv * 64) * 4], vo, K_AT(k0) * (N * 4));
 #elif MODE == 0
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_row[e] < K) ? vo : OOB;
-            dma4(desc_b, dst, vo, k0 * (N * 4));
+            dma4(desc_b, dst, vo, K_AT(k0) * (N * 4));
 #elif KHOIST
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_row[e] < K) ? vo : OOB;
-            dma4(desc_b, dst, vo, (k0 / (CR * CS)) * (CH * CW * 4));
+            dma4(desc_b, dst, vo, (K_AT(k0) / (CR * CS)) * (CH * CW * 4));
 #else
             const int k = k0 + b_row[e];
             const int c = k / (CR * CS);
@@ -931,10 +939,10 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
             unsigned vo = a_voff[e];
 #if TA
             if (KP != K) vo = (k0 + a_row[e] < K) ? vo : OOB;
-            areg[set][e] = LOAD_A(rsrc_a, vo, k0 * (M * 4));
+            areg[set][e] = LOAD_A(rsrc_a, vo, K_AT(k0) * (M * 4));
 #else
             if (KP != K) vo = (k0 + a_col[e] < K) ? vo : OOB;
-            areg[set][e] = LOAD_A(rsrc_a, vo, k0 * 4);
+            areg[set][e] = LOAD_A(rsrc_a, vo, K_AT(k0) * 4);
 #endif
         }
 #pragma unroll
@@ -942,15 +950,15 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #if MODE == 2
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_col[e] < K) ? vo : OOB;
-            breg[set][e] = LOAD_B(rsrc_b, vo, k0 * 4);
+            breg[set][e] = LOAD_B(rsrc_b, vo, K_AT(k0) * 4);
 #elif MODE == 0
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_row[e] < K) ? vo : OOB;
-            breg[set][e] = LOAD_B(rsrc_b, vo, k0 * (N * 4));
+            breg[set][e] = LOAD_B(rsrc_b, vo, K_AT(k0) * (N * 4));
 #elif KHOIST
             unsigned vo = b_voff[e];
             if (KP != K) vo = (k0 + b_row[e] < K) ? vo : OOB;
-            breg[set][e] = LOAD_B(rsrc_b, vo, (k0 / (CR * CS)) * (CH * CW * 4));
+            breg[set][e] = LOAD_B(rsrc_b, vo, (K_AT(k0) / (CR * CS)) * (CH * CW * 4));
 #else
             const int k = k0 + b_row[e];
             const int c = k / (CR * CS);

@@ -128,3 +128,35 @@ def test_batched_products_of_odd_extents(b, m, k, n, trans_b):
     c = torch.full((b, m, n), -7.0, device="cuda")
     f(placed(x), placed(np.ascontiguousarray(y.transpose(0, 2, 1)) if trans_b else y), c)
     assert close(c.cpu().numpy(), np.matmul(x.astype(np.float64), y.astype(np.float64)))
+
+
+@pytest.mark.parametrize("m,k,groups", [(1, 257, 2), (3, 259, 4), (1, 385, 2)])
+def test_int8_tiles_wholly_behind_k(oracle, m, k, groups):
+    """K divided so that the last group's last tiles lie behind K altogether, over operands of few rows: the
+    tile's scalar offset would be beyond the buffer."""
+    import torch
+    from flextensor_amd.task import gemm_int8
+    n, bk = 33, 128
+    config = dict(spatial=[[1, 1, 1, 16], [3, 1, 1, 16]], reduce=[[groups, -(-k // (groups * bk)), bk]], unroll=[[2, 1]],
+                  fuse=[[4]], reorder=[[1, 1, 0]], inline=[], merge=[], special=[])
+    f, _ = build_config(gemm_int8, (m, k, n), config)
+    rng = np.random.default_rng(k)
+    a, b = [rng.integers(-128, 128, size=s, dtype=np.int8) for s in ((m, k), (n, k))]
+    c = torch.full((m, n), -7, dtype=torch.int32, device="cuda")
+    f(placed(a), placed(b), c)
+    assert np.array_equal(c.cpu().numpy(), oracle.gemm_i8_c(a, b))
+
+
+@pytest.mark.parametrize("depth", [3, 5, 8])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_fp32_tiles_wholly_behind_k(oracle, depth, trans_b):
+    import torch
+    m, k, n, groups, bk = 1, 416, 64, 4, 32        # 13 tiles of K for 4 groups of 4
+    cfg = gemm_config(m, k, n, 1, 1, 1, 16, bk, depth, groups)
+    cfg["spatial"] = [[1, 1, 1, 16], [1, 1, 4, 16]]
+    f, _ = build_config(gemm_of(trans_b), (m, k, n), cfg)
+    rng = np.random.default_rng(k)
+    a, b = [rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n))]
+    c = torch.full((m, n), -7.0, device="cuda")
+    f(placed(a), placed(np.ascontiguousarray(b.T) if trans_b else b), c)
+    assert close(c.cpu().numpy(), oracle.gemm_f32_c(a, b))
