@@ -944,11 +944,18 @@ def default_config(op):
         cfg["reorder"] = [[1, 0, 0]]
     elif op.kind == "depthwise_conv2d_nchw":
         b, c, p, q = [x.extent for x in op.axis]
-        th = 4 if p >= 4 else 1
+        # Rows per lane patch: 4 (3 at stride 2, where a row more is two more input rows to hold), fewer while
+        # that leaves less than a wavefront per SIMD; small workgroups of two wavefronts, which retire and
+        # start at a finer grain. Over 22 layers (1 .. 31 images, 24 .. 511 channels, 10 .. 104 rows; 3x3 and 5x5,
+        # stride 1 and 2) this is 4 % off the best of 1 .. 8 rows and 1 .. 4 wavefronts in the geometric mean, 4 rows
+        # and 4 wavefronts everywhere are 19 % off: 17x413x66x20 5x5 stride 2 33.9 -> 17.6 us.
         tw = 4 if q >= 4 else 1
+        th = min(4 if op.attrs["stride"][0] == 1 else 3, p)
+        while th > 1 and b * c * ceil_div(p, th) * ceil_div(q, tw) < 64 * 4 * NUM_CUS:
+            th //= 2
         cfg["spatial"] = [[b, 1, 1, 1], [c, 1, 1, 1], [ceil_div(p, th), 1, 1, th],
                           [ceil_div(q, tw), 1, 1, tw]]
-        cfg["fuse"] = [[4]]
+        cfg["fuse"] = [[2]]
     return cfg
 
 

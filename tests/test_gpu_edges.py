@@ -160,3 +160,29 @@ def test_fp32_tiles_wholly_behind_k(oracle, depth, trans_b):
     c = torch.full((m, n), -7.0, device="cuda")
     f(placed(a), placed(np.ascontiguousarray(b.T) if trans_b else b), c)
     assert close(c.cpu().numpy(), oracle.gemm_f32_c(a, b))
+
+
+# ---- depthwise rows of any length --------------------------------------------------------------------------
+
+@pytest.mark.parametrize("args", [
+    # b, c, h, w, factor, r, stride, padding, dilation
+    (2, 5, 57, 57, 1, 3, 1, 1, 1), (1, 3, 7, 7, 1, 3, 1, 1, 1), (2, 4, 9, 10, 1, 5, 1, 2, 1), (2, 4, 11, 13, 1, 3, 2, 1, 1),
+    (1, 6, 14, 14, 2, 3, 1, 1, 1), (2, 3, 12, 17, 1, 5, 2, 2, 1), (1, 2, 13, 15, 1, 3, 1, 2, 2), (3, 4, 6, 5, 1, 3, 1, 0, 1),
+    (1, 4, 30, 31, 1, 4, 3, 1, 1), (2, 2, 8, 6, 1, 5, 1, 4, 1)])
+def test_depthwise_rows_of_any_length(oracle, args):
+    """Row lengths, strides and paddings whose rows are no whole vectors; the image is surrounded by NaN so that
+    an element from beyond a row's or the tensor's end would show."""
+    import torch
+    from flextensor_amd.task import depthwise_conv2d
+    b, c, h, w, fa, r, st, pd, dl = args
+    rng = np.random.default_rng(sum(args))
+    x, wt = rng.standard_normal((b, c, h, w)).astype(np.float32), rng.standard_normal((c, fa, r, r)).astype(np.float32)
+    want = oracle.depthwise_nchw_c(x, wt, st, pd, dl)
+    f, _ = build_default(depthwise_conv2d, "conv2d", args)
+    flat = torch.full((x.size + 64,), float("nan"), device="cuda")
+    flat[33:33 + x.size] = torch.from_numpy(x).cuda().flatten()
+    y = torch.full((want.size + 64,), -7.0, device="cuda")
+    f(flat[33:33 + x.size].view(x.shape), placed(wt, 1), y[31:31 + want.size].view(want.shape))
+    got = y.cpu().numpy()
+    assert close(got[31:31 + want.size].reshape(want.shape), want)
+    assert (got[:31] == -7).all() and (got[31 + want.size:] == -7).all()
