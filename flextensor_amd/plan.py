@@ -144,6 +144,28 @@ class BuiltPlan(object):
         else:
             for name, (shape, dtype) in plan.workspaces.items():
                 self.scratch[name] = torch.zeros(shape, dtype=_torch_dtype(dtype), device="cuda")
+        self._native = None if static_workspace else self._native_call()
+
+    def _native_call(self):
+        """The launches laid out for the native call (csrc/ftcall.cpp): everything but the tensors' addresses."""
+        try:
+            from . import _ftcall
+        except ImportError as e:
+            raise rt.RuntimeError_("_ftcall.so is not built (%s); run `make -C flextensor_amd/csrc` or "
+                                   "__graft_entry__.build()" % e)
+        index = dict((name, i) for i, name in enumerate(self.plan.buf_names))
+        launches = []
+        for spec, mod in zip(self.plan.specs, self.modules):
+            args = []
+            for kind, v in spec.args:
+                if kind == "buf":
+                    args.append((index[v], 0) if v in index else (-1, self.scratch[v].data_ptr()))
+                else:
+                    args.append((-1, int(v) & (0xffffffffffffffff if kind == "i64" else 0xffffffff)))
+            grid, block = [tuple(int(x) for x in g) + (1,) * (3 - len(g)) for g in (spec.grid, spec.block)]
+            launches.append((mod.handle.value, grid, block, int(spec.lds_bytes), args))
+        bufs = [(b.dtype, tuple(int(e) for e in b.shape)) for b in self.plan.bufs]
+        return _ftcall.Call(rt.address("ftr_launch_seq"), rt.address("ftr_last_error"), rt.RuntimeError_, bufs, launches)
 
     def attrs(self):
         return [m.attrs() for m in self.modules]
@@ -188,6 +210,8 @@ class BuiltPlan(object):
         return out
 
     def __call__(self, *tensors):
+        if self._native is not None and self._native(*tensors):
+            return
         launches = self.launches(tensors)
         if self.static_layout is not None:
             rt.launch_seq_static_ws(launches, self._binds, stream=current_stream())
@@ -213,6 +237,7 @@ class BuiltPlan(object):
         return rt.time_seq(sets, warmup=warmup, iters=iters, stream=stream, timeout=timeout)
 
     def close(self):
+        self._native = None
         for m in self.modules:
             m.close()
         self.modules = []

@@ -147,6 +147,11 @@ def _check(rc, what):
         raise DeviceTimeout(text) if rc == FTR_TIMEOUT else RuntimeError_(text)
 
 
+def address(name):
+    """Address of one of the library's functions, for native callers."""
+    return ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
+
+
 def device_count():
     return lib().ftr_device_count()
 

@@ -186,3 +186,41 @@ def test_depthwise_rows_of_any_length(oracle, args):
     got = y.cpu().numpy()
     assert close(got[31:31 + want.size].reshape(want.shape), want)
     assert (got[:31] == -7).all() and (got[31 + want.size:] == -7).all()
+
+
+# ---- the native call ----------------------------------------------------------------------------------------
+
+def test_a_plan_refuses_what_it_does_not_take():
+    import torch
+    f, _ = build_config(gemm_of(False), (16, 8, 12), None)
+    a, b, c = torch.randn(16, 8, device="cuda"), torch.randn(8, 12, device="cuda"), torch.empty(16, 12, device="cuda")
+    f(a, b, c)
+    assert torch.allclose(c, a @ b, atol=1e-4)
+    for bad in ((a, b), (a, b, c, c), (a.t(), b, c), (a.double(), b, c), (a.cpu(), b, c), (torch.randn(8, 16, device="cuda").t(), b, c),
+                (a, torch.randn(8, 24, device="cuda")[:, ::2], c)):
+        with pytest.raises(ValueError):
+            f(*bad)
+    f(torch.nn.Parameter(a), b, c)
+
+
+def test_a_plan_called_by_threads_on_streams():
+    import threading
+    import torch
+    f, _ = build_config(gemm_of(False), (96, 64, 80), None)
+    sets = [[torch.randn(96, 64, device="cuda"), torch.randn(64, 80, device="cuda"), torch.empty(96, 80, device="cuda")] for _ in range(4)]
+    streams = [torch.cuda.Stream() for _ in sets]
+    torch.cuda.synchronize()
+
+    def work(ts, stream):
+        with torch.cuda.stream(stream):
+            for _ in range(200):
+                f(*ts)
+
+    threads = [threading.Thread(target=work, args=p) for p in zip(sets, streams)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for a, b, c in sets:
+        assert torch.allclose(c, a @ b, atol=1e-4)
