@@ -896,7 +896,7 @@ def schedule_with_config_ops(ops, bufs, configs, op_pos=None, target="rocm", tas
             in_names.append(names[src])
         config = op_config_lst[i] if i < len(op_config_lst) and op_config_lst[i] else None
         if config is None or not any(config.get(k) for k in ("spatial", "reduce", "fuse")):
-            config = gfx950.default_config(op)
+            config = gfx950.untuned_config(op, special)
         template = OpScheduler.generate_op_schedule(target, config)
         specs.extend(template(op, special, names[out_t], in_names, materialized_pad, bias_name,
                               through=tuple(through), merged_out=merged_out))

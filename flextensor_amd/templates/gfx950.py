@@ -763,7 +763,7 @@ I8_TILES = (((2, 1), (2, 1)), ((2, 1), (2, 2)), ((2, 2), (2, 2)), ((2, 2), (4, 2
             ((4, 4), (4, 4)), ((1, 1), (4, 1)))
 
 
-def _default_i8(view):
+def _default_i8(view, padded=False):
     """Tile, K tile and K division of an int8 GEMM nobody tuned: the smallest predicted time over a few
     tiles that between them are within 3 % of the best measured one everywhere.
 
@@ -778,7 +778,7 @@ def _default_i8(view):
     times as fast as the rule before it (square-ish power-of-two tiles until every compute unit has one, K tiles of
     64 through registers): 64x3632x1376 12.0 -> 4.8 us, 1712x1584x2080 21.3 -> 13.6, 3488x176x80 4.2 -> 2.6.
     """
-    aligned = view.K % 16 == 0        # tiles straight into LDS
+    aligned = view.K % 16 == 0 and not padded        # tiles straight into LDS
     best = None
     for (wm, rm), (wn, rn) in I8_TILES:
         bm, bn = wm * rm * 16, wn * rn * 16
@@ -849,7 +849,7 @@ def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups):
             + (38 * rm * rn * mf * mf / 64 * (groups - 1)))
 
 
-def _default_f32(view):
+def _default_f32(view, padded=False):
     """Tile, K tile, pipeline and K division of an fp32 GEMM (or a batch of them) nobody tuned: the smallest
     predicted time over F32_KERNELS, which between them are within 2 % of the best measured kernel everywhere.
 
@@ -864,8 +864,17 @@ def _default_f32(view):
     44.4, 96 x 74x96x133 6.8 -> 5.4, 32x4096x3072 43.6 -> 16.5. K streaming is left to the search: a plan that owns a
     workspace cannot run on two streams at once, and a default plan can.
     """
+    return _pick_f32(view, F32_KERNELS, _f32_clocks, padded)
+
+
+def _pick_f32(view, kernels, predict, padded):
+    """The config of the kernel and number of wavefront K groups with the smallest predicted time; where the LDS
+    rows are to be padded, among the kernels whose tiles pass through registers, with K undivided (the groups' tiles
+    lie beside each other in LDS)."""
     best = None
-    for m, n, mf, bk, depth in F32_KERNELS:
+    for m, n, mf, bk, depth in kernels:
+        if padded and depth >= 5:
+            continue
         bm, bn = m[0] * m[1] * mf, n[0] * n[1] * mf
         if bm >= 2 * max(view.M, 16) or bn >= 2 * max(view.N, 16):
             continue
@@ -877,13 +886,13 @@ def _default_f32(view):
         tm, tn = ceil_div(view.M, bm), ceil_div(view.N, bn)
         tiles = tm * tn * view.groups
         for groups in (1, 2, 4, 8, 16):
-            if groups > 1 and (tiles > 400 or groups * m[0] * n[0] > 16):
+            if groups > 1 and (padded or tiles > 400 or groups * m[0] * n[0] > 16):
                 break
             steps = ceil_div(view.K, bk * groups)
             kp = steps * bk * groups
             if kp not in view.KP_options and kp * 4 > view.K * 5:
                 break
-            clocks = _f32_clocks(view, tiles, m, n, mf, bk, depth, groups)
+            clocks = predict(view, tiles, m, n, mf, bk, depth, groups)
             if clocks is not None and (best is None or clocks < best[0]):
                 best = (clocks, [tm, m[0], m[1], mf], [tn, n[0], n[1], mf], [groups, steps, bk], depth)
     cfg = _empty_config()
@@ -895,14 +904,63 @@ def _default_f32(view):
     return cfg
 
 
-def default_config(op):
-    """A reasonable untuned config: what schedule_with_config falls back to
-    when a task has no tuned entry, and the seed point of the search."""
+# kernels of the convolution's default, as F32_KERNELS; the K tiles of 72 and 144 hold whole windows of 3x3 (and of
+# whatever else divides them) and are for those
+CONV_KERNELS = (((1, 1), (1, 1), 16, 16, 2), ((1, 1), (1, 1), 16, 32, 3), ((2, 1), (2, 1), 16, 32, 3),
+                ((4, 1), (2, 1), 16, 32, 3), ((2, 2), (4, 1), 16, 16, 2), ((2, 1), (4, 1), 16, 16, 2),
+                ((4, 2), (4, 1), 16, 32, 5), ((2, 1), (2, 1), 32, 16, 3))
+CONV_WINDOW_KERNELS = (((1, 1), (1, 1), 16, 144, 8), ((2, 1), (2, 1), 16, 144, 8), ((2, 1), (4, 1), 16, 144, 8),
+                       ((2, 1), (2, 1), 32, 72, 8), ((4, 1), (2, 1), 32, 72, 8))
+
+
+def _default_conv(view, padded=False):
+    """Tile, K tile, pipeline and K division of a convolution nobody tuned, by predicted time like _default_f32.
+
+    What differs from the plain product is the gathered operand. One float per lane and load, with its own address:
+    where the K tile holds whole windows (or the window is one pixel) the address advances by a constant, else
+    channel, tap and padding predicate are computed anew for every element of every tile, about 50 clocks per 64 of
+    them, and an untiled 3x3 layer spends more on that than on its products. Whole windows pay where tiles are many;
+    with few tiles K is divided over wavefront groups instead, which shortens the serial chain of k steps.
+    Constants fitted to 3 600 timings over 45 layers (1 .. 16 images, 16 .. 512 channels, 7 .. 112 rows; 1x1 and
+    3x3, stride 1 and 2); the pick is within 7 % of the best measured kernel in the geometric mean, the rule before it
+    (square-ish power-of-two tiles until every unit has one, K tiles of up to 32, K undivided) 1.77 times off.
+    """
+    window = view.conv["CR"] * view.conv["CS"]
+
+    def clocks(view, tiles, m, n, mf, bk, depth, groups):
+        (wm, rm), (wn, rn) = m, n
+        bm, bn = wm * rm * mf, wn * rn * mf
+        steps = ceil_div(view.K, bk * groups)
+        nw = wm * wn * groups
+        lds = groups * 2 * 4 * (bm + bn) * bk
+        if lds > LDS_BYTES:
+            return None
+        share = ceil_div(tiles, NUM_CUS)
+        turns = ceil_div(share, max(1, min(LDS_BYTES // lds, 32 // nw)))
+        step = rm * rn * mf * mf * 2 * bk / 64.0                        # matrix clocks of one wavefront's k step
+        gathered = groups * bn * bk / 64.0                              # loads of a step's gather, all wavefronts
+        hoisted = bk % window == 0
+        latency = {2: 129, 3: 125, 5: 457, 8: 1499}[depth] * (1 + 0.12 * bk / 32) + 33 * nw
+        overlap = {2: 0.8, 3: 0.4, 5: 0.3, 8: 0.35}[depth]
+        compute = ceil_div(share * nw, 4) * step * steps + share * steps * gathered * (3.7 if hoisted else 51.6) / 4
+        chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap + (0 if hoisted else 80 * gathered / nw)) + 3230)
+        operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / 16
+        longest = max(compute, chain, operands)
+        return (longest + 0.47 * (compute + chain + operands - longest) + share * bm * bn * 4 * 3.0 / 64
+                + 82 * rm * rn * mf * mf / 64 * (groups - 1))
+
+    return _pick_f32(view, CONV_KERNELS + (CONV_WINDOW_KERNELS if window > 1 and 72 % window == 0 else ()),
+                     clocks, padded)
+
+
+def default_config(op, padded=False):
+    """A reasonable untuned config: the point a search begins with, and for all operators but the convolution
+    what an untuned task runs on (untuned_config)."""
     cfg = _empty_config()
     if op.kind == "gemm_int8":
-        return _default_i8(GemmView(op))
+        return _default_i8(GemmView(op), padded)
     if op.kind in ("gemm", "batch_gemm"):
-        return _default_f32(GemmView(op))
+        return _default_f32(GemmView(op), padded)
     if op.kind in GEMM_KINDS:
         view = GemmView(op)
 
@@ -957,6 +1015,16 @@ def default_config(op):
                           [ceil_div(q, tw), 1, 1, tw]]
         cfg["fuse"] = [[2]]
     return cfg
+
+
+def untuned_config(op, special=None):
+    """What schedule_with_config falls back to when a task has no tuned entry. The convolution's search keeps
+    beginning at a square-ish tile with K undivided, beside which its other seed points lie. An LDS layout that
+    the graph config names (``special``) is one that tiles straight into LDS may not be able to have."""
+    padded = _special(special, "lds_pad") != SPECIAL_DEFAULTS["lds_pad"]
+    if op.kind in ("conv2d_nchw", "col_gemm"):
+        return _default_conv(GemmView(op), padded)
+    return default_config(op, padded)
 
 
 def seed_configs(op, limit=24):

@@ -162,6 +162,33 @@ def test_fp32_tiles_wholly_behind_k(oracle, depth, trans_b):
     assert close(c.cpu().numpy(), oracle.gemm_f32_c(a, b))
 
 
+# ---- convolutions on the default plan ----------------------------------------------------------------------
+
+@pytest.mark.parametrize("args", [
+    # b, c, h, w, o, r, stride, padding, dilation, groups
+    (1, 1, 5, 5, 1, 3, 1, 1, 1, 1), (2, 3, 9, 7, 5, 1, 1, 0, 1, 1), (1, 17, 6, 6, 33, 1, 1, 0, 1, 1), (3, 16, 7, 7, 17, 3, 1, 1, 1, 1),
+    (4, 64, 7, 7, 64, 3, 2, 1, 1, 1), (9, 78, 8, 8, 69, 3, 2, 1, 1, 1),       # K over wavefront groups, tiles behind K
+    (2, 223, 13, 15, 56, 3, 1, 1, 1, 1), (11, 152, 7, 17, 30, 3, 2, 1, 1, 1),
+    (8, 130, 29, 31, 130, 3, 1, 1, 1, 1), (16, 129, 33, 33, 255, 3, 2, 1, 1, 1),    # whole windows, ragged K and edges
+    (5, 33, 57, 61, 150, 1, 1, 0, 1, 1), (10, 17, 94, 94, 67, 1, 1, 0, 1, 1), (4, 139, 41, 12, 235, 1, 2, 0, 1, 1),
+    (2, 12, 15, 17, 20, 5, 1, 2, 1, 1), (2, 24, 15, 17, 36, 3, 1, 2, 2, 2), (1, 3, 40, 40, 24, 7, 2, 3, 1, 1)])
+def test_convolutions_of_any_extent(oracle, args):
+    """Default plans: pixels and windows, strides, dilation and groups, K that no K tile divides; the image lies
+    between NaN so that a gather from beyond it would show."""
+    import torch
+    from flextensor_amd.task import conv2d
+    b, c, h, w, o, r, st, pd, dl, gr = args
+    rng = np.random.default_rng(sum(args))
+    x, wt = rng.standard_normal((b, c, h, w)).astype(np.float32), rng.standard_normal((o, c // gr, r, r)).astype(np.float32)
+    f, bufs = build_default(conv2d, "conv2d", args)
+    flat = torch.full((x.size + 64,), float("nan"), device="cuda")
+    flat[33:33 + x.size] = torch.from_numpy(x).cuda().flatten()
+    y = torch.full(tuple(int(e) for e in bufs[-1].shape), -7.0, device="cuda")
+    f(flat[33:33 + x.size].view(x.shape), placed(wt, 1), y)
+    want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), None, st, pd, dl, gr).numpy()
+    assert close(y.cpu().numpy(), want)
+
+
 # ---- depthwise rows of any length --------------------------------------------------------------------------
 
 @pytest.mark.parametrize("args", [

@@ -625,3 +625,32 @@ def test_clock_probe_plan_is_a_copy_with_one_more_argument():
     from flextensor_amd.plan import KernelPlan
     with pytest.raises(ValueError):
         KernelPlan("x", s.bufs, [], {}, None).with_clock_probe()
+
+
+@pytest.mark.parametrize("lds_pad", [[-1, -1], [4, -1], [4, 8], [0, 0], [8, -1], [12, 8]])
+def test_untuned_operators_lower_under_every_lds_layout(lds_pad):
+    """A graph config may name an LDS layout for an operator without a config of its own: the default kernel is then
+    one that can have it (tiles straight into LDS need unpadded rows), also with K long and tiles few."""
+    from flextensor_amd import nn
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.te import placeholder
+
+    def conv(b, c, h, o, r):
+        x, wt = placeholder((b, c, h, h), name="X"), placeholder((o, c, r, r), name="W")
+        return nn.conv2d_nchw(x, wt, stride=1, padding=r // 2), [x, wt]
+
+    def gemm(m, k, n):
+        a, b = placeholder((m, k), name="A"), placeholder((k, n), name="B")
+        return nn.gemm(a, b), [a, b]
+
+    def gemm_i8(m, k, n):
+        a, b = placeholder((m, k), dtype="int8", name="A"), placeholder((n, k), dtype="int8", name="B")
+        return nn.gemm_int8(a, b), [a, b]
+
+    for out, bufs in (conv(1, 130, 7, 16, 7), conv(1, 512, 5, 2, 5), conv(8, 256, 28, 256, 3), conv(2, 240, 35, 160, 1),
+                      gemm(32, 4096, 4096), gemm(1000, 1531, 777), gemm(1024, 1024, 1024), gemm_i8(64, 4096, 64),
+                      gemm_i8(4096, 4096, 4096)):
+        pad = [max(lds_pad[0], -1), 0] if out.dtype == "int32" or bufs[0].dtype == "int8" else lds_pad
+        s, _ = schedule_with_config_ops([out.op], bufs + [out], Config([], {"inline": [], "merge": [], "special": [pad]}),
+                                        special_names=["lds_pad"])
+        assert s.specs[-1].defines.get("APAD", s.specs[-1].defines.get("PAD")) in (pad[0], pad[0] * 4)
