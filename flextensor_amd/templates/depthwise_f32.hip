@@ -149,7 +149,9 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 /* Rows of any length, stride and padding: the IW_T columns of a patch row as 16-byte loads from its first
  * column on (a buffer load needs dword alignment only). The leftmost patch of a row begins in the padding: its
  * vectors start at column 0 and its elements move up by PADW. Elements beyond the row's right end come from the
- * next row (or, behind the tensor, read as zero): they become zeros. A row of a 3x3 window is two
+ * next row (or, behind the tensor, read as zero): they become zeros. A vector's place in the row is part of
+ * the lane's offset: the range check compares that offset with (bytes - scalar offset), and a scalar offset beyond an
+ * image of a few bytes would wrap the difference and let every lane pass. A row of a 3x3 window is two
  * loads instead of six, and a row of four results one store instead of four: 16x144x57x57 3x3 with a bias goes from
  * 25.1 to 11.6 us (60 MB: 5.2 TB/s), as fast as rows of whole vectors. */
 #if !VEC_IN && !SHFL && (TW == 4) && (PADW <= 4 * STRW)
@@ -503,14 +505,15 @@ void depthwise_f32(const float* __restrict__ X, const float* __restrict__ Wt,
             const unsigned vo = row_ok ? off : OOB;
 #pragma unroll
             for (int v = 0; v < NANY; ++v) {
+                const int at = (int)(vo + 16u * v);
                 if (IW_T - 4 * v == 1) {
-                    rows[k][y][4 * v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, (int)vo, v * 16, LD_AUX));
+                    rows[k][y][4 * v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, at, 0, LD_AUX));
                 } else if (IW_T - 4 * v == 2) {
-                    const f32x2 d = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rx, (int)vo, v * 16, LD_AUX));
+                    const f32x2 d = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rx, at, 0, LD_AUX));
                     rows[k][y][4 * v] = d[0];
                     rows[k][y][4 * v + 1] = d[1];
                 } else {
-                    const f32x4 q = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)vo, v * 16, LD_AUX));
+                    const f32x4 q = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, at, 0, LD_AUX));
 #pragma unroll
                     for (int i = 0; i < 4; ++i) rows[k][y][4 * v + i] = q[i];
                 }

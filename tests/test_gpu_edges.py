@@ -195,7 +195,9 @@ def test_convolutions_of_any_extent(oracle, args):
     # b, c, h, w, factor, r, stride, padding, dilation
     (2, 5, 57, 57, 1, 3, 1, 1, 1), (1, 3, 7, 7, 1, 3, 1, 1, 1), (2, 4, 9, 10, 1, 5, 1, 2, 1), (2, 4, 11, 13, 1, 3, 2, 1, 1),
     (1, 6, 14, 14, 2, 3, 1, 1, 1), (2, 3, 12, 17, 1, 5, 2, 2, 1), (1, 2, 13, 15, 1, 3, 1, 2, 2), (3, 4, 6, 5, 1, 3, 1, 0, 1),
-    (1, 4, 30, 31, 1, 4, 3, 1, 1), (2, 2, 8, 6, 1, 5, 1, 4, 1)])
+    (1, 4, 30, 31, 1, 4, 3, 1, 1), (2, 2, 8, 6, 1, 5, 1, 4, 1),
+    # images of a few bytes, smaller than a patch row's vectors
+    (1, 1, 1, 3, 1, 3, 1, 2, 1), (1, 1, 1, 5, 1, 7, 1, 3, 1), (1, 1, 1, 1, 1, 5, 1, 4, 1), (1, 1, 2, 2, 1, 5, 2, 5, 1)])
 def test_depthwise_rows_of_any_length(oracle, args):
     """Row lengths, strides and paddings whose rows are no whole vectors; the image is surrounded by NaN so that
     an element from beyond a row's or the tensor's end would show."""

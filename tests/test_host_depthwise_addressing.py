@@ -133,3 +133,131 @@ def test_full_rows_and_narrow_kernels_need_no_clip():
         defs = dict(NT=64, TH=1, TW=4, NT_STORE=0, SHFL=0, CB=1, CC=2, CH=cw, CW=cw, CR=cs, CS=cs,
                     STRH=stride, STRW=stride, PADH=pad, PADW=pad, DILH=dil, DILW=dil, FACT=1, CP=cq, CQ=cq)
         assert template_flags(defs) == (True, False)
+
+
+# ---- rows of any length (VEC_ANY) ---------------------------------------------------------------------------
+
+def emulate_any(x, wt, stride, pad, dil):
+    """Planes through the addressing of the rows of any length: TH = 1, TW = 4. What lies behind the
+    tensor reads as zero; rows in the padding ask for nothing."""
+    planes, ch, cw = x.shape
+    cr, cs = wt.shape[1:]
+    cp = (ch + 2 * pad - dil * (cr - 1) - 1) // stride + 1
+    cq = (cw + 2 * pad - dil * (cs - 1) - 1) // stride + 1
+    iw_t = 3 * stride + (cs - 1) * dil + 1
+    nany = (iw_t + 3) // 4
+    flat = np.concatenate([x.reshape(-1), np.zeros(4 * nany, x.dtype)])
+    out = np.zeros((planes, cp, cq))
+    for pl, oh, tw in itertools.product(range(planes), range(cp), range((cq + 3) // 4)):
+        iw0 = tw * 4 * stride - pad
+        ic0 = 0 if pad > 0 and tw == 0 else iw0
+        acc = np.zeros(4)
+        for r in range(cr):
+            ih = oh * stride - pad + r * dil
+            row = np.zeros(4 * nany)
+            if 0 <= ih < ch:
+                off = pl * ch * cw + ih * cw + ic0
+                assert off >= 0
+                got = flat[off:off + 4 * nany]
+                row[:len(got)] = got
+            inp = row[:iw_t].copy()
+            if pad > 0 and tw == 0:
+                inp = np.array([row[j - pad] if j >= pad else 0.0 for j in range(iw_t)])
+            inp[[j for j in range(iw_t) if iw0 + j >= cw]] = 0.0
+            for j, s in itertools.product(range(4), range(cs)):
+                acc[j] += inp[j * stride + s * dil] * wt[pl, r, s]
+        n = min(4, cq - tw * 4)
+        out[pl, oh, tw * 4:tw * 4 + n] = acc[:n]
+    return out
+
+
+def test_rows_of_any_length_match_the_definition():
+    rng = np.random.default_rng(6)
+    taken = 0
+    for cs, stride, pad, dil, cw in itertools.product((1, 3, 5), (1, 2, 3), (0, 1, 2, 4), (1, 2), (1, 3, 5, 8, 11, 14)):
+        ch = 4
+        cq = (cw + 2 * pad - dil * (cs - 1) - 1) // stride + 1
+        cp = (ch + 2 * pad - dil * (cs - 1) - 1) // stride + 1
+        if cq < 4 or cp < 1 or pad > 4 * stride:
+            continue
+        defs = dict(NT=64, TH=1, TW=4, NT_STORE=0, SHFL=0, CB=1, CC=2, CH=ch, CW=cw, CR=cs, CS=cs, STRH=stride,
+                    STRW=stride, PADH=pad, PADW=pad, DILH=dil, DILW=dil, FACT=1, CP=cp, CQ=cq)
+        if template_flags(defs)[0]:
+            continue
+        taken += 1
+        x, wt = rng.uniform(-1, 1, (2, ch, cw)), rng.uniform(-1, 1, (2, cs, cs))
+        ref = oracle.depthwise_nchw_np(x[None], wt[:, None], stride, pad, dil)[0]
+        assert np.max(np.abs(emulate_any(x, wt, stride, pad, dil) - ref)) < 1e-12, (cs, stride, pad, dil, cw)
+    assert taken >= 100
+
+
+# ---- scalar offsets stay inside their buffers ----------------------------------------------------------------
+
+def _c_value(expr, env):
+    expr = re.sub(r"\([a-z_ ]*(?:int|unsigned)\)", "", expr)
+    expr = expr.replace("&&", " and ").replace("||", " or ").replace("/", "//")
+    return int(eval(re.sub(r"!(?!=)", " not ", expr), {}, env))
+
+
+def _arguments(text, at):
+    """The top-level arguments of the call whose opening parenthesis is text[at]."""
+    depth, args, start = 0, [], at + 1
+    for i in range(at, len(text)):
+        if text[i] in "([{":
+            depth += 1
+        elif text[i] in ")]}":
+            depth -= 1
+            if depth == 0:
+                return [a.strip() for a in args + [text[start:i]]]
+        elif text[i] == "," and depth == 1:
+            args.append(text[start:i])
+            start = i + 1
+    raise AssertionError("unbalanced call")
+
+
+def scalar_offsets(spec):
+    """[(descriptor, its bytes, largest scalar offset)] of every buffer access of a depthwise kernel, from the
+    preprocessed template: the loops around an access give its variables their values."""
+    cmd = ["gcc", "-E", "-P", "-x", "c", "-"] + spec.options()
+    text = subprocess.run(cmd, input=spec.source(), capture_output=True, text=True, check=True).stdout
+    sizes = dict((m.group(1), _c_value(_arguments(text, m.end() - 1)[2], {}))
+                 for m in re.finditer(r"rsrc_t (\w+) = __builtin_amdgcn_make_buffer_rsrc\(", text))
+    found = []
+    for m in re.finditer(r"__builtin_amdgcn_raw_buffer_(load|store)_b\d+\(", text):
+        args = _arguments(text, m.end() - 1)[1 if m.group(1) == "store" else 0:]
+        values = [{}]
+        for var in set(re.findall(r"[a-z]\w*", args[2])):
+            loop = re.findall(r"for \(int %s = ([^;]*); ([^;]*); ([^)]*)\)" % var, text[:m.start()])[-1]
+            v, steps = _c_value(loop[0], {}), []
+            while _c_value(loop[1], {var: v}):
+                steps.append(v)
+                v += int(loop[2].split("+=")[1]) if "+=" in loop[2] else 1
+            values = [dict(e, **{var: s}) for e in values for s in steps]
+        found += [(args[0], sizes[args[0]], max(_c_value(args[2], e) for e in values))] if values else []
+    return found
+
+
+def test_scalar_offsets_stay_inside_small_tensors():
+    """The range check of a buffer access compares the lane's offset with (bytes - scalar offset): a scalar offset
+    beyond the buffer would wrap that difference and let every lane pass, those of the padding rows too. Default
+    plans over the smallest images, with every window, stride and padding that leaves four columns or more."""
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.task import depthwise_conv2d
+    from flextensor_amd.templates.gfx950 import InvalidConfig
+    from flextensor_amd.utils import Config
+    checked = 0
+    for h, w, r, stride, pad, dil in itertools.product((1, 2), (1, 2, 3, 5, 6), (1, 2, 3, 5, 7), (1, 2), (0, 1, 2, 3, 4, 8), (1, 2)):
+        q = (w + 2 * pad - dil * (r - 1) - 1) // stride + 1
+        if q < 4 or (h + 2 * pad - dil * (r - 1) - 1) // stride + 1 < 1:
+            continue
+        ops, bufs = depthwise_conv2d(1, 1, h, w, 1, r, stride, pad, dil)
+        try:
+            spec = schedule_with_config_ops(ops, bufs, Config([], None))[0].specs[-1]
+        except InvalidConfig:              # a window too large for the registers
+            continue
+        accesses = scalar_offsets(spec)
+        assert {a[0] for a in accesses} == {"rx", "rw", "ro"}
+        for name, nbytes, offset in accesses:
+            assert offset <= nbytes, (h, w, r, stride, pad, dil, name, nbytes, offset)
+        checked += 1
+    assert checked >= 150
