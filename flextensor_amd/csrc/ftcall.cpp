@@ -5,7 +5,7 @@
 // call (ctypes objects for every argument and descriptor, made anew each time), more than most kernels of a
 // single layer: back to back, a 3x3 layer on 1x64x56x56 now takes its 5.1 us on the device instead of 15.7, a depthwise layer
 // on 8x512x28x28 4.9 instead of 15.8. Everything but the addresses is laid out once, when the plan is built; a
-// call keeps its argument arrays on its own stack, so several threads may call one plan.
+// call's argument arrays are its own, so several threads may call one plan.
 //
 // A call returns True when the work is enqueued and False when the tensors are not what the plan takes or are not
 // plain tensors: the caller then goes the general way, which says what is wrong.
@@ -13,6 +13,7 @@
 
 #include <Python.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/SmallVector.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -44,7 +45,8 @@ struct Call {
     std::vector<Arg> *args;
 };
 
-constexpr size_t kMaxArgs = 64, kMaxLaunches = 16, kMaxBufs = 16;
+// a call's own arrays: on its stack up to these sizes (a few operators), on the heap for larger graphs
+constexpr unsigned kInlineArgs = 64, kInlineLaunches = 16, kInlineBufs = 16;
 
 bool fits(const at::Tensor &t, const Buffer &b) {
     const auto *impl = t.unsafeGetTensorImpl();
@@ -57,30 +59,27 @@ PyObject *call(PyObject *self_, PyObject *const *argv, size_t nargsf, PyObject *
     Call *self = reinterpret_cast<Call *>(self_);
     const size_t n = PyVectorcall_NARGS(nargsf);
     if (n != self->bufs->size() || (kwnames && PyTuple_GET_SIZE(kwnames))) Py_RETURN_FALSE;
-    void *ptr[kMaxBufs];
+    c10::SmallVector<void *, kInlineBufs> ptr(n);
     for (size_t i = 0; i < n; ++i) {
         if (!THPVariable_CheckExact(argv[i])) Py_RETURN_FALSE;
         const at::Tensor &t = THPVariable_Unpack(argv[i]);
         if (!fits(t, (*self->bufs)[i])) Py_RETURN_FALSE;
         ptr[i] = t.data_ptr();
     }
-    unsigned long long values[kMaxArgs];
-    void *slots[kMaxArgs];
     const std::vector<Arg> &args = *self->args;
+    c10::SmallVector<unsigned long long, kInlineArgs> values(args.size());
+    c10::SmallVector<void *, kInlineArgs> slots(args.size());
     for (size_t i = 0; i < args.size(); ++i) {
         values[i] = args[i].tensor < 0 ? args[i].value : reinterpret_cast<unsigned long long>(ptr[args[i].tensor]);
         slots[i] = &values[i];
     }
-    ftr_launch_desc_t seq[kMaxLaunches];
-    const int nl = static_cast<int>(self->launches->size());
-    for (int i = 0; i < nl; ++i) {
-        seq[i] = (*self->launches)[i];
-        seq[i].args = slots + reinterpret_cast<size_t>(seq[i].args);
-    }
+    c10::SmallVector<ftr_launch_desc_t, kInlineLaunches> seq(self->launches->begin(), self->launches->end());
+    const int nl = static_cast<int>(seq.size());
+    for (ftr_launch_desc_t &d : seq) d.args = slots.data() + reinterpret_cast<size_t>(d.args);
     void *stream = c10::hip::getCurrentHIPStream().stream();
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = self->launch_seq(seq, nl, stream);
+    rc = self->launch_seq(seq.data(), nl, stream);
     Py_END_ALLOW_THREADS
     if (rc != 0) {
         PyErr_Format(self->error, "ftr_launch_seq: %s", self->last_error());
@@ -111,7 +110,7 @@ bool dtype_of(const char *name, c10::ScalarType &out) {
 }
 
 // Call(launch_seq, last_error, error, [(dtype, shape)...], [(module, grid, block, lds_bytes, [(tensor, value)...])...]);
-// raises ValueError for what does not fit the fixed sizes above
+// raises ValueError for a type it does not know and for an argument that names no buffer
 PyObject *create(PyTypeObject *type, PyObject *args, PyObject *) {
     unsigned long long launch_seq, last_error;
     PyObject *error, *bufs, *launches;
@@ -153,9 +152,8 @@ PyObject *create(PyTypeObject *type, PyObject *args, PyObject *) {
         }
         self->launches->push_back(d);
     }
-    if (!ok || PyErr_Occurred() || self->bufs->size() > kMaxBufs || self->launches->size() > kMaxLaunches ||
-        self->args->size() > kMaxArgs) {
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "_ftcall.Call: not a plan it can hold");
+    if (!ok || PyErr_Occurred()) {
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "_ftcall.Call: unknown type or buffer index");
         Py_DECREF(self);
         return nullptr;
     }

@@ -253,3 +253,26 @@ def test_a_plan_called_by_threads_on_streams():
     torch.cuda.synchronize()
     for a, b, c in sets:
         assert torch.allclose(c, a @ b, atol=1e-4)
+
+
+@pytest.mark.parametrize("n", [15, 22])
+def test_a_plan_of_many_operators(n):
+    """More buffers and launches than a call keeps on its stack: the native call and the general one agree, and with
+    the product in float64 to n stages of |fl(xW) - xW| <= K u |x||W| (2-norms; W orthogonal, | |W| | <= sqrt(K))."""
+    import torch
+    from test_host_scheduler import chain_of_gemms
+    m, k = 20, 24
+    f, _ = build_config(lambda: chain_of_gemms(n, m, k), (), None)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    ws = [np.linalg.qr(rng.standard_normal((k, k)))[0].astype(np.float32) for _ in range(n)]
+    tensors = [placed(a) for a in [x] + ws]
+    outs = [torch.full((m, k), -7.0, device="cuda") for _ in range(2)]
+    assert f._native(*tensors, outs[0]) is True
+    f._native = None
+    f(*tensors, outs[1])
+    assert torch.equal(outs[0], outs[1])
+    want = x.astype(np.float64)
+    for w in ws:
+        want = want @ w
+    assert np.linalg.norm(outs[0].cpu().numpy() - want) <= n * k * k ** 0.5 * 2.0 ** -24 * np.linalg.norm(want)

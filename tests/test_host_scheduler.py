@@ -654,3 +654,44 @@ def test_untuned_operators_lower_under_every_lds_layout(lds_pad):
         s, _ = schedule_with_config_ops([out.op], bufs + [out], Config([], {"inline": [], "merge": [], "special": [pad]}),
                                         special_names=["lds_pad"])
         assert s.specs[-1].defines.get("APAD", s.specs[-1].defines.get("PAD")) in (pad[0], pad[0] * 4)
+
+
+def chain_of_gemms(n, m=20, k=24):
+    """n products in a row, x W1 .. Wn: (ops, bufs)."""
+    from flextensor_amd import nn
+    from flextensor_amd.te import placeholder
+    c, bufs = placeholder((m, k), name="X"), []
+    bufs.append(c)
+    for i in range(n):
+        bufs.append(placeholder((k, k), name="W%d" % i))
+        c = nn.gemm(c, bufs[-1])
+    return [c.op], bufs + [c]
+
+
+@pytest.mark.parametrize("n", [14, 15, 16, 17, 22])
+def test_the_native_call_holds_plans_of_any_length(n):
+    """A plan's launches laid out for the native call, on both sides of what a call keeps on its stack (16 buffers,
+    16 launches, 64 arguments)."""
+    from flextensor_amd import _ftcall, runtime as rt
+    from flextensor_amd.plan import BuiltPlan
+    from flextensor_amd.scheduler import schedule_with_config_ops
+
+    class Loaded(object):
+        class handle(object):
+            value = 0
+
+    class Scratch(object):
+        def data_ptr(self):
+            return 0
+
+    plan, _ = schedule_with_config_ops(*chain_of_gemms(n), Config([], None))
+    assert len(plan.specs) == n and len(plan.bufs) == n + 2
+    built = BuiltPlan.__new__(BuiltPlan)
+    built.plan, built.modules = plan, [Loaded] * n
+    built.scratch = dict((name, Scratch()) for name in plan.intermediates)
+    assert isinstance(built._native_call(), _ftcall.Call)
+    launch = (0, (1, 1, 1), (64, 1, 1), 0)
+    args = rt.address("ftr_launch_seq"), rt.address("ftr_last_error"), rt.RuntimeError_, [("float32", (2, 2))]
+    _ftcall.Call(*args, [launch + ([(0, 0)] * 70,)])
+    with pytest.raises(ValueError):
+        _ftcall.Call(*args, [launch + ([(1, 0)],)])            # names no buffer
