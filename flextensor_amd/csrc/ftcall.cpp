@@ -1,14 +1,15 @@
 // _ftcall: the call of a built plan, natively.
 //
-// A call checks its tensors (type, shape, place, contiguity), puts their addresses into the argument arrays of
+// A call checks its tensors (type, shape, place, contiguity, alignment), puts their addresses into the argument arrays of
 // the plan's launches and hands these to ftr_launch_seq on torch's current stream. In Python that took 16 us a
 // call (ctypes objects for every argument and descriptor, made anew each time), more than most kernels of a
 // single layer: back to back, a 3x3 layer on 1x64x56x56 now takes its 5.1 us on the device instead of 15.7, a depthwise layer
 // on 8x512x28x28 4.9 instead of 15.8. Everything but the addresses is laid out once, when the plan is built; a
 // call's argument arrays are its own, so several threads may call one plan.
 //
-// A call returns True when the work is enqueued and False when the tensors are not what the plan takes or are not
-// plain tensors: the caller then goes the general way, which says what is wrong.
+// A call returns True when the work is enqueued and False when the tensors are not what the plan takes, begin at an
+// address its kernels do not load from or are not plain tensors: the caller then goes the general way, which copies
+// what is misplaced and says what is wrong.
 #include "ftrocm.h"
 
 #include <Python.h>
@@ -27,6 +28,7 @@ typedef const char *(*last_error_t)(void);
 struct Buffer {
     c10::ScalarType dtype;
     std::vector<int64_t> shape;
+    unsigned align;          // the address is a multiple of it
 };
 
 struct Arg {
@@ -65,6 +67,7 @@ PyObject *call(PyObject *self_, PyObject *const *argv, size_t nargsf, PyObject *
         const at::Tensor &t = THPVariable_Unpack(argv[i]);
         if (!fits(t, (*self->bufs)[i])) Py_RETURN_FALSE;
         ptr[i] = t.data_ptr();
+        if (reinterpret_cast<uintptr_t>(ptr[i]) % (*self->bufs)[i].align) Py_RETURN_FALSE;
     }
     const std::vector<Arg> &args = *self->args;
     c10::SmallVector<unsigned long long, kInlineArgs> values(args.size());
@@ -109,7 +112,7 @@ bool dtype_of(const char *name, c10::ScalarType &out) {
     return false;
 }
 
-// Call(launch_seq, last_error, error, [(dtype, shape)...], [(module, grid, block, lds_bytes, [(tensor, value)...])...]);
+// Call(launch_seq, last_error, error, [(dtype, shape, align)...], [(module, grid, block, lds_bytes, [(tensor, value)...])...]);
 // raises ValueError for a type it does not know and for an argument that names no buffer
 PyObject *create(PyTypeObject *type, PyObject *args, PyObject *) {
     unsigned long long launch_seq, last_error;
@@ -131,7 +134,8 @@ PyObject *create(PyTypeObject *type, PyObject *args, PyObject *) {
         const char *name;
         PyObject *shape;
         Buffer b;
-        ok = PyArg_ParseTuple(PyList_GET_ITEM(bufs, i), "sO!", &name, &PyTuple_Type, &shape) && dtype_of(name, b.dtype);
+        ok = PyArg_ParseTuple(PyList_GET_ITEM(bufs, i), "sO!I", &name, &PyTuple_Type, &shape, &b.align) &&
+             dtype_of(name, b.dtype) && b.align > 0;
         for (Py_ssize_t d = 0; ok && d < PyTuple_GET_SIZE(shape); ++d)
             b.shape.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(shape, d)));
         self->bufs->push_back(b);

@@ -109,6 +109,12 @@ def current_stream():
     return int(torch.cuda.current_stream().cuda_stream)
 
 
+def _placed(tensor, align):
+    """The tensor, or a copy of it (enqueued on the current stream) where its address is no multiple of ``align``:
+    an int8 slice may begin at any byte."""
+    return tensor if tensor.data_ptr() % align == 0 else tensor.clone()
+
+
 class BuiltPlan(object):
     """Loaded kernels of a plan; call it with device tensors in ``bufs`` order."""
 
@@ -164,8 +170,18 @@ class BuiltPlan(object):
                     args.append((-1, int(v) & (0xffffffffffffffff if kind == "i64" else 0xffffffff)))
             grid, block = [tuple(int(x) for x in g) + (1,) * (3 - len(g)) for g in (spec.grid, spec.block)]
             launches.append((mod.handle.value, grid, block, int(spec.lds_bytes), args))
-        bufs = [(b.dtype, tuple(int(e) for e in b.shape)) for b in self.plan.bufs]
+        align = self._align()
+        bufs = [(b.dtype, tuple(int(e) for e in b.shape), align.get(name, 1))
+                for name, b in zip(self.plan.buf_names, self.plan.bufs)]
         return _ftcall.Call(rt.address("ftr_launch_seq"), rt.address("ftr_last_error"), rt.RuntimeError_, bufs, launches)
+
+    def _align(self):
+        """Name of a caller's buffer -> bytes its address has to be a multiple of."""
+        out = {}
+        for spec in self.plan.specs:
+            for name, n in spec.align.items():
+                out[name] = max(n, out.get(name, 1))
+        return out
 
     def attrs(self):
         return [m.attrs() for m in self.modules]
@@ -187,6 +203,7 @@ class BuiltPlan(object):
         """Launch descriptors of one run over ``tensors`` (validated)."""
         self._check(tensors)
         named = dict(zip(self.plan.buf_names, tensors))
+        named.update((name, _placed(named[name], n)) for name, n in self._align().items() if name in named)
         named.update(self.scratch)
         out = []
         self._binds = []
@@ -206,7 +223,7 @@ class BuiltPlan(object):
                     vals.append(ctypes.c_longlong(int(v)))
                 else:
                     raise ValueError("unknown argument kind %s" % kind)
-            out.append(rt.Launch(mod, spec.grid, spec.block, vals, spec.lds_bytes))
+            out.append(rt.Launch(mod, spec.grid, spec.block, vals, spec.lds_bytes, keep=named))
         return out
 
     def __call__(self, *tensors):

@@ -363,9 +363,11 @@ class Module(object):
 
 
 class Launch(object):
-    """One kernel launch of a plan: module, geometry, packed arguments."""
+    """One kernel launch of a plan: module, geometry, packed arguments. ``keep``: what has to live as long as the
+    addresses among the arguments are used."""
 
-    def __init__(self, module, grid, block, args, lds_bytes=0):
+    def __init__(self, module, grid, block, args, lds_bytes=0, keep=None):
+        self.keep = keep
         self.module = module
         self.grid = tuple(int(x) for x in grid)
         self.block = tuple(int(x) for x in block)

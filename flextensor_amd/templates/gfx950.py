@@ -58,10 +58,13 @@ class KernelSpec(object):
     args         list of argument descriptors: ("buf", name) for a device
                  buffer bound by the plan, ("i32", value) / ("i64", value) /
                  ("u32", value) for scalars
+    align        dict buffer name -> bytes its address has to be a multiple of, where that is
+                 more than its type's size
     """
 
     def __init__(self, template, kernel, defines, grid, block, args, lds_bytes=0, note="",
-                 workspace=None):
+                 workspace=None, align=None):
+        self.align = dict(align or {})
         # name -> (shape, dtype) of zero-initialised device buffers the plan
         # owns and the kernel leaves zeroed where it relies on zeros
         self.workspace = dict(workspace or {})
@@ -436,8 +439,11 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
         if waves_k > 1:
             D.update(WAVES_K=waves_k)
         grid = (gm * gn * splitk, 1, 1)
+        # rows of whole dwords are loaded as they lie, which takes operands that begin at a dword; for other K the
+        # kernel shifts every chunk by the byte it begins at, the operand's own included
+        align = {} if view.K % 4 else dict.fromkeys(in_names[:2], 4)
         specs.append(KernelSpec("gemm_i8.hip", "gemm_i8", D, grid, (nt * waves_k, 1, 1),
-                                [("buf", in_names[0]), ("buf", in_names[1]), ("buf", out_name)]))
+                                [("buf", in_names[0]), ("buf", in_names[1]), ("buf", out_name)], align=align))
         return specs
 
     kblk = 4 * (64 // mfm)

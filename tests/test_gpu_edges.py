@@ -64,14 +64,15 @@ def placed(array, offset=0):
     (64, 2080, 192), (32, 1000, 32), (520, 144, 514), (1030, 112, 1026)])
 def test_int8_rows_at_any_byte(oracle, m, k, n):
     """K of every alignment (16-byte rows straight into LDS, dword-aligned rows, rows that begin at any byte),
-    tails inside a 16-byte chunk, and operands that begin at an odd address themselves."""
+    tails inside a 16-byte chunk, and operands that begin at an odd address themselves (copied where the rows are whole
+    dwords) or at a dword that begins no 16 bytes."""
     import torch
     from flextensor_amd.task import gemm_int8
     f, _ = build_default(gemm_int8, "gemm", (m, k, n))
     rng = np.random.default_rng(m * 7 + k * 3 + n)
     a, b = [rng.integers(-128, 128, size=s, dtype=np.int8) for s in ((m, k), (n, k))]
     want = oracle.gemm_i8_c(a, b)
-    for oa, ob in ((0, 0), (1, 3), (2, 1)) if k % 4 else ((0, 0),):
+    for oa, ob in ((0, 0), (1, 3), (2, 1), (4, 8)):
         c = torch.full((m, n), -7, dtype=torch.int32, device="cuda")
         f(placed(a, oa), placed(b, ob), c)
         assert np.array_equal(c.cpu().numpy(), want), (oa, ob)

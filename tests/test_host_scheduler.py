@@ -691,7 +691,35 @@ def test_the_native_call_holds_plans_of_any_length(n):
     built.scratch = dict((name, Scratch()) for name in plan.intermediates)
     assert isinstance(built._native_call(), _ftcall.Call)
     launch = (0, (1, 1, 1), (64, 1, 1), 0)
-    args = rt.address("ftr_launch_seq"), rt.address("ftr_last_error"), rt.RuntimeError_, [("float32", (2, 2))]
+    args = rt.address("ftr_launch_seq"), rt.address("ftr_last_error"), rt.RuntimeError_, [("float32", (2, 2), 1)]
     _ftcall.Call(*args, [launch + ([(0, 0)] * 70,)])
     with pytest.raises(ValueError):
         _ftcall.Call(*args, [launch + ([(1, 0)],)])            # names no buffer
+
+
+@pytest.mark.parametrize("k", [64, 68, 67])
+def test_int8_operands_that_begin_inside_a_dword_are_moved(k):
+    """Rows of whole dwords are loaded as they lie: the kernel gets addresses of whole dwords, of a copy where the
+    caller's operand begins elsewhere. Rows of other lengths may begin anywhere."""
+    import torch
+    from flextensor_amd.plan import BuiltPlan
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.task import gemm_int8
+
+    class Loaded(object):
+        handle = 0
+
+    plan, _ = schedule_with_config_ops(*gemm_int8(32, k, 48), Config([], None))
+    built = BuiltPlan.__new__(BuiltPlan)
+    built.plan, built.modules, built.scratch, built.static_layout = plan, [Loaded], {}, None
+    built._check = lambda tensors: None                # the tensors of this test lie on the host
+    flat = torch.arange(4096, dtype=torch.int32).to(torch.int8)
+    c = torch.empty(32, 48, dtype=torch.int32)
+    for oa, ob in ((0, 0), (1, 3), (2, 0), (4, 8)):
+        a, b = flat[oa:oa + 32 * k].view(32, k), flat[ob:ob + 48 * k].view(48, k)
+        launch, = built.launches((a, b, c))
+        for tensor, arg, name in zip((a, b, c), launch.pack.values, plan.buf_names):
+            assert (arg.value == tensor.data_ptr()) == (k % 4 != 0 or tensor.data_ptr() % 4 == 0)
+            assert arg.value == launch.keep[name].data_ptr() and torch.equal(launch.keep[name], tensor)
+            assert k % 4 or arg.value % 4 == 0
+    assert built._align() == ({} if k % 4 else {"in0": 4, "in1": 4})
