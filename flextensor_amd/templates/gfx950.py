@@ -1014,7 +1014,7 @@ def default_config(op, padded=False):
         # stride 1 and 2) this is 4 % off the best of 1 .. 8 rows and 1 .. 4 wavefronts in the geometric mean, 4 rows
         # and 4 wavefronts everywhere are 19 % off: 17x413x66x20 5x5 stride 2 33.9 -> 17.6 us.
         tw = 4 if q >= 4 else 1
-        th = min(4 if op.attrs["stride"][0] == 1 else 3, p)
+        th = max(1, min(4 if op.attrs["stride"][0] == 1 else 3, p))        # no rows at all: refused in the lowering
         while th > 1 and b * c * ceil_div(p, th) * ceil_div(q, tw) < 64 * 4 * NUM_CUS:
             th //= 2
         cfg["spatial"] = [[b, 1, 1, 1], [c, 1, 1, 1], [ceil_div(p, th), 1, 1, th],

@@ -723,3 +723,13 @@ def test_int8_operands_that_begin_inside_a_dword_are_moved(k):
             assert arg.value == launch.keep[name].data_ptr() and torch.equal(launch.keep[name], tensor)
             assert k % 4 or arg.value % 4 == 0
     assert built._align() == ({} if k % 4 else {"in0": 4, "in1": 4})
+
+
+@pytest.mark.parametrize("args", [(7, 2, 2, 5, 1, 3, 3, 0, 1), (1, 2, 5, 2, 1, 3, 1, 0, 1)])
+def test_a_depthwise_layer_without_rows_or_columns_is_refused(args):
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.task import depthwise_conv2d
+    from flextensor_amd.templates.gfx950 import InvalidConfig
+    ops, bufs = depthwise_conv2d(*args)
+    with pytest.raises(InvalidConfig):
+        schedule_with_config_ops(ops, bufs, Config([], None))
