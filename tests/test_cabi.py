@@ -73,3 +73,21 @@ def test_every_template_compiles_for_gfx950():
             assert code[:4] == b"\x7fELF"
     from flextensor_amd.templates import gfx950
     assert rt.compile_to_code(gfx950.template_source("naive.hip"), [])[:4] == b"\x7fELF"
+
+
+def test_build_makes_the_extension_for_the_interpreter_that_runs_it(monkeypatch):
+    """The native call is an extension of one interpreter and its torch: not of whichever python3 is on PATH."""
+    import sys
+    import __graft_entry__ as entry
+
+    class Stop(Exception):
+        pass
+
+    def check_call(cmd, **kwargs):
+        raise Stop(cmd)
+
+    monkeypatch.setattr(entry.subprocess, "check_call", check_call)
+    monkeypatch.setattr(sys, "executable", "/some/other/python")
+    with pytest.raises(Stop) as e:
+        entry.build()
+    assert "PYTHON=/some/other/python" in e.value.args[0]
