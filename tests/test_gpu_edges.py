@@ -256,6 +256,42 @@ def test_a_plan_called_by_threads_on_streams():
         assert torch.allclose(c, a @ b, atol=1e-4)
 
 
+@pytest.mark.parametrize("native", [True, False])
+def test_a_call_runs_on_the_current_stream(native):
+    """Each stream is busy for milliseconds before it writes the operand the call reads: a launch on any other
+    stream would read the operand as it was, and its result would be taken before it is there."""
+    import threading
+    import torch
+    f, _ = build_config(gemm_of(False), (96, 64, 80), None)
+    if not native:
+        f._native = None
+    busy = torch.randn(2048, 2048, device="cuda")
+    sets = [[torch.randn(96, 64, device="cuda"), torch.randn(64, 80, device="cuda"),
+             torch.zeros(96, 64, device="cuda"), torch.zeros(96, 80, device="cuda")] for _ in range(3)]
+    streams, results = [torch.cuda.Stream() for _ in sets], [None] * len(sets)
+    busy @ busy
+    torch.cuda.synchronize()
+
+    def work(i):
+        new, b, a, c = sets[i]
+        with torch.cuda.stream(streams[i]):
+            for _ in range(20):
+                busy @ busy
+            a.copy_(new)
+            f(a, b, c)
+            results[i] = c.clone()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sets))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for (new, b, a, c), got in zip(sets, results):
+        want = new.double() @ b.double()
+        assert close(got.cpu().numpy(), want.cpu().numpy())
+
+
 @pytest.mark.parametrize("n", [15, 22])
 def test_a_plan_of_many_operators(n):
     """More buffers and launches than a call keeps on its stack: the native call and the general one agree, and with
