@@ -849,7 +849,10 @@ def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups):
     overlap = {1: 0.2, 2: 0.8, 3: 0.4, 5: 0.3, 8: 0.35}[depth]      # share of a step's own MFMAs the chain waits for
     turns = ceil_div(share, beside)
     chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap) + 930)
-    operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / 31
+    # workgroups are renumbered by XCD where their count is a multiple of 8; where it is not, a batch's panels are
+    # fetched by all eight L2s
+    rate = 31 if view.groups == 1 or tiles % 8 == 0 else 14
+    operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
     longest = max(matrix, chain, operands)
     return (longest + 0.35 * (matrix + chain + operands - longest) + share * bm * bn * 4 * 4.8 / 64
             + (38 * rm * rn * mf * mf / 64 * (groups - 1)))
@@ -867,7 +870,10 @@ def _default_f32(view, padded=False):
     sizes (M, N, K 8 .. 4096, batches of 26 .. 128; half of them no multiples of 4); the pick is within 5 % of the
     best measured in the geometric mean and 1.6 times as fast as the rule before it (square-ish power-of-two
     tiles until every unit has one, K tiles of 32): 1100x1301x900 47.1 -> 30.0 us, 863x1862x1280 (B^T) 69.7 ->
-    44.4, 96 x 74x96x133 6.8 -> 5.4, 32x4096x3072 43.6 -> 16.5. K streaming is left to the search: a plan that owns a
+    44.4, 96 x 74x96x133 6.8 -> 5.4, 32x4096x3072 43.6 -> 16.5. Batches whose tiles are no multiple of 8 go at the rate
+    of grids that are not renumbered (14 bytes per clock and unit; 86 batches measured: 3.8 % off the best kernel, with
+    one rate for all 11.5 % off and up to 1.5 times as slow as the rule before): 121 x 35x80x124 6.33 -> 4.16 us,
+    114 x 68x110x63 (B^T) 6.38 -> 4.88, 63 x 52x80x274 7.01 -> 5.21. K streaming is left to the search: a plan that owns a
     workspace cannot run on two streams at once, and a default plan can.
     """
     return _pick_f32(view, F32_KERNELS, _f32_clocks, padded)

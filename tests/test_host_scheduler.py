@@ -733,3 +733,18 @@ def test_a_depthwise_layer_without_rows_or_columns_is_refused(args):
     ops, bufs = depthwise_conv2d(*args)
     with pytest.raises(InvalidConfig):
         schedule_with_config_ops(ops, bufs, Config([], None))
+
+
+@pytest.mark.parametrize("args", [
+    (121, 35, 80, 124, False), (63, 52, 80, 274, False), (76, 34, 128, 138, False), (36, 45, 80, 199, False),
+    (114, 68, 110, 63, True), (92, 33, 64, 172, False), (33, 239, 96, 40, False), (76, 141, 48, 196, False)])
+def test_untuned_batches_get_a_grid_that_is_renumbered_by_xcd(args):
+    """Grids of no multiple of 8 workgroups keep no XCD locality; with the kernel that was best but for that, these batches
+    ran 1.2 to 1.7 times as long as with one whose tiles are a multiple of 8."""
+    from flextensor_amd import nn
+    from flextensor_amd.te import placeholder
+    from flextensor_amd.templates import gfx950
+    b, m, k, n, trans_b = args
+    c = nn.batch_gemm(placeholder((b, m, k)), placeholder((b, n, k) if trans_b else (b, k, n)), transposeB=trans_b)
+    spatial = gfx950.untuned_config(c.op)["spatial"]
+    assert b * spatial[0][0] * spatial[1][0] % 8 == 0
