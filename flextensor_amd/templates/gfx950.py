@@ -933,9 +933,13 @@ def _default_conv(view, padded=False):
     channel, tap and padding predicate are computed anew for every element of every tile, about 50 clocks per 64 of
     them, and an untiled 3x3 layer spends more on that than on its products. Whole windows pay where tiles are many;
     with few tiles K is divided over wavefront groups instead, which shortens the serial chain of k steps.
-    Constants fitted to 3 600 timings over 45 layers (1 .. 16 images, 16 .. 512 channels, 7 .. 112 rows; 1x1 and
-    3x3, stride 1 and 2); the pick is within 7 % of the best measured kernel in the geometric mean, the rule before it
-    (square-ish power-of-two tiles until every unit has one, K tiles of up to 32, K undivided) 1.77 times off.
+    Checked against 3 200 timings over 180 layers (1 .. 16 images, 16 .. 512 channels, 7 .. 112 rows; 1x1 and
+    3x3, stride 1 and 2): the pick is 8 % off the best measured kernel in the geometric mean (1x1 5 %, 3x3 9 %; 1.57
+    times for the worst layer), the rule before it (square-ish power-of-two tiles until every unit has one, K tiles of up
+    to 32, K undivided) 1.86 times off. Above 4 microseconds the pick is 2 to 5 % slower than that rule's for six of the
+    layers; near the floor of a launch the two differ by up to 0.45 microseconds either way. Pointwise layers whose tiles are no multiple of 8 go at
+    the rate of grids that are not renumbered by XCD: 4 x 464x49x49 -> 48 stride 2 11.96 -> 7.93 us, 8 x 144x30x30 -> 192
+    stride 2 6.84 -> 5.09, 15 x 131x21x21 -> 45 5.42 -> 4.29 (with one rate up to 15 % slower than the rule before).
     """
     window = view.conv["CR"] * view.conv["CS"]
 
@@ -956,7 +960,8 @@ def _default_conv(view, padded=False):
         overlap = {2: 0.8, 3: 0.4, 5: 0.3, 8: 0.35}[depth]
         compute = ceil_div(share * nw, 4) * step * steps + share * steps * gathered * (3.7 if hoisted else 51.6) / 4
         chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap + (0 if hoisted else 80 * gathered / nw)) + 3230)
-        operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / 16
+        rate = 16 if window > 1 or tiles % 8 == 0 else 9        # as in _f32_clocks; only one-pixel windows show it
+        operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
         longest = max(compute, chain, operands)
         return (longest + 0.47 * (compute + chain + operands - longest) + share * bm * bn * 4 * 3.0 / 64
                 + 82 * rm * rn * mf * mf / 64 * (groups - 1))

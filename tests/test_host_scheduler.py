@@ -748,3 +748,17 @@ def test_untuned_batches_get_a_grid_that_is_renumbered_by_xcd(args):
     c = nn.batch_gemm(placeholder((b, m, k)), placeholder((b, n, k) if trans_b else (b, k, n)), transposeB=trans_b)
     spatial = gfx950.untuned_config(c.op)["spatial"]
     assert b * spatial[0][0] * spatial[1][0] % 8 == 0
+
+
+@pytest.mark.parametrize("args", [
+    (8, 144, 30, 30, 192, 1, 2, 0, 1, 1), (15, 131, 21, 21, 45, 1, 1, 0, 1, 1), (4, 464, 49, 49, 48, 1, 2, 0, 1, 1),
+    (8, 227, 30, 30, 273, 1, 2, 0, 1, 1)])
+def test_untuned_pointwise_layers_get_larger_tiles_where_the_grid_is_not_renumbered(args):
+    """The tiles of these layers are no multiple of 8, so every XCD fetches the operands: 32x32 and 16x16 tiles with
+    their larger traffic ran 1.2 to 1.5 times as long as the next larger one."""
+    from flextensor_amd.scheduler import flatten_graph
+    from flextensor_amd.task import conv2d
+    from flextensor_amd.templates import gfx950
+    op, = [o for o in flatten_graph(conv2d(*args)[0])[0] if o.kind == "conv2d_nchw"]
+    (tm, wm, rm, mf), (tn, wn, rn, _) = gfx950.untuned_config(op)["spatial"]
+    assert wm * rm * mf * wn * rn * mf >= (64 * 32 if args[1] != 464 else 32 * 32)
