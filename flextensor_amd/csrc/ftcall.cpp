@@ -5,7 +5,8 @@
 // call (ctypes objects for every argument and descriptor, made anew each time), more than most kernels of a
 // single layer: back to back, a 3x3 layer on 1x64x56x56 now takes its 5.1 us on the device instead of 15.7, a depthwise layer
 // on 8x512x28x28 4.9 instead of 15.8. Everything but the addresses is laid out once, when the plan is built; a
-// call's argument arrays are its own, so several threads may call one plan.
+// call's argument arrays are its own, so several threads may call one plan, and on several streams where the plan
+// owns no buffers: its intermediates and workspaces exist once, and calls that use them must not overlap on the device.
 //
 // A call returns True when the work is enqueued and False when the tensors are not what the plan takes, begin at an
 // address its kernels do not load from or are not plain tensors: the caller then goes the general way, which copies

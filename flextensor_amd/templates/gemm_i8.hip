@@ -149,7 +149,7 @@ typedef i32x4 acc_t;
 #define OOB 0x80000000u
 #define TILES_M ((M + BM - 1) / BM)
 #define TILES_N ((N + BN - 1) / BN)
-/* KP = K rounded up to a multiple of 64 (host checks KP % BK == 0); chunks
+/* KP = SPLITK * WAVES_K * (K tiles of a group) * BK, which covers K; chunks
  * beyond K are zero-filled by the load predicate. When K is no multiple of 16
  * the rows of A and B are not 16-byte aligned: a buffer load of 16 bytes needs
  * dword alignment only, which is enough for K % 4 == 0; otherwise a chunk is cut

@@ -391,8 +391,8 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
         if bk % mfma_k != 0:
             raise InvalidConfig("BK must be a multiple of the MFMA K extent")
         if view.K % 16 != 0 and depth >= 6:
-            # rows that are not 16-byte aligned: chunks are put together from dword or byte loads in
-            # registers, which the loads that write LDS directly cannot do
+            # a row's last chunk runs into the next row, and for K % 4 != 0 every chunk is cut out of five
+            # dwords: both happen in registers, which the loads that write LDS directly pass by
             raise InvalidConfig("int8 tiles straight into LDS need K to be a multiple of 16")
         pad = int(_special(special, "lds_pad")[0])
         pad = -1 if pad < 0 else pad * 4

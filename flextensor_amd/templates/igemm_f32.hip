@@ -230,8 +230,8 @@ typedef f32x4 acc_t;
 #endif
 #define TILES_M ((M + BM - 1) / BM)
 #define TILES_N ((N + BN - 1) / BN)
-/* KP = K, or K rounded up to a multiple of 16 when K % 8 != 0; the host checks KP % (SPLITK*BK) == 0.
- * When KP != K the tail is zero-filled by the load predicates. */
+/* KP = SPLITK * WAVES_K * (K tiles of a group) * BK: K itself, K rounded up to a multiple of 16, or the fewest whole
+ * tiles that cover K, up to a quarter more than K. When KP != K the tail is zero-filled by the load predicates. */
 #define KSPLIT_LEN (KP / SPLITK)
 #define KGROUP_LEN (KSPLIT_LEN / WAVES_K)
 #define KT (KGROUP_LEN / BK)
@@ -853,7 +853,8 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #pragma unroll
     for (int e = 0; e < EA; ++e) {
 #if TA
-        /* a_row = k inside the tile, a_col = first of AV consecutive rows m (M % AV == 0) */
+        /* a_row = k inside the tile, a_col = first of AV consecutive rows m; those beyond M belong to the next k and
+         * feed results that are not stored */
         const int m = m0 + a_col[e];
         bool ok = (A_CHUNKS % NT == 0) || (tid + e * NT < A_CHUNKS);
         if (M % BM != 0) ok = ok & (m < M);

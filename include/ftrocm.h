@@ -13,8 +13,9 @@
  *     owns every device buffer (plain device pointers) and must keep them
  *     alive until the call (or the stream work it enqueued) has finished.
  *   - no torch types, no C++ types: plain pointers and sizes only.
- *   - a module is not safe to use from two threads at once; distinct modules
- *     are independent.
+ *   - launches only read a module, so several threads may launch one at once
+ *     (each with argument arrays of its own); freeing it must not overlap
+ *     with them, nor with the work they enqueued.
  */
 #ifndef FTROCM_H
 #define FTROCM_H
