@@ -88,7 +88,7 @@ class KernelPlan(object):
 
 
 # templates that take the FT_CLKPROBE instrumentation
-PROBE_TEMPLATES = ("igemm_f32.hip", "gemm_i8.hip", "depthwise_f32.hip")
+PROBE_TEMPLATES = ("igemm_f32.hip", "direct_f32.hip", "gemm_i8.hip", "depthwise_f32.hip")
 
 
 _TORCH_DTYPES = None

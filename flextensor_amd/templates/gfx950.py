@@ -12,6 +12,8 @@ Operator kinds and the template each one lowers to:
   conv2d_nchw            igemm_f32.hip  MODE 1 (implicit GEMM, padding folded
                                          into the gather; or PAD=0 over a
                                          materialised padded tensor)
+  both and batch_gemm    direct_f32.hip (operands straight into registers, no LDS tiles: fourth number of the
+                                         reorder entry 1; chosen by the defaults, not searched)
   gemm_int8              gemm_i8.hip
   depthwise_conv2d_nchw  depthwise_f32.hip (direct; also what conv2d_nchw builds
                                          for one input channel per group)
@@ -354,8 +356,8 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
     # loads of the next tile are spread (1 = all in front of the tile's first MFMAs)
     load_spread = int((config.get("unroll") or [[2, 1]])[0][1]) if frag_prefetch else 1
     group_m = int((config.get("fuse") or [[4]])[0][0])
-    ro = list((config.get("reorder") or [[1, 0]])[0]) + [0, 0]
-    xcd, in_wg, stream_k = int(ro[0]), int(ro[1]), int(ro[2])
+    ro = list((config.get("reorder") or [[1, 0]])[0]) + [0, 0, 0]
+    xcd, in_wg, stream_k, direct = int(ro[0]), int(ro[1]), int(ro[2]), int(ro[3])
     i8 = view.dtype == "int8"
     waves_k = 1
     if in_wg and splitk > 1:
@@ -375,14 +377,17 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
     if nacc > MAX_ACC_REGS:
         raise InvalidConfig("accumulators need %d registers per lane" % nacc)
     kp = splitk * waves_k * kiters * bk
-    # the fewest whole tiles that cover K will do as well (zeros behind it): int8 always, fp32 up to a quarter more
-    if kp not in view.KP_options and not (view.K <= kp < view.K + splitk * waves_k * bk and (i8 or kp * 4 <= view.K * 5)):
+    # the fewest whole tiles that cover K will do as well (zeros behind it): int8 always, fp32 up to a quarter more;
+    # tiles without LDS multiply no zeros but give some groups of wavefronts fewer steps
+    if kp not in view.KP_options and not (view.K <= kp < view.K + splitk * waves_k * bk and (i8 or direct or kp * 4 <= view.K * 5)):
         raise InvalidConfig("reduce split does not multiply to K, nor to the fewest whole tiles that cover it")
     nt = wm * wn * 64          # threads of one k-group
     D = dict(M=view.M, N=view.N, K=view.K, KP=kp, MFMA=mfm, WAVES_M=wm, WAVES_N=wn, REP_M=rm,
              REP_N=rn, BK=bk, STAGES=stages, GROUP_M=group_m, XCD_REMAP=xcd)
 
     if i8:
+        if direct:
+            raise InvalidConfig("operands straight into registers are an fp32 path")
         if stream_k:
             # the grid-level split (integer atomics: exact, any order) and the in-workgroup split
             # cover the int8 operator; the balanced K streaming protocol is an fp32 path
@@ -445,6 +450,13 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
         specs.append(KernelSpec("gemm_i8.hip", "gemm_i8", D, grid, (nt * waves_k, 1, 1),
                                 [("buf", in_names[0]), ("buf", in_names[1]), ("buf", out_name)], align=align))
         return specs
+
+    if direct:
+        if mfm != 16 or bk != 32 or splitk > 1 or stream_k:
+            raise InvalidConfig("operands straight into registers: 16x16 tiles, k steps of 32, K divided inside the "
+                                "workgroup only")
+        return _lower_direct(op, view, D, direct, depth, out_name, in_names, materialized_pad, bias_name, merged_out,
+                             waves_k=waves_k)
 
     kblk = 4 * (64 // mfm)
     if bk % kblk != 0:
@@ -577,6 +589,53 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
     specs.append(KernelSpec("igemm_f32.hip", "igemm_f32", D, grid, (nt * waves_k, 1, 1), args,
                             workspace=workspace))
     return specs
+
+
+def _lower_direct(op, view, D, direct, depth, out_name, in_names, materialized_pad, bias_name, merged_out, waves_k):
+    """Tiles whose operands go straight into registers (direct_f32.hip)."""
+    if direct != 1:
+        raise InvalidConfig("no variant %d of the tiles without LDS" % direct)
+    if view.trans_a or view.K < 32:
+        raise InvalidConfig("operands straight into registers need a K of 32 and more and A stored [M][K]")
+    waves, rm, rn = D["WAVES_M"] * D["WAVES_N"] * waves_k, D["REP_M"], D["REP_N"]
+    if view.mode == 0 and rn not in (1, 2, 4):
+        raise InvalidConfig("a lane's neighbouring columns are one load: 1, 2 or 4 blocks")
+    if view.mode == 1 and view.conv["CR"] * view.conv["CS"] > 31:
+        raise InvalidConfig("a pixel's valid taps are bits of a word")
+    steps = ceil_div(view.K, 32)
+    pd = min(depth, ceil_div(steps, waves_k))          # no group loads more steps ahead than it has
+    regs = 4 * rm * rn + 8 * (rm + rn) * pd + rm + 2 * rn + 24
+    if pd > 4 or regs > (256 if waves <= 8 else 128):
+        raise InvalidConfig("the tile and its loads need %d registers per lane" % regs)
+    # one after the other in the same LDS: the offsets of the gathered operand's k, the groups' partial sums
+    if max(waves * rm * rn * 1024 if waves_k > 1 else 0, steps * 32 * 8 if view.mode == 1 else 0) + 16 > LDS_BYTES:
+        raise InvalidConfig("partial sums or the offsets of a gathered operand need more than %d bytes" % LDS_BYTES)
+    D = {k: D[k] for k in ("M", "N", "K", "WAVES_M", "WAVES_N", "REP_M", "REP_N", "GROUP_M")}
+    D.update(MODE=view.mode, WAVES_K=waves_k, PD=pd)
+    a_name, b_name = in_names[0], in_names[1]
+    b_bytes = view.groups * view.K * view.N * 4
+    if view.mode == 1:
+        conv = dict(view.conv)
+        if materialized_pad:
+            conv["CH"] += 2 * conv["CPADH"]
+            conv["CW"] += 2 * conv["CPADW"]
+            conv["CPADH"] = conv["CPADW"] = 0
+        D.update(conv)
+        b_bytes = conv["CB"] * conv["CC"] * conv["CH"] * conv["CW"] * 4
+        if op.kind == "col_gemm" and merged_out is None:
+            D.update(COLOUT=1)
+    elif view.groups > 1:
+        D.update(CG=view.groups)
+    if op.kind in ("col_gemm", "conv2d_nchw"):
+        a_name, b_name = b_name, a_name          # A = weight, B = the image or the stored columns
+    if max(view.groups * view.M * view.K * 4, b_bytes, view.groups * view.M * view.N * 4) >= 2 ** 31:
+        raise InvalidConfig("operands of 2 GiB or more are not addressable by the buffer loads")
+    args = [("buf", a_name), ("buf", b_name), ("buf", out_name)]
+    if bias_name is not None:
+        D.update(HAS_BIAS=1)
+        args.append(("buf", bias_name))
+    tiles = ceil_div(view.M, D["WAVES_M"] * rm * 16) * ceil_div(view.N, D["WAVES_N"] * rn * 16)
+    return [KernelSpec("direct_f32.hip", "igemm_f32", D, (tiles * view.groups, 1, 1), (waves * 64, 1, 1), args)]
 
 
 def _lower_depthwise(op, config, special, out_name, in_names, materialized_pad=False, bias_name=None):
@@ -858,7 +917,7 @@ def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups):
             + (38 * rm * rn * mf * mf / 64 * (groups - 1)))
 
 
-def _default_f32(view, padded=False):
+def _default_f32(view, padded=False, direct=True):
     """Tile, K tile, pipeline and K division of an fp32 GEMM (or a batch of them) nobody tuned: the smallest
     predicted time over F32_KERNELS, which between them are within 2 % of the best measured kernel everywhere.
 
@@ -876,14 +935,44 @@ def _default_f32(view, padded=False):
     114 x 68x110x63 (B^T) 6.38 -> 4.88, 63 x 52x80x274 7.01 -> 5.21. K streaming is left to the search: a plan that owns a
     workspace cannot run on two streams at once, and a default plan can.
     """
-    return _pick_f32(view, F32_KERNELS, _f32_clocks, padded)
+    return _pick_f32(view, F32_KERNELS, _f32_clocks, padded, direct)
 
 
-def _pick_f32(view, kernels, predict, padded):
+# kernels without LDS tiles that the defaults choose among: MFMA tiles per wavefront along M and N, k steps ahead
+DIRECT_KERNELS = ((1, 1, 2), (1, 2, 2), (2, 2, 2), (1, 4, 2))
+
+
+def _direct_clocks(view, m, n, pd, groups):
+    """Predicted clocks (2.38 GHz) of a call on tiles without LDS, the launch included; see _pick_f32."""
+    tiles = ceil_div(view.M, m * 16) * ceil_div(view.N, n * 16)
+    steps = ceil_div(ceil_div(view.K, 32), groups)
+    share = ceil_div(tiles, NUM_CUS)
+    beside = max(1, min(share, min(8, 512 // (4 * m * n + 8 * (m + n) * pd + 40)) * 4 // groups))
+    step = m * n * 256                                              # matrix clocks of a wavefront's k step
+    # clocks a unit spends on a step's loads: two vectors per row block; per column one float and k, or a vector
+    loads = 2 * m * 26 + (8 * n * 16.3 if view.conv else 8 * (26 if n == 4 else 13.6))
+    matrix = ceil_div(share * groups, 4) * steps * step
+    memory = share * groups * steps * loads
+    chain = (ceil_div(share, beside) * (steps * max(94.0 / pd + 0.19 * step, step) + 1500)
+             + (510.0 * view.K / (64 * groups) if view.conv else 0))
+    stream = (view.M * view.K + view.K * view.N) * 4 / 1930.0       # operands once at the rate of a large copy
+    longest = max(matrix, memory, chain)
+    return max(longest + 0.37 * (matrix + memory + chain - longest), stream) + share * m * n * 1024 * 1.9 / 64 + 4360
+
+
+def _pick_f32(view, kernels, predict, padded, direct):
     """The config of the kernel and number of wavefront K groups with the smallest predicted time; where the LDS
     rows are to be padded, among the kernels whose tiles pass through registers, with K undivided (the groups' tiles
-    lie beside each other in LDS)."""
+    lie beside each other in LDS).
+
+    Against it stand the tiles without LDS, which have to be predicted a tenth faster. The two predictions are off by
+    17 % (one standard deviation) each, fitted to 1 800 timings of the tiles without LDS and to the times of the other picks
+    over 132 operators (GEMMs and convolutions over the ranges above).
+    Not for 1x1 windows, whose gathers the LDS kernels do without index arithmetic (7 x 259x90x90 -> 25 16.4 us, 18.4
+    without LDS), and not for B stored [N][K] nor for batches: with few k steps the operands' latency is all there is, and tiles that share it
+    through LDS have it once (96 x 197x64x197 10.0 us, 14.5 without LDS; 57x1249x714 with B^T 5.3 and 7.0)."""
     best = None
+    window = view.conv["CR"] * view.conv["CS"] if view.conv else 1
     for m, n, mf, bk, depth in kernels:
         if padded and depth >= 5:
             continue
@@ -907,12 +996,34 @@ def _pick_f32(view, kernels, predict, padded):
             clocks = predict(view, tiles, m, n, mf, bk, depth, groups)
             if clocks is not None and (best is None or clocks < best[0]):
                 best = (clocks, [tm, m[0], m[1], mf], [tn, n[0], n[1], mf], [groups, steps, bk], depth)
+    if direct and view.groups == 1 and view.mode != 2 and not view.trans_a and view.K >= 32 \
+            and (not view.conv or 1 < window <= 31 and view.K * 8 + 256 < LDS_BYTES):
+        # the other prediction in clocks of a call (launch included), fitted to what its picks took
+        limit = (0.837 * best[0] + 4190 if view.conv else 1.02 * best[0] + 3750) / 1.1
+        if not view.conv and view.M <= 64:
+            # few rows of a large weight: where the weight's rows are no whole vectors the LDS kernels take 1.2 to 2 times
+            # what was predicted (57x1610x1067 14.9 us for 7.5), where they are it is right (32x4096x4096)
+            limit *= 0.88 if view.N % 4 == 0 and view.K % 4 == 0 else 1.4 if view.N * view.K > 1e6 else 1.0
+        for m, n, pd in DIRECT_KERNELS:
+            if m * 16 >= 2 * max(view.M, 16) or n * 16 >= 2 * max(view.N, 16):
+                continue
+            tm, tn = ceil_div(view.M, m * 16), ceil_div(view.N, n * 16)
+            if tm * tn * m * n * view.K * 8.0 / (4 * NUM_CUS) + 4360 > limit:          # matrix clocks alone
+                continue
+            for groups in (1, 2, 4, 8):
+                kp = ceil_div(view.K, 32 * groups) * 32 * groups
+                if groups > 1 and tm * tn > 3000 or tm * tn * groups < 128 or kp * 4 > view.K * 5 and kp not in view.KP_options:
+                    continue
+                clocks = _direct_clocks(view, m, n, pd, groups)
+                if clocks < limit:
+                    limit = clocks
+                    best = (clocks, [tm, 1, m, 16], [tn, 1, n, 16], [groups, kp // (32 * groups), 32], pd, 1)
     cfg = _empty_config()
     cfg["spatial"] = [best[1], best[2]]
     cfg["reduce"] = [best[3]]
     cfg["unroll"] = [[best[4], 1]]
     cfg["fuse"] = [[4]]
-    cfg["reorder"] = [[1, 1 if best[3][0] > 1 else 0, 0]]
+    cfg["reorder"] = [[1, 1 if best[3][0] > 1 else 0, 0] + list(best[5:])]
     return cfg
 
 
@@ -925,7 +1036,7 @@ CONV_WINDOW_KERNELS = (((1, 1), (1, 1), 16, 144, 8), ((2, 1), (2, 1), 16, 144, 8
                        ((2, 1), (2, 1), 32, 72, 8), ((4, 1), (2, 1), 32, 72, 8))
 
 
-def _default_conv(view, padded=False):
+def _default_conv(view, padded=False, direct=True):
     """Tile, K tile, pipeline and K division of a convolution nobody tuned, by predicted time like _default_f32.
 
     What differs from the plain product is the gathered operand. One float per lane and load, with its own address:
@@ -967,17 +1078,17 @@ def _default_conv(view, padded=False):
                 + 82 * rm * rn * mf * mf / 64 * (groups - 1))
 
     return _pick_f32(view, CONV_KERNELS + (CONV_WINDOW_KERNELS if window > 1 and 72 % window == 0 else ()),
-                     clocks, padded)
+                     clocks, padded, direct)
 
 
-def default_config(op, padded=False):
+def default_config(op, padded=False, direct=True):
     """A reasonable untuned config: the point a search begins with, and for all operators but the convolution
     what an untuned task runs on (untuned_config)."""
     cfg = _empty_config()
     if op.kind == "gemm_int8":
         return _default_i8(GemmView(op), padded)
     if op.kind in ("gemm", "batch_gemm"):
-        return _default_f32(GemmView(op), padded)
+        return _default_f32(GemmView(op), padded, direct)
     if op.kind in GEMM_KINDS:
         view = GemmView(op)
 
@@ -1037,11 +1148,13 @@ def default_config(op, padded=False):
 def untuned_config(op, special=None):
     """What schedule_with_config falls back to when a task has no tuned entry. The convolution's search keeps
     beginning at a square-ish tile with K undivided, beside which its other seed points lie. An LDS layout that
-    the graph config names (``special``) is one that tiles straight into LDS may not be able to have."""
+    the graph config names (``special``) is one that tiles straight into LDS may not be able to have, and that tiles
+    without LDS do not have at all."""
     padded = _special(special, "lds_pad") != SPECIAL_DEFAULTS["lds_pad"]
+    direct = not (special and "lds_pad" in special)
     if op.kind in ("conv2d_nchw", "col_gemm"):
-        return _default_conv(GemmView(op), padded)
-    return default_config(op, padded)
+        return _default_conv(GemmView(op), padded, direct)
+    return default_config(op, padded, direct)
 
 
 def seed_configs(op, limit=24):
