@@ -949,15 +949,21 @@ def _direct_clocks(view, m, n, pd, groups):
     share = ceil_div(tiles, NUM_CUS)
     beside = max(1, min(share, min(8, 512 // (4 * m * n + 8 * (m + n) * pd + 40)) * 4 // groups))
     step = m * n * 256                                              # matrix clocks of a wavefront's k step
-    # clocks a unit spends on a step's loads: two vectors per row block; per column one float and k, or a vector
-    loads = 2 * m * 26 + (8 * n * 16.3 if view.conv else 8 * (26 if n == 4 else 13.6))
+    # clocks a unit spends on a step's loads: two vectors per row block; per column one float and k (with a stride along
+    # the rows two lines where there was one), or a vector
+    if view.conv:
+        loads = 2 * m * 40 + 8 * n * (18.4 if view.conv["CSTRW"] > 1 else 9.5)
+        start, table, mix, store = 3330, 210.0 * view.K / (64 * groups), 0.43, 2.43
+    else:
+        loads = 2 * m * 26 + 8 * (26 if n == 4 else 13.6)
+        start, table, mix, store = 1500, 0, 0.37, 1.9
     matrix = ceil_div(share * groups, 4) * steps * step
     memory = share * groups * steps * loads
-    chain = (ceil_div(share, beside) * (steps * max(94.0 / pd + 0.19 * step, step) + 1500)
-             + (510.0 * view.K / (64 * groups) if view.conv else 0))
-    stream = (view.M * view.K + view.K * view.N) * 4 / 1930.0       # operands once at the rate of a large copy
+    chain = ceil_div(share, beside) * (steps * max(94.0 / pd + 0.19 * step, step) + start) + table
+    # operands once at the rate of a large copy
+    stream = 0 if view.conv else (view.M * view.K + view.K * view.N) * 4 / 1930.0
     longest = max(matrix, memory, chain)
-    return max(longest + 0.37 * (matrix + memory + chain - longest), stream) + share * m * n * 1024 * 1.9 / 64 + 4360
+    return max(longest + mix * (matrix + memory + chain - longest), stream) + share * m * n * 1024 * store / 64 + 4360
 
 
 def _pick_f32(view, kernels, predict, padded, direct):
@@ -965,9 +971,9 @@ def _pick_f32(view, kernels, predict, padded, direct):
     rows are to be padded, among the kernels whose tiles pass through registers, with K undivided (the groups' tiles
     lie beside each other in LDS).
 
-    Against it stand the tiles without LDS, which have to be predicted a tenth faster. The two predictions are off by
-    17 % (one standard deviation) each, fitted to 1 800 timings of the tiles without LDS and to the times of the other picks
-    over 132 operators (GEMMs and convolutions over the ranges above).
+    Against it stand the tiles without LDS, which for GEMMs have to be predicted a tenth faster: the two predictions are
+    off by 17 % (one standard deviation) each, fitted to 1 800 timings of the tiles without LDS and to the times of the
+    other picks over 132 operators. Convolutions: both fitted to the same layers, off by 7 and 11 %.
     Not for 1x1 windows, whose gathers the LDS kernels do without index arithmetic (7 x 259x90x90 -> 25 16.4 us, 18.4
     without LDS), and not for B stored [N][K] nor for batches: with few k steps the operands' latency is all there is, and tiles that share it
     through LDS have it once (96 x 197x64x197 10.0 us, 14.5 without LDS; 57x1249x714 with B^T 5.3 and 7.0)."""
@@ -999,7 +1005,7 @@ def _pick_f32(view, kernels, predict, padded, direct):
     if direct and view.groups == 1 and view.mode != 2 and not view.trans_a and view.K >= 32 \
             and (not view.conv or 1 < window <= 31 and view.K * 8 + 256 < LDS_BYTES):
         # the other prediction in clocks of a call (launch included), fitted to what its picks took
-        limit = (0.837 * best[0] + 4190 if view.conv else 1.02 * best[0] + 3750) / 1.1
+        limit = (best[0] + 4360) / 1.03 if view.conv else (1.02 * best[0] + 3750) / 1.1
         if not view.conv and view.M <= 64:
             # few rows of a large weight: where the weight's rows are no whole vectors the LDS kernels take 1.2 to 2 times
             # what was predicted (57x1610x1067 14.9 us for 7.5), where they are it is right (32x4096x4096)
@@ -1027,58 +1033,72 @@ def _pick_f32(view, kernels, predict, padded, direct):
     return cfg
 
 
-# kernels of the convolution's default, as F32_KERNELS; the K tiles of 72 and 144 hold whole windows of 3x3 (and of
-# whatever else divides them) and are for those
+# kernels of the convolution's default, as F32_KERNELS: for windows of one pixel, and for larger ones (the K tiles of 72 and
+# 144 hold whole windows of 3x3 and of whatever else divides them)
 CONV_KERNELS = (((1, 1), (1, 1), 16, 16, 2), ((1, 1), (1, 1), 16, 32, 3), ((2, 1), (2, 1), 16, 32, 3),
                 ((4, 1), (2, 1), 16, 32, 3), ((2, 2), (4, 1), 16, 16, 2), ((2, 1), (4, 1), 16, 16, 2),
                 ((4, 2), (4, 1), 16, 32, 5), ((2, 1), (2, 1), 32, 16, 3))
-CONV_WINDOW_KERNELS = (((1, 1), (1, 1), 16, 144, 8), ((2, 1), (2, 1), 16, 144, 8), ((2, 1), (4, 1), 16, 144, 8),
-                       ((2, 1), (2, 1), 32, 72, 8), ((4, 1), (2, 1), 32, 72, 8))
+WINDOW_KERNELS = (((1, 1), (1, 1), 16, 16, 2), ((2, 1), (4, 1), 16, 16, 2),            # any K
+                  ((1, 1), (1, 1), 16, 32, 3), ((4, 1), (2, 1), 16, 32, 3), ((2, 1), (4, 1), 16, 32, 5),
+                  ((4, 2), (4, 1), 16, 32, 3), ((4, 1), (4, 1), 16, 32, 8), ((4, 1), (4, 1), 16, 64, 8),
+                  ((2, 1), (2, 1), 16, 144, 8), ((2, 1), (2, 1), 32, 72, 8), ((4, 1), (2, 1), 32, 72, 8))
+
+
+def _conv_clocks(view, tiles, m, n, mf, bk, depth, groups):
+    """Predicted clocks (2.38 GHz) of a convolution on the busiest compute unit; see _default_conv."""
+    (wm, rm), (wn, rn) = m, n
+    bm, bn = wm * rm * mf, wn * rn * mf
+    steps = ceil_div(view.K, bk * groups)
+    nw = wm * wn * groups
+    lds = groups * 2 * 4 * (bm + bn) * bk
+    if lds > LDS_BYTES:
+        return None
+    share = ceil_div(tiles, NUM_CUS)
+    turns = ceil_div(share, max(1, min(LDS_BYTES // lds, 32 // nw)))
+    step = rm * rn * mf * mf * 2 * bk / 64.0                            # matrix clocks of one wavefront's k step
+    gathered = groups * bn * bk / 64.0                                  # loads of a step's gather, all wavefronts
+    window = view.conv["CR"] * view.conv["CS"]
+    stride = 1
+    if window == 1:
+        latency = {2: 129, 3: 125, 5: 457, 8: 1499}[depth] * (1 + 0.12 * bk / 32) + 33 * nw
+        overlap = {2: 0.8, 3: 0.4, 5: 0.3, 8: 0.35}[depth]
+        gather, gather_chain, start, mix, store = 3.7, 0, 3230, 0.47, 3.0
+        rate = 16 if tiles % 8 == 0 else 9                              # as in _f32_clocks
+    else:
+        latency = {2: 135, 3: 57, 5: 294, 8: 295 if bk > 64 else 63}[depth] * (1 + 0.12 * bk / 32) + 8.4 * nw
+        overlap = {2: 0.56, 3: 0.23, 5: 0.1, 8: 0.17}[depth]
+        # channel and tap: hoisted out of the loop (what is left are the loads), scalars, or lane by lane
+        hoisted = bk % window == 0
+        gather = 41 if hoisted else 50 if bn % 64 else 29
+        gather_chain = 0 if hoisted else 93
+        if window > 31:                                                 # position and predicate for every element
+            gather, gather_chain = gather * 2.5, gather_chain * 2
+        start, mix, store, rate = 1914, 0.88, 1.49, 274
+        stride = 6.1 if view.conv["CSTRW"] > 1 else 1                   # half of a line's pixels are used
+    compute = ceil_div(share * nw, 4) * step * steps + share * steps * gathered * gather / 4
+    chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap + gather_chain * gathered / nw) + start)
+    operands = tiles * (bm + bn * stride) * steps * bk * groups * 4.0 / NUM_CUS / rate
+    longest = max(compute, chain, operands)
+    return (longest + mix * (compute + chain + operands - longest) + share * bm * bn * 4 * store / 64
+            + 82 * rm * rn * mf * mf / 64 * (groups - 1))
 
 
 def _default_conv(view, padded=False, direct=True):
     """Tile, K tile, pipeline and K division of a convolution nobody tuned, by predicted time like _default_f32.
 
-    What differs from the plain product is the gathered operand. One float per lane and load, with its own address:
-    where the K tile holds whole windows (or the window is one pixel) the address advances by a constant, else
-    channel, tap and padding predicate are computed anew for every element of every tile, about 50 clocks per 64 of
-    them, and an untiled 3x3 layer spends more on that than on its products. Whole windows pay where tiles are many;
-    with few tiles K is divided over wavefront groups instead, which shortens the serial chain of k steps.
-    Checked against 3 200 timings over 180 layers (1 .. 16 images, 16 .. 512 channels, 7 .. 112 rows; 1x1 and
-    3x3, stride 1 and 2): the pick is 8 % off the best measured kernel in the geometric mean (1x1 5 %, 3x3 9 %; 1.57
-    times for the worst layer), the rule before it (square-ish power-of-two tiles until every unit has one, K tiles of up
-    to 32, K undivided) 1.86 times off. Above 4 microseconds the pick is 2 to 5 % slower than that rule's for six of the
-    layers; near the floor of a launch the two differ by up to 0.45 microseconds either way. Pointwise layers whose tiles are no multiple of 8 go at
+    What differs from the plain product is the gathered operand: one float per lane and load, with its own address.
+    Where the K tile holds whole windows (or the window is one pixel) the address advances by a constant; else an
+    element costs its channel and tap, which are scalars where a wavefront loads from one row of the tile. Windows of
+    several pixels: fitted to 3 000 timings over 69 layers (1 .. 16 images, 16 .. 512 channels, 7 .. 112 rows; 3x3,
+    stride 1 and 2) together with the tiles without LDS; the pick is 7.8 % off the best measured kernel in the geometric
+    mean and 1.34 times for the worst layer (11 % and 1.7 times with the constants and kernels before, fitted when
+    channel, tap and predicate were computed anew for every element).
+    One pixel: 5 % off (1 .. 16 images, 16 .. 512 channels). Pointwise layers whose tiles are no multiple of 8 go at
     the rate of grids that are not renumbered by XCD: 4 x 464x49x49 -> 48 stride 2 11.96 -> 7.93 us, 8 x 144x30x30 -> 192
     stride 2 6.84 -> 5.09, 15 x 131x21x21 -> 45 5.42 -> 4.29 (with one rate up to 15 % slower than the rule before).
     """
     window = view.conv["CR"] * view.conv["CS"]
-
-    def clocks(view, tiles, m, n, mf, bk, depth, groups):
-        (wm, rm), (wn, rn) = m, n
-        bm, bn = wm * rm * mf, wn * rn * mf
-        steps = ceil_div(view.K, bk * groups)
-        nw = wm * wn * groups
-        lds = groups * 2 * 4 * (bm + bn) * bk
-        if lds > LDS_BYTES:
-            return None
-        share = ceil_div(tiles, NUM_CUS)
-        turns = ceil_div(share, max(1, min(LDS_BYTES // lds, 32 // nw)))
-        step = rm * rn * mf * mf * 2 * bk / 64.0                        # matrix clocks of one wavefront's k step
-        gathered = groups * bn * bk / 64.0                              # loads of a step's gather, all wavefronts
-        hoisted = bk % window == 0
-        latency = {2: 129, 3: 125, 5: 457, 8: 1499}[depth] * (1 + 0.12 * bk / 32) + 33 * nw
-        overlap = {2: 0.8, 3: 0.4, 5: 0.3, 8: 0.35}[depth]
-        compute = ceil_div(share * nw, 4) * step * steps + share * steps * gathered * (3.7 if hoisted else 51.6) / 4
-        chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap + (0 if hoisted else 80 * gathered / nw)) + 3230)
-        rate = 16 if window > 1 or tiles % 8 == 0 else 9        # as in _f32_clocks; only one-pixel windows show it
-        operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
-        longest = max(compute, chain, operands)
-        return (longest + 0.47 * (compute + chain + operands - longest) + share * bm * bn * 4 * 3.0 / 64
-                + 82 * rm * rn * mf * mf / 64 * (groups - 1))
-
-    return _pick_f32(view, CONV_KERNELS + (CONV_WINDOW_KERNELS if window > 1 and 72 % window == 0 else ()),
-                     clocks, padded, direct)
+    return _pick_f32(view, WINDOW_KERNELS if window > 1 else CONV_KERNELS, _conv_clocks, padded, direct)
 
 
 def default_config(op, padded=False, direct=True):

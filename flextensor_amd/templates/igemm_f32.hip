@@ -430,6 +430,32 @@ static __device__ __forceinline__ f32x4 ld_f32x4(__amdgpu_buffer_rsrc_t r, unsig
 #else
 #define BROW_LINEAR 0
 #endif
+/* Tiles that cut windows (BK no multiple of CR * CS): which taps of a pixel are padding does not change from tile to
+ * tile, so they are bits of a word, made once, and an element costs its k's channel and tap, an add, a shift and an
+ * and-or. Where a wavefront's 64 elements are one row of the tile, channel and tap are scalars. Windows of more
+ * taps than a word has bits compute position and predicate for every element. */
+#if !KHOIST && CR * CS <= 31
+#define TAP_BITS 1
+#define PADDED (CPADH > 0 || CPADW > 0)
+#define ROW_SCALAR (BN % 64 == 0)
+/* all elements of a thread are of one pixel (those behind the tile are loaded with it and not stored) */
+#if NT % BN == 0 && (!defined(BSWZ1) || BROW_LINEAR)
+#define PXE(e) 0
+#else
+#define PXE(e) (e)
+#endif
+/* k / (CR * CS) and tap / CS by 24-bit products: x * m >> s with m = ceil(2^s / d) is x / d as long as x * d < 2^s and
+ * the product fits 32 bits. A tile's idle elements reach 64 rows behind it. */
+#define WINDOW_MAGIC (((1 << 18) + CR * CS - 1) / (CR * CS))
+#if (KP + 64) * CR * CS < (1 << 18) && (KP + 64) * WINDOW_MAGIC < (1ll << 32)
+#define DIV_WINDOW(k) (__umul24((k), WINDOW_MAGIC) >> 18)
+#else
+#define DIV_WINDOW(k) ((k) / (unsigned)(CR * CS))
+#endif
+#define DIV_ROW(t) (__umul24((t), (1024u + CS - 1) / CS) >> 10)       /* t * CS <= 30 * 31 */
+#else
+#define TAP_BITS 0
+#endif
 #else
 /* a batch of independent GEMMs (flextensor/nn/ops.py:1111-1158) reuses the
  * group index: operand b of every matrix starts b*M*K, b*K*N, b*M*N floats in */
@@ -690,8 +716,12 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
     const int kbase = kz * KSPLIT_LEN + kg * KGROUP_LEN + kt_lo * BK;
 
 #if MODE == 1
+#if TAP_BITS
+    unsigned px_base[EB], px_bad[EB];        /* tap (0, 0) of each pixel this thread gathers; bit 31 - t: tap t is padding */
+#else
     int px_off[EB], px_h[EB], px_w[EB];      /* pixel decomposition of each column this thread gathers */
     bool px_ok[EB];
+#endif
 #endif
 
     /* ---- global loads: raw buffer loads with hardware bounds checking --- */
@@ -705,6 +735,39 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
     const __amdgpu_buffer_rsrc_t rsrc_b =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, B_BYTES, 0x00020000);
     unsigned a_voff[EA], b_voff[EB];
+#if MODE == 1 && !KHOIST
+    /* byte offset of element e of the tile at k0, a select of two values or bits, no branch (see a_voff) */
+#if TAP_BITS && ROW_SCALAR
+    const int gather_wave = __builtin_amdgcn_readfirstlane(wave);
+#endif
+    auto gather_offset = [&](int k0, int e) -> unsigned {
+#if TAP_BITS
+#if ROW_SCALAR
+        const unsigned k = (unsigned)(k0 + (e * NT + gather_wave * 64) / BN);
+        const unsigned c = k / (unsigned)(CR * CS), t = k % (unsigned)(CR * CS), r = t / CS;
+#else
+        const unsigned k = (unsigned)(k0 + b_row[e]);
+        const unsigned c = DIV_WINDOW(k), t = k - c * (CR * CS), r = DIV_ROW(t);
+#endif
+        const unsigned off = px_base[PXE(e)] + (c * (CH * CW) + r * (CDILH * CW) + (t - r * CS) * CDILW) * 4u;
+#if PADDED || KP != K || N % BN != 0 || B_CHUNKS % NT != 0
+        return off | ((px_bad[PXE(e)] << (KP == K || k < K ? t : 31u)) & OOB);
+#else
+        return off;
+#endif
+#else
+        const int k = k0 + b_row[e];
+        const int c = k / (CR * CS);
+        const int rs = k % (CR * CS);
+        const int ih = px_h[e] + (rs / CS) * CDILH;
+        const int iw = px_w[e] + (rs % CS) * CDILW;
+        bool ok = px_ok[e] & ((unsigned)ih < (unsigned)CH) & ((unsigned)iw < (unsigned)CW);
+        if (KP != K) ok = ok & (k < K);
+        const unsigned off = (unsigned)(px_off[e] + c * (CH * CW) + ih * CW + iw) * 4u;
+        return ok ? off : OOB;
+#endif
+    };
+#endif
 #if DTL
     /* The loads are written as instructions, not through the builtin: the
      * compiler makes every later LDS read wait for a direct-to-LDS load it
@@ -795,16 +858,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
             if (KP != K) vo = (k0 + b_row[e] < K) ? vo : OOB;
             dma4(desc_b, dst, vo, (K_AT(k0) / (CR * CS)) * (CH * CW * 4));
 #else
-            const int k = k0 + b_row[e];
-            const int c = k / (CR * CS);
-            const int rs = k % (CR * CS);
-            const int ih = px_h[e] + (rs / CS) * CDILH;
-            const int iw = px_w[e] + (rs % CS) * CDILW;
-            bool ok = px_ok[e] & ((unsigned)ih < (unsigned)CH) & ((unsigned)iw < (unsigned)CW);
-            if (KP != K) ok = ok & (k < K);
-            const unsigned off = (unsigned)(px_off[e] + c * (CH * CW) + ih * CW + iw) * 4u;
-            const unsigned vo = ok ? off : OOB;      /* a select of two values, no branch (see a_voff) */
-            dma4(desc_b, dst, vo, 0);
+            dma4(desc_b, dst, gather_offset(k0, e), 0);
 #endif
 #endif
         }
@@ -878,13 +932,26 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #pragma unroll
     for (int e = 0; e < EB; ++e) {
         const int n = n0 + b_col[e];
-        px_ok[e] = (n < N) & (tid + e * NT < B_CHUNKS);
-        const int nn = px_ok[e] ? n : 0;
+        const bool inside = (n < N) & (tid + e * NT < B_CHUNKS);
+        const int nn = inside ? n : 0;
         const int b = nn / OHW;
         const int p = nn % OHW;
+#if TAP_BITS
+        if (PXE(e) != e) continue;
+        const int h0 = (p / CQ) * CSTRH - CPADH, w0 = (p % CQ) * CSTRW - CPADW;
+        px_base[e] = (unsigned)((b * CC + gi * (CC / CG)) * (CH * CW) + h0 * CW + w0) * 4u;
+        unsigned bad = 1;               /* the tap of a k behind K */
+#pragma unroll
+        for (int t = 0; t < CR * CS; ++t)
+            bad |= (((unsigned)(h0 + t / CS * CDILH) < (unsigned)CH) & ((unsigned)(w0 + t % CS * CDILW) < (unsigned)CW)
+                    ? 0u : OOB) >> t;
+        px_bad[e] = inside ? bad : ~0u;
+#else
+        px_ok[e] = inside;
         px_h[e] = (p / CQ) * CSTRH - CPADH;
         px_w[e] = (p % CQ) * CSTRW - CPADW;
         px_off[e] = b * (CC * CH * CW) + gi * ((CC / CG) * CH * CW);
+#endif
     }
 #endif
 #pragma unroll
@@ -961,16 +1028,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
             if (KP != K) vo = (k0 + b_row[e] < K) ? vo : OOB;
             breg[set][e] = LOAD_B(rsrc_b, vo, (K_AT(k0) / (CR * CS)) * (CH * CW * 4));
 #else
-            const int k = k0 + b_row[e];
-            const int c = k / (CR * CS);
-            const int rs = k % (CR * CS);
-            const int ih = px_h[e] + (rs / CS) * CDILH;
-            const int iw = px_w[e] + (rs % CS) * CDILW;
-            bool ok = px_ok[e] & ((unsigned)ih < (unsigned)CH) & ((unsigned)iw < (unsigned)CW);
-            if (KP != K) ok = ok & (k < K);
-            const unsigned off = (unsigned)(px_off[e] + c * (CH * CW) + ih * CW + iw) * 4u;
-            const unsigned vo = ok ? off : OOB;      /* a select of two values, no branch (see a_voff) */
-            breg[set][e] = LOAD_B(rsrc_b, vo, 0);
+            breg[set][e] = LOAD_B(rsrc_b, gather_offset(k0, e), 0);
 #endif
         }
     };
