@@ -20,6 +20,11 @@
 //                             Grouped convolution (CG groups) runs one GEMM
 //                             per group: M = Kout/CG, K = (C/CG)*R*S, and the
 //                             group index is one more grid factor.
+//                             IMAGES n: a 1x1 / stride 1 / unpadded layer over n
+//                             images of N pixels each as n products
+//                             W [M][K] x X_i [K][N], which is MODE 0 with one A
+//                             for all: the image loads in 16-byte vectors, where
+//                             the gather takes one float per lane and load.
 //                             COLOUT 1 stores C as [CG][M][N], the layout of the
 //                             GEMM stage of a convolution written as im2col,
 //                             GEMM, col2img (ops.py:982-1044), instead of NCHW.
@@ -78,7 +83,15 @@
 
 /* Constants arrive as -DFT_<NAME>=value: single-letter macros on the command line
  * would be visible to (and break) the runtime-compilation built-in headers. */
+#ifdef FT_IMAGES
+#define MODE 0
+#define IMAGES FT_IMAGES
+#define AGROUP(g) 0               /* one weight and bias for every image */
+#else
 #define MODE FT_MODE
+#define IMAGES 0
+#define AGROUP(g) (g)
+#endif
 #define M FT_M
 #define N FT_N
 #define K FT_K
@@ -459,12 +472,14 @@ static __device__ __forceinline__ f32x4 ld_f32x4(__amdgpu_buffer_rsrc_t r, unsig
 #else
 /* a batch of independent GEMMs (flextensor/nn/ops.py:1111-1158) reuses the
  * group index: operand b of every matrix starts b*M*K, b*K*N, b*M*N floats in */
-#ifdef FT_CG
+#if IMAGES
+#define CG IMAGES
+#elif defined(FT_CG)
 #define CG FT_CG
 #else
 #define CG 1
 #endif
-#define A_BYTES (CG * M * K * 4)
+#define A_BYTES ((IMAGES ? 1 : CG) * M * K * 4)
 #define B_BYTES (CG * K * N * 4)
 #endif
 
@@ -607,7 +622,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #endif
                         float val = acc[i][j][v];
 #if HAS_BIAS
-                        if (first_k_part) val += bias[gi_ * M + m];
+                        if (first_k_part) val += bias[AGROUP(gi_) * M + m];
 #endif
 #if SPLITK > 1
                         unsafeAtomicAdd(dst, val);
@@ -918,7 +933,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
         const int m = m0 + a_row[e];
         bool ok = (A_CHUNKS % NT == 0) || (tid + e * NT < A_CHUNKS);
         if (M % BM != 0) ok = ok & (m < M);
-        const unsigned off = (unsigned)((gi * M + m) * K + a_col[e]) * 4u;
+        const unsigned off = (unsigned)((AGROUP(gi) * M + m) * K + a_col[e]) * 4u;
         a_voff[e] = ok ? off : OOB;
 #endif
     }
