@@ -17,7 +17,8 @@ with a "rocm" target):
   fuse      [[GROUP_M]] tile-traversal group height (depthwise: [[wavefronts
             per workgroup]])
   reorder   [[0|1]]   1 = remap workgroup ids so that neighbouring tiles run
-            on the same XCD (shared L2)
+            on the same XCD (shared L2); a fourth number selects a variant the
+            defaults choose (1 = tiles without LDS, 2 = 1x1 layers image by image)
   special   enumerated knobs attached to a task (LDS padding, load width,
             non-temporal stores, ...)
 """
