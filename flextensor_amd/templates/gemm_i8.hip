@@ -251,7 +251,8 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
     const int nblk = TILES_M * TILES_N * SPLITK;
     int bid = blockIdx.x;
 #if XCD_REMAP
-    if (nblk % 8 == 0) bid = (bid % 8) * (nblk / 8) + bid / 8;
+    /* as in igemm_f32.hip: 2752x1120x80, 172 tiles, 4.43 -> 3.77 us for renumbering counts that 8 does not divide too */
+    bid = (bid % 8) * (nblk / 8) + (bid % 8 < nblk % 8 ? bid % 8 : nblk % 8) + bid / 8;
 #endif
 #if SPLITK > 1
     const int kz = bid / (TILES_M * TILES_N);       /* which part of K */

@@ -930,8 +930,8 @@ def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups):
     overlap = {1: 0.2, 2: 0.8, 3: 0.4, 5: 0.3, 8: 0.35}[depth]      # share of a step's own MFMAs the chain waits for
     turns = ceil_div(share, beside)
     chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap) + 930)
-    # workgroups are renumbered by XCD where their count is a multiple of 8; where it is not, a batch's panels are
-    # fetched by all eight L2s
+    # the lower rate was fitted when only counts that 8 divides were renumbered by XCD; it still steers to those, which
+    # end in whole rounds (one rate for all: 24 drawn batches 1 % faster in the mean, single pointwise layers up to 16 % slower)
     rate = 31 if view.groups == 1 or tiles % 8 == 0 else 14
     operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
     longest = max(matrix, chain, operands)
@@ -951,8 +951,8 @@ def _default_f32(view, padded=False, direct=True):
     sizes (M, N, K 8 .. 4096, batches of 26 .. 128; half of them no multiples of 4); the pick is within 5 % of the
     best measured in the geometric mean and 1.6 times as fast as the rule before it (square-ish power-of-two
     tiles until every unit has one, K tiles of 32): 1100x1301x900 47.1 -> 30.0 us, 863x1862x1280 (B^T) 69.7 ->
-    44.4, 96 x 74x96x133 6.8 -> 5.4, 32x4096x3072 43.6 -> 16.5. Batches whose tiles are no multiple of 8 go at the rate
-    of grids that are not renumbered (14 bytes per clock and unit; 86 batches measured: 3.8 % off the best kernel, with
+    44.4, 96 x 74x96x133 6.8 -> 5.4, 32x4096x3072 43.6 -> 16.5. Batches whose tiles are no multiple of 8 go at a lower
+    rate (14 bytes per clock and unit, fitted when such grids were not renumbered; 86 batches measured: 3.8 % off the best kernel, with
     one rate for all 11.5 % off and up to 1.5 times as slow as the rule before): 121 x 35x80x124 6.33 -> 4.16 us,
     114 x 68x110x63 (B^T) 6.38 -> 4.88, 63 x 52x80x274 7.01 -> 5.21. K streaming is left to the search: a plan that owns a
     workspace cannot run on two streams at once, and a default plan can.
@@ -1116,7 +1116,7 @@ def _default_conv(view, padded=False, direct=True, by_image=False):
     mean and 1.34 times for the worst layer (11 % and 1.7 times with the constants and kernels before, fitted when
     channel, tap and predicate were computed anew for every element).
     One pixel: 5 % off (1 .. 16 images, 16 .. 512 channels). Pointwise layers whose tiles are no multiple of 8 go at
-    the rate of grids that are not renumbered by XCD: 4 x 464x49x49 -> 48 stride 2 11.96 -> 7.93 us, 8 x 144x30x30 -> 192
+    the lower rate of grids that were not renumbered by XCD: 4 x 464x49x49 -> 48 stride 2 11.96 -> 7.93 us, 8 x 144x30x30 -> 192
     stride 2 6.84 -> 5.09, 15 x 131x21x21 -> 45 5.42 -> 4.29 (with one rate up to 15 % slower than the rule before).
 
     A pointwise layer whose images are matrices as they lie in memory goes image by image: 16-byte loads instead of one
