@@ -1136,9 +1136,10 @@ def _default_conv(view, padded=False, direct=True, by_image=False):
     return cfg
 
 
-def default_config(op, padded=False, direct=True):
-    """A reasonable untuned config: the point a search begins with, and for all operators but the convolution
-    what an untuned task runs on (untuned_config)."""
+def default_config(op, padded=False, direct=False):
+    """A reasonable untuned config: the point a search begins with, and with ``direct`` (tiles without LDS stand for
+    choice too, which are not in the space) for all operators but the convolution what an untuned task runs on
+    (untuned_config)."""
     cfg = _empty_config()
     if op.kind == "gemm_int8":
         return _default_i8(GemmView(op), padded)

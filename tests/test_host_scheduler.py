@@ -762,3 +762,17 @@ def test_untuned_pointwise_layers_get_larger_tiles_where_the_grid_is_not_renumbe
     op, = [o for o in flatten_graph(conv2d(*args)[0])[0] if o.kind == "conv2d_nchw"]
     (tm, wm, rm, mf), (tn, wn, rn, _) = gfx950.untuned_config(op)["spatial"]
     assert wm * rm * mf * wn * rn * mf >= (64 * 32 if args[1] != 464 else 32 * 32)
+
+
+@pytest.mark.parametrize("m,k,n", [(23, 2029, 1834), (40, 2048, 1333), (48, 1280, 2001)])
+def test_search_begins_at_a_point_of_its_space(m, k, n):
+    """Where an untuned product runs on tiles without LDS, which the space does not hold, the first seed is the best
+    predicted kernel of the space."""
+    from flextensor_amd import nn
+    from flextensor_amd.te import placeholder
+    op = nn.gemm(placeholder((m, k)), placeholder((k, n))).op
+    assert gfx950.untuned_config(op)["reorder"][0][3:] == [1]
+    seed, space = gfx950.seed_configs(op)[0], gfx950.generate_space(op)
+    for kind in ("spatial", "reduce", "unroll", "fuse", "reorder"):
+        for name, entity in zip(space.types[kind], seed[kind]):
+            assert list(entity) in [list(e) for e in space.subspaces[name].static_entities], (kind, entity)
