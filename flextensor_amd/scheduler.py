@@ -318,6 +318,21 @@ class Scheduler(object):
                 warm_up_enough = True
         self.timeout = old_timeout
 
+    def _indices(self, cfg, type_keys):
+        """A config's place in the space, or None."""
+        indices = {}
+        for type_key in type_keys:
+            names = self.space.types[type_key]
+            ents = cfg.get(type_key, []) if cfg else []
+            if len(names) != len(ents):
+                return None
+            for name, ent in zip(names, ents):
+                try:
+                    indices[name] = self.space.subspaces[name].static_entities.index(list(ent))
+                except ValueError:
+                    return None
+        return indices
+
     def _seed(self, configs, type_keys):
         """Measure known-good points first so that the walk starts from them:
         the template's default config and, when the task has one, the entry of
@@ -339,23 +354,8 @@ class Scheduler(object):
             candidates.append(shipped.op_config_lst[self.op_pos])
         points = []
         for cfg in candidates:
-            indices = {}
-            ok = True
-            for type_key in type_keys:
-                names = self.space.types[type_key]
-                ents = cfg.get(type_key, []) if cfg else []
-                if len(names) != len(ents):
-                    ok = False
-                    break
-                for name, ent in zip(names, ents):
-                    try:
-                        indices[name] = self.space.subspaces[name].static_entities.index(list(ent))
-                    except ValueError:
-                        ok = False
-                        break
-                if not ok:
-                    break
-            if not ok or not indices or self.walker_group.ever_met(indices) \
+            indices = self._indices(cfg, type_keys)
+            if not indices or self.walker_group.ever_met(indices) \
                     or any(str(indices) == str(p) for p in points):
                 continue
             if not self._lowers(configs, self.walker_group.to_config(indices)):
@@ -609,13 +609,32 @@ class OpScheduler(Scheduler):
         if perf_path is not None:
             self.walker_group.model_dir = perf_path
         if method == "searching":
-            return self._searching_schedule(configs, wanted_types, use_model=use_model)
+            found = self._searching_schedule(configs, wanted_types, use_model=use_model)
         elif method == "random":
-            return self._random_schedule(configs, wanted_types, use_model=use_model)
+            found = self._random_schedule(configs, wanted_types, use_model=use_model)
         elif method == "q":
-            return self._q_schedule(configs, wanted_types, use_model=use_model)
+            found = self._q_schedule(configs, wanted_types, use_model=use_model)
         else:
             raise RuntimeError("Currently no support for method %s" % method)
+        return self._or_untuned(configs, found, wanted_types)
+
+    def _or_untuned(self, configs, found, type_keys):
+        """The faster of what the search found and what the operator runs on untuned, where that is no point of
+        the space: a rule may choose kernels that the space does not hold (tiles without LDS, images one at a time,
+        K divided with zeros behind it), and a tuned operator is not to be slower than an untuned one."""
+        ops, _ = self.task.func(*self.task.args)
+        op = flatten_graph(ops)[0][self.op_pos]
+        graph = configs.graph_config or {}
+        special = dict(zip(self.task.special_space, graph["special"])) if graph.get("special") else None
+        try:
+            untuned = gfx950.untuned_config(op, special)
+        except (gfx950.InvalidConfig, NotImplementedError):
+            return found
+        if self._indices(untuned, type_keys) is not None or not self._lowers(configs, untuned):
+            return found
+        cost, cost_untuned = self.parallel_evaluate(configs, [found, untuned], number=self.number)
+        self._log("found %.6f, untuned %.6f" % (cost, cost_untuned))
+        return untuned if cost_untuned < cost else found
 
     def parallel_evaluate(self, configs, next_op_configs, number=1, rpc_info=None):
         return self._parallel_evaluate(configs, next_op_configs, mode="op", number=number)

@@ -776,3 +776,23 @@ def test_search_begins_at_a_point_of_its_space(m, k, n):
     for kind in ("spatial", "reduce", "unroll", "fuse", "reorder"):
         for name, entity in zip(space.types[kind], seed[kind]):
             assert list(entity) in [list(e) for e in space.subspaces[name].static_entities], (kind, entity)
+
+
+@pytest.mark.parametrize("method", ["searching", "random"])
+@pytest.mark.parametrize("func,args,variant", [(gemm, (40, 2048, 1333), 1), (conv2d, (2, 240, 35, 35, 160, 1, 1, 0, 1, 1), 2)])
+def test_a_tuned_operator_is_not_slower_than_an_untuned_one(func, args, variant, method):
+    """The untuned config, where it is no point of the space, is measured beside what the search found, and the faster
+    of the two is returned."""
+    task = Task("gemm" if func is gemm else "conv2d", "beside_untuned", func, args, "rocm", 0)
+    register_task(task, override=True)
+
+    def untuned(cfg):
+        return any((c.get("reorder") or [[]])[0][3:] == [variant] for c in cfg.op_config_lst)
+
+    for faster in (True, False):
+        def cost(k, c, p, n):
+            schedule_with_config(k, c, op_pos=p)            # points the templates refuse cost inf
+            return (1.0 if faster else 3.0) if untuned(c) else 2.0
+        _, _, configs = schedule(task.key, op_trial=3, graph_trial=1, parallel=2, method=method, evaluator=cost,
+                                 warm_up=(1, 4), verbose=False)
+        assert untuned(configs) == faster
