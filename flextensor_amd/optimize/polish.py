@@ -73,8 +73,8 @@ def neighbours(key, cfg):
         out += [("load spread %d" % x, with_op("unroll", [[8, x]])) for x in (1, 2, 4, 6, 7, 8) if x != spread]
     group = (op.get("fuse") or [[4]])[0][0]
     out += [("group %d" % x, with_op("fuse", [[x]])) for x in (1, 2, 4, 8, 16) if x != group]
-    order = (list((op.get("reorder") or [[1, 0, 0]])[0]) + [0, 0])[:3]
-    out.append(("xcd %d" % (1 - order[0]), with_op("reorder", [[1 - order[0], order[1], order[2]]])))
+    order = list((op.get("reorder") or [[1, 0, 0]])[0])         # what stands behind the first number stays
+    out.append(("xcd %d" % (1 - order[0]), with_op("reorder", [[1 - order[0]] + order[1:]])))
     return out
 
 

@@ -144,3 +144,23 @@ def test_layer_tuned_at_another_batch_size_seeds_the_search():
     assert lookup("conv2d_t_(4, 250, 56, 56, 512, 3, 1, 1, 1, 1)_rocm(0)", similar=True) is None
     assert lookup("conv2d_depthwise_(4, 512, 28, 28, 1, 3, 1, 1, 1)_rocm(0)", similar=True) is None
     assert lookup("not a key", similar=True) is None
+
+
+def test_polish_turns_the_renumbering_and_keeps_the_kernel():
+    """The "xcd" neighbour differs in the first number of the reorder entry only, whatever stands behind it."""
+    from flextensor_amd.optimize import polish
+    from flextensor_amd.task import Task, conv2d, gemm, register_task
+    from flextensor_amd.templates import gfx950
+    for func, args, variant in ((gemm, (1024, 1024, 1024), []), (gemm, (40, 2048, 1333), [1]),
+                                (conv2d, (2, 240, 35, 35, 160, 1, 1, 0, 1, 1), [2])):
+        task = Task("gemm" if func is gemm else "conv2d", "polished", func, args, "rocm", 0)
+        register_task(task, override=True)
+        ops, _ = func(*args)
+        ops = [ops[0].input_tensors[0].op, ops[0]] if func is conv2d else ops
+        cfg = Config([gfx950.untuned_config(op) if op.kind in gfx950.GEMM_KINDS else gfx950._empty_config() for op in ops], {})
+        entry = cfg.op_config_lst[-1]["reorder"][0]
+        assert entry[3:] == variant
+        (turned,) = [c for what, c in polish.neighbours(task.key, cfg) if what == "xcd 0"]
+        assert turned.op_config_lst[-1]["reorder"] == [[0] + entry[1:]]
+        before, after = (schedule_with_config(task.key, c)[0].specs[-1] for c in (cfg, turned))
+        assert before.template == after.template and before.defines.get("IMAGES") == after.defines.get("IMAGES")
