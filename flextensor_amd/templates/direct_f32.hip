@@ -27,6 +27,7 @@
 #define REP_N FT_REP_N
 #define WAVES_K FT_WAVES_K      /* wavefront groups that divide K, summed through LDS */
 #define GROUP_M FT_GROUP_M
+#define XCD_REMAP FT_XCD_REMAP
 #define PD FT_PD                /* k steps in registers or on their way to them */
 #ifdef FT_HAS_BIAS
 #define HAS_BIAS FT_HAS_BIAS
@@ -146,13 +147,13 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
     const int kg = wave / NW, wm = wave % NW / WAVES_N, wn = wave % WAVES_N;
     const int li = lane & 15, lg = lane >> 4;
 
-    /* ---- workgroup -> (group, tile): consecutive logical tiles stay on one XCD, whatever their number (the
-     * first nblk % 8 XCDs have one more) ------------------------------------------------------------------- */
+    /* ---- workgroup -> (group, tile): with XCD_REMAP consecutive logical tiles stay on one XCD, whatever their number
+     * (the first nblk % 8 XCDs have one more) --------------------------------------------------------------- */
     int bid = blockIdx.x;
-    {
-        const int nblk = TILES_M * TILES_N * CG, x = bid % 8;
-        bid = x * (nblk / 8) + (x < nblk % 8 ? x : nblk % 8) + bid / 8;
-    }
+#if XCD_REMAP
+    const int nblk = TILES_M * TILES_N * CG;
+    bid = (bid % 8) * (nblk / 8) + (bid % 8 < nblk % 8 ? bid % 8 : nblk % 8) + bid / 8;
+#endif
     const int gi = bid / (TILES_M * TILES_N);
     int m0, n0;                         /* of the wavefront's tile */
     {

@@ -632,7 +632,7 @@ def _lower_direct(op, view, D, direct, depth, out_name, in_names, materialized_p
     # one after the other in the same LDS: the offsets of the gathered operand's k, the groups' partial sums
     if max(waves * rm * rn * 1024 if waves_k > 1 else 0, steps * 32 * 8 if view.mode == 1 else 0) + 16 > LDS_BYTES:
         raise InvalidConfig("partial sums or the offsets of a gathered operand need more than %d bytes" % LDS_BYTES)
-    D = {k: D[k] for k in ("M", "N", "K", "WAVES_M", "WAVES_N", "REP_M", "REP_N", "GROUP_M")}
+    D = {k: D[k] for k in ("M", "N", "K", "WAVES_M", "WAVES_N", "REP_M", "REP_N", "GROUP_M", "XCD_REMAP")}
     D.update(MODE=view.mode, WAVES_K=waves_k, PD=pd)
     a_name, b_name = in_names[0], in_names[1]
     b_bytes = view.groups * view.K * view.N * 4

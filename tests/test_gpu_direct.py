@@ -8,7 +8,7 @@ TOL = 1e-5
 VARIANTS = (1,)
 
 
-def direct_plan(func, args, tile, groups, ahead, variant):
+def direct_plan(func, args, tile, groups, ahead, variant, xcd=1):
     """The plan of the operator's contraction on tiles of (wavefronts, MFMA tiles each) along M and along N, K divided
     among ``groups`` of wavefronts, ``ahead`` k steps on their way."""
     from flextensor_amd.scheduler import flatten_graph, schedule_with_config_ops
@@ -23,7 +23,7 @@ def direct_plan(func, args, tile, groups, ahead, variant):
             (wm, rm, wn, rn), view = tile, gfx950.GemmView(op)
             cfg["spatial"] = [[ceil_div(view.M, 16 * wm * rm), wm, rm, 16], [ceil_div(view.N, 16 * wn * rn), wn, rn, 16]]
             cfg["reduce"], cfg["unroll"] = [[groups, ceil_div(view.K, 32 * groups), 32]], [[ahead, 1]]
-            cfg["fuse"], cfg["reorder"] = [[4]], [[1, 1 if groups > 1 else 0, 0, variant]]
+            cfg["fuse"], cfg["reorder"] = [[4]], [[xcd, 1 if groups > 1 else 0, 0, variant]]
         configs.append(cfg)
     plan, bufs = schedule_with_config_ops(ops, bufs, Config(configs, None))
     assert [s.template for s in plan.specs] == ["direct_f32.hip"]
@@ -124,3 +124,13 @@ def test_defaults_take_the_tiles_without_lds(oracle, shape, func):
     with torch.cuda.stream(stream):
         out = run(plan, bufs, host)
     assert rel(out, ref) <= TOL
+
+
+@pytest.mark.parametrize("xcd", [0, 1])
+def test_order_of_the_workgroups(oracle, xcd):
+    """The first number of the reorder entry: workgroups in order, or renumbered by XCD. 15 tiles in three batches."""
+    from flextensor_amd.measure import seeded_inputs
+    plan, bufs = direct_plan(gemm_of(False), (3, 40, 64, 70), (1, 1, 1, 1), 1, 2, 1, xcd)
+    assert plan.specs[0].defines["XCD_REMAP"] == xcd and plan.specs[0].grid[0] == 45
+    a, b = seeded_inputs(bufs, seed=xcd)
+    assert rel(run(plan, bufs, [a, b]), np.matmul(a.astype(np.float64), b.astype(np.float64))) <= TOL
