@@ -913,8 +913,9 @@ F32_KERNELS = (((1, 1), (1, 1), 16, 16, 2), ((1, 1), (1, 1), 16, 32, 3), ((1, 1)
                ((2, 2), (4, 1), 16, 32, 5), ((4, 2), (4, 2), 16, 16, 1))
 
 
-def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups):
-    """Predicted clocks (2.38 GHz) of an fp32 contraction on the busiest compute unit; see _default_f32."""
+def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups, call=False):
+    """Predicted clocks (2.38 GHz) of an fp32 contraction on the busiest compute unit, see _default_f32; or of a whole
+    ``call``, to be held against tiles without LDS, see _pick_f32."""
     (wm, rm), (wn, rn) = m, n
     bm, bn = wm * rm * mf, wn * rn * mf
     steps = ceil_div(view.K, bk * groups)
@@ -935,8 +936,17 @@ def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups):
     rate = 31 if view.groups == 1 or tiles % 8 == 0 else 14
     operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
     longest = max(matrix, chain, operands)
-    return (longest + 0.35 * (matrix + chain + operands - longest) + share * bm * bn * 4 * 4.8 / 64
-            + (38 * rm * rn * mf * mf / 64 * (groups - 1)))
+    clocks = (longest + 0.35 * (matrix + chain + operands - longest) + share * bm * bn * 4 * 4.8 / 64
+              + (38 * rm * rn * mf * mf / 64 * (groups - 1)))
+    if not call:
+        return clocks
+    # what the picks' times showed beside the launch: rows of A that are no whole vectors, and several workgroups of
+    # wavefront groups side by side, which are in each other's way (210 and 294 tiles of 80 and 112x1500x667: 6.7 and 10.2 us)
+    if view.K % 4:
+        clocks += 0.34 * tiles * bm * steps * bk * groups * 4.0 / NUM_CUS / 31
+    if groups > 1 and min(share, beside) > 1:
+        clocks += 0.32 * chain
+    return 0.974 * clocks + 4110
 
 
 def _default_f32(view, padded=False, direct=True):
@@ -972,30 +982,39 @@ def _direct_clocks(view, m, n, pd, groups):
     beside = max(1, min(share, min(8, 512 // (4 * m * n + 8 * (m + n) * pd + 40)) * 4 // groups))
     step = m * n * 256                                              # matrix clocks of a wavefront's k step
     # clocks a unit spends on a step's loads: two vectors per row block; per column one float and k (with a stride along
-    # the rows two lines where there was one), or a vector
+    # the rows a load spreads over up to twice the lines), or a vector of n floats. Before the first step: the operands'
+    # latency, or the gathered operand's table of offsets, made once, and every pixel's padding bits; the table's entries
+    # are read anew in every step.
     if view.conv:
         loads = 2 * m * 40 + 8 * n * (18.4 if view.conv["CSTRW"] > 1 else 9.5)
-        start, table, mix, store = 3330, 210.0 * view.K / (64 * groups), 0.43, 2.43
+        table, start, mix, store, sums, launch, entries = 210.0 * view.K / (64 * groups), 3330, 0.43, 2.43, 0, 4360, 0
     else:
-        loads = 2 * m * 26 + 8 * (26 if n == 4 else 13.6)
-        start, table, mix, store = 1500, 0, 0.37, 1.9
-    matrix = ceil_div(share * groups, 4) * steps * step
+        loads = 2 * m * 50 + 8 * {1: 9.7, 2: 19, 4: 26}[n]
+        table, start, mix, store, sums, launch, entries = 0, 1380, 0.23, 7.6, 29, 3930, 0
+    # wavefronts of one matrix core; two workgroups of two wavefronts begin on the same two of the four
+    wavefronts = 2 if share == groups == 2 and not view.conv else ceil_div(share * groups, 4)
+    matrix = wavefronts * steps * step
     memory = share * groups * steps * loads
     chain = ceil_div(share, beside) * (steps * max(94.0 / pd + 0.19 * step, step) + start) + table
     # operands once at the rate of a large copy
     stream = 0 if view.conv else (view.M * view.K + view.K * view.N) * 4 / 1930.0
     longest = max(matrix, memory, chain)
-    return max(longest + mix * (matrix + memory + chain - longest), stream) + share * m * n * 1024 * store / 64 + 4360
+    return (max(longest + mix * (matrix + memory + chain - longest), stream) + share * m * n * 1024 * store / 64
+            + entries * share * groups * steps + sums * m * n * (groups - 1) + launch)
 
 
 def _pick_f32(view, kernels, predict, padded, direct):
-    """The config of the kernel and number of wavefront K groups with the smallest predicted time, and that time; where the LDS
-    rows are to be padded, among the kernels whose tiles pass through registers, with K undivided (the groups' tiles
-    lie beside each other in LDS).
+    """The config of the kernel and number of wavefront K groups with the smallest predicted time, and that time (the
+    LDS kernel's also where tiles without LDS are taken); where the LDS rows are to be padded, among the kernels whose tiles
+    pass through registers, with K undivided (the groups' tiles lie beside each other in LDS).
 
-    Against it stand the tiles without LDS, which for GEMMs have to be predicted a tenth faster: the two predictions are
-    off by 17 % (one standard deviation) each, fitted to 1 800 timings of the tiles without LDS and to the times of the
-    other picks over 132 operators. Convolutions: both fitted to the same layers, off by 7 and 11 %.
+    Against it stand the tiles without LDS, which have to be predicted 8 % faster (windows of several pixels: 3 %). The
+    two predictions of a call are off by 10 % each (one standard deviation; windows 7 and 11 %), fitted to the LDS picks and
+    to 1 180 timings of the tiles without LDS over 210 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16).
+    Of those GEMMs 58 go without LDS; all 210 take 0.978 times the LDS
+    kernels' time in the geometric mean, six are more than 3 % slower than those, at most 1.09 times. One rule whatever the
+    rows and their alignment: 64x1500x667 6.9 us with LDS and 7.3 without, 32x4096x4096 18.7 and 19.7, 74x3120x1200 22.7 and
+    14.3, 112x4096x4096 36.6 and 50.4; 64x1610x1067 keeps LDS, wrongly (11.2 and 10.0).
     Not for 1x1 windows, whose gathers the LDS kernels do without index arithmetic (7 x 259x90x90 -> 25 16.4 us, 18.4
     without LDS), and not for B stored [N][K] nor for batches: with few k steps the operands' latency is all there is, and tiles that share it
     through LDS have it once (96 x 197x64x197 10.0 us, 14.5 without LDS; 57x1249x714 with B^T 5.3 and 7.0)."""
@@ -1024,19 +1043,15 @@ def _pick_f32(view, kernels, predict, padded, direct):
             clocks = predict(view, tiles, m, n, mf, bk, depth, groups)
             if clocks is not None and (best is None or clocks < best[0]):
                 best = (clocks, [tm, m[0], m[1], mf], [tn, n[0], n[1], mf], [groups, steps, bk], depth)
+                kernel = (tiles, m, n, mf, bk, depth, groups)
     if direct and view.groups == 1 and view.mode != 2 and not view.trans_a and view.K >= 32 \
             and (not view.conv or 1 < window <= 31 and view.K * 8 + 256 < LDS_BYTES):
-        # the other prediction in clocks of a call (launch included), fitted to what its picks took
-        limit = (best[0] + 4360) / 1.03 if view.conv else (1.02 * best[0] + 3750) / 1.1
-        if not view.conv and view.M <= 64:
-            # few rows of a large weight: where the weight's rows are no whole vectors the LDS kernels take 1.2 to 2 times
-            # what was predicted (57x1610x1067 14.9 us for 7.5), where they are it is right (32x4096x4096)
-            limit *= 0.88 if view.N % 4 == 0 and view.K % 4 == 0 else 1.4 if view.N * view.K > 1e6 else 1.0
+        limit = (best[0] + 4360) / 1.03 if view.conv else predict(view, *kernel, call=True) / 1.08
         for m, n, pd in DIRECT_KERNELS:
             if m * 16 >= 2 * max(view.M, 16) or n * 16 >= 2 * max(view.N, 16):
                 continue
             tm, tn = ceil_div(view.M, m * 16), ceil_div(view.N, n * 16)
-            if tm * tn * m * n * view.K * 8.0 / (4 * NUM_CUS) + 4360 > limit:          # matrix clocks alone
+            if tm * tn * m * n * view.K * 8.0 / (4 * NUM_CUS) > limit:          # matrix clocks alone
                 continue
             for groups in (1, 2, 4, 8):
                 kp = ceil_div(view.K, 32 * groups) * 32 * groups
@@ -1045,7 +1060,7 @@ def _pick_f32(view, kernels, predict, padded, direct):
                 clocks = _direct_clocks(view, m, n, pd, groups)
                 if clocks < limit:
                     limit = clocks
-                    best = (clocks, [tm, 1, m, 16], [tn, 1, n, 16], [groups, kp // (32 * groups), 32], pd, 1)
+                    best = (best[0], [tm, 1, m, 16], [tn, 1, n, 16], [groups, kp // (32 * groups), 32], pd, 1)
     cfg = _empty_config()
     cfg["spatial"] = [best[1], best[2]]
     cfg["reduce"] = [best[3]]

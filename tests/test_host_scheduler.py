@@ -764,7 +764,7 @@ def test_untuned_pointwise_layers_get_larger_tiles_where_the_grid_is_not_renumbe
     assert wm * rm * mf * wn * rn * mf >= (64 * 32 if args[1] != 464 else 32 * 32)
 
 
-@pytest.mark.parametrize("m,k,n", [(23, 2029, 1834), (40, 2048, 1333), (48, 1280, 2001)])
+@pytest.mark.parametrize("m,k,n", [(108, 896, 1027), (107, 875, 1469), (158, 1661, 1138)])
 def test_search_begins_at_a_point_of_its_space(m, k, n):
     """Where an untuned product runs on tiles without LDS, which the space does not hold, the first seed is the best
     predicted kernel of the space."""
@@ -779,7 +779,7 @@ def test_search_begins_at_a_point_of_its_space(m, k, n):
 
 
 @pytest.mark.parametrize("method", ["searching", "random"])
-@pytest.mark.parametrize("func,args,variant", [(gemm, (40, 2048, 1333), 1), (conv2d, (2, 240, 35, 35, 160, 1, 1, 0, 1, 1), 2)])
+@pytest.mark.parametrize("func,args,variant", [(gemm, (38, 1088, 2331), 1), (conv2d, (2, 240, 35, 35, 160, 1, 1, 0, 1, 1), 2)])
 def test_a_tuned_operator_is_not_slower_than_an_untuned_one(func, args, variant, method):
     """The untuned config, where it is no point of the space, is measured beside what the search found, and the faster
     of the two is returned."""
@@ -796,3 +796,20 @@ def test_a_tuned_operator_is_not_slower_than_an_untuned_one(func, args, variant,
         _, _, configs = schedule(task.key, op_trial=3, graph_trial=1, parallel=2, method=method, evaluator=cost,
                                  warm_up=(1, 4), verbose=False)
         assert untuned(configs) == faster
+
+
+@pytest.mark.parametrize("m,k,n,direct", [
+    # us on tiles with LDS and on those without
+    (112, 4096, 4096, False),       # 36.6, 50.4
+    (99, 1920, 3488, False),        # 18.3, 24.9
+    (160, 768, 3072, False),        # 9.3, 16.2
+    (16, 1500, 667, False),         # 5.7, 7.2: few rows, N no multiple of 4
+    (32, 4096, 4096, False),        # 18.7, 19.7
+    (74, 3120, 1200, True),         # 22.7, 14.3
+    (40, 410, 879, True),           # 3.8, 3.1
+])
+def test_tiles_without_lds_only_where_they_are_faster(m, k, n, direct):
+    from flextensor_amd import nn
+    from flextensor_amd.te import placeholder
+    op = nn.gemm(placeholder((m, k)), placeholder((k, n))).op
+    assert (gfx950.untuned_config(op)["reorder"][0][3:] == [1]) == direct
