@@ -940,13 +940,15 @@ def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups, call=False):
               + (38 * rm * rn * mf * mf / 64 * (groups - 1)))
     if not call:
         return clocks
-    # what the picks' times showed beside the launch: rows of A that are no whole vectors, and several workgroups of
-    # wavefront groups side by side, which are in each other's way (210 and 294 tiles of 80 and 112x1500x667: 6.7 and 10.2 us)
-    if view.K % 4:
-        clocks += 0.34 * tiles * bm * steps * bk * groups * 4.0 / NUM_CUS / 31
+    # what the picks' times showed beside the launch: vectors of rows that are no whole ones lie across two lines each, and
+    # several workgroups of wavefront groups on one unit are in each other's way (210 and 294 tiles of 80 and
+    # 112x1500x667: 6.7 and 10.2 us)
+    clocks *= 0.976
+    vectors = share * steps * bk * groups * 4 / 64.0
+    clocks += 0.6 * vectors * ((bm if view.K % 4 else 0) + (bn if view.N % 4 else 0))
     if groups > 1 and min(share, beside) > 1:
-        clocks += 0.32 * chain
-    return 0.974 * clocks + 4110
+        clocks += 0.29 * chain
+    return clocks + 4150
 
 
 def _default_f32(view, padded=False, direct=True):
@@ -1011,10 +1013,10 @@ def _pick_f32(view, kernels, predict, padded, direct):
     Against it stand the tiles without LDS, which have to be predicted 8 % faster (windows of several pixels: 3 %). The
     two predictions of a call are off by 10 % each (one standard deviation; windows 7 and 11 %), fitted to the LDS picks and
     to 1 180 timings of the tiles without LDS over 210 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16).
-    Of those GEMMs 58 go without LDS; all 210 take 0.978 times the LDS
-    kernels' time in the geometric mean, six are more than 3 % slower than those, at most 1.09 times. One rule whatever the
+    Of those GEMMs 68 go without LDS; all 210 take 0.975 times the LDS
+    kernels' time in the geometric mean, nine are more than 3 % slower than those, at most 1.12 times. One rule whatever the
     rows and their alignment: 64x1500x667 6.9 us with LDS and 7.3 without, 32x4096x4096 18.7 and 19.7, 74x3120x1200 22.7 and
-    14.3, 112x4096x4096 36.6 and 50.4; 64x1610x1067 keeps LDS, wrongly (11.2 and 10.0).
+    14.3, 64x1610x1067 11.2 and 10.0, 112x4096x4096 36.6 and 50.4.
     Not for 1x1 windows, whose gathers the LDS kernels do without index arithmetic (7 x 259x90x90 -> 25 16.4 us, 18.4
     without LDS), and not for B stored [N][K] nor for batches: with few k steps the operands' latency is all there is, and tiles that share it
     through LDS have it once (96 x 197x64x197 10.0 us, 14.5 without LDS; 57x1249x714 with B^T 5.3 and 7.0)."""
