@@ -983,21 +983,22 @@ def _direct_clocks(view, m, n, pd, groups):
     share = ceil_div(tiles, NUM_CUS)
     beside = max(1, min(share, min(8, 512 // (4 * m * n + 8 * (m + n) * pd + 40)) * 4 // groups))
     step = m * n * 256                                              # matrix clocks of a wavefront's k step
-    # clocks a unit spends on a step's loads: two vectors per row block; per column one float and k (with a stride along
-    # the rows a load spreads over up to twice the lines), or a vector of n floats. Before the first step: the operands'
-    # latency, or the gathered operand's table of offsets, made once, and every pixel's padding bits; the table's entries
+    # clocks a unit spends on a step's loads: two vectors per row block; per column one float and k (with a stride of 2
+    # along the rows a load spreads over twice the lines), or a vector of n floats. Before the first step: the operands'
+    # latency, or the gathered operand's table of offsets and its pixels' padding bits, both once; the table's entries
     # are read anew in every step.
     if view.conv:
-        loads = 2 * m * 40 + 8 * n * (18.4 if view.conv["CSTRW"] > 1 else 9.5)
-        table, start, mix, store, sums, launch, entries = 210.0 * view.K / (64 * groups), 3330, 0.43, 2.43, 0, 4360, 0
+        loads = (2 * m * 25 + 8 * n * 7.5 * (2 if view.conv["CSTRW"] > 1 else 1)) * (1 + 0.05 * (groups - 1))
+        once = 188.0 * view.K / (64 * groups) + 97 * n * view.conv["CR"] * view.conv["CS"]
+        start, mix, store, sums, launch, entries = 0, 0.35, 10.2, 0, 5000, 54
     else:
         loads = 2 * m * 50 + 8 * {1: 9.7, 2: 19, 4: 26}[n]
-        table, start, mix, store, sums, launch, entries = 0, 1380, 0.23, 7.6, 29, 3930, 0
+        once, start, mix, store, sums, launch, entries = 0, 1380, 0.23, 7.6, 29, 3930, 0
     # wavefronts of one matrix core; two workgroups of two wavefronts begin on the same two of the four
-    wavefronts = 2 if share == groups == 2 and not view.conv else ceil_div(share * groups, 4)
+    wavefronts = 2 if share == groups == 2 else ceil_div(share * groups, 4)
     matrix = wavefronts * steps * step
     memory = share * groups * steps * loads
-    chain = ceil_div(share, beside) * (steps * max(94.0 / pd + 0.19 * step, step) + start) + table
+    chain = ceil_div(share, beside) * (steps * max(94.0 / pd + 0.19 * step, step) + start) + once
     # operands once at the rate of a large copy
     stream = 0 if view.conv else (view.M * view.K + view.K * view.N) * 4 / 1930.0
     longest = max(matrix, memory, chain)
@@ -1011,15 +1012,17 @@ def _pick_f32(view, kernels, predict, padded, direct):
     pass through registers, with K undivided (the groups' tiles lie beside each other in LDS).
 
     Against it stand the tiles without LDS, which have to be predicted 8 % faster (windows of several pixels: 3 %). The
-    two predictions of a call are off by 10 % each (one standard deviation; windows 7 and 11 %), fitted to the LDS picks and
-    to 1 180 timings of the tiles without LDS over 210 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16).
-    Of those GEMMs 68 go without LDS; all 210 take 0.975 times the LDS
-    kernels' time in the geometric mean, nine are more than 3 % slower than those, at most 1.12 times. One rule whatever the
-    rows and their alignment: 64x1500x667 6.9 us with LDS and 7.3 without, 32x4096x4096 18.7 and 19.7, 74x3120x1200 22.7 and
-    14.3, 64x1610x1067 11.2 and 10.0, 112x4096x4096 36.6 and 50.4.
+    two predictions of a call are off by 10 % each (one standard deviation), fitted to the LDS picks and to 1 180 timings of
+    the tiles without LDS over 210 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16), for windows to 1 853
+    and 1 242 timings over 230 layers. Of those GEMMs 68 go without LDS; all 210 take 0.975 times the LDS kernels' time in the
+    geometric mean, nine are more than 3 % slower than those, at most 1.12 times. One rule whatever the rows and their
+    alignment: 64x1500x667 6.9 us with LDS and 7.3 without, 32x4096x4096 18.7 and 19.7, 74x3120x1200 22.7 and 14.3,
+    64x1610x1067 11.2 and 10.0, 112x4096x4096 36.6 and 50.4.
     Not for 1x1 windows, whose gathers the LDS kernels do without index arithmetic (7 x 259x90x90 -> 25 16.4 us, 18.4
-    without LDS), and not for B stored [N][K] nor for batches: with few k steps the operands' latency is all there is, and tiles that share it
-    through LDS have it once (96 x 197x64x197 10.0 us, 14.5 without LDS; 57x1249x714 with B^T 5.3 and 7.0)."""
+    without LDS); not for strides of more than 2 along the rows, where the few layers timed took up to 1.5 times the predicted
+    time (16x208x51x15 -> 164 1x3 stride 3 10.9 us, 16.4 without LDS); and not for B stored [N][K] nor for batches: with few
+    k steps the operands' latency is all there is, and tiles that share it through LDS have it once (96 x 197x64x197 10.0 us,
+    14.5 without LDS; 57x1249x714 with B^T 5.3 and 7.0)."""
     best = None
     window = view.conv["CR"] * view.conv["CS"] if view.conv else 1
     for m, n, mf, bk, depth in kernels:
@@ -1047,8 +1050,8 @@ def _pick_f32(view, kernels, predict, padded, direct):
                 best = (clocks, [tm, m[0], m[1], mf], [tn, n[0], n[1], mf], [groups, steps, bk], depth)
                 kernel = (tiles, m, n, mf, bk, depth, groups)
     if direct and view.groups == 1 and view.mode != 2 and not view.trans_a and view.K >= 32 \
-            and (not view.conv or 1 < window <= 31 and view.K * 8 + 256 < LDS_BYTES):
-        limit = (best[0] + 4360) / 1.03 if view.conv else predict(view, *kernel, call=True) / 1.08
+            and (not view.conv or 1 < window <= 31 and view.K * 8 + 256 < LDS_BYTES and view.conv["CSTRW"] <= 2):
+        limit = predict(view, *kernel, call=True) / (1.03 if view.conv else 1.08)
         for m, n, pd in DIRECT_KERNELS:
             if m * 16 >= 2 * max(view.M, 16) or n * 16 >= 2 * max(view.N, 16):
                 continue
@@ -1072,54 +1075,62 @@ def _pick_f32(view, kernels, predict, padded, direct):
     return cfg, best[0]
 
 
-# kernels of the convolution's default, as F32_KERNELS: for windows of one pixel, and for larger ones (the K tiles of 72 and
-# 144 hold whole windows of 3x3 and of whatever else divides them)
+# kernels of the convolution's default, as F32_KERNELS: for windows of one pixel, and for larger ones
 CONV_KERNELS = (((1, 1), (1, 1), 16, 16, 2), ((1, 1), (1, 1), 16, 32, 3), ((2, 1), (2, 1), 16, 32, 3),
                 ((4, 1), (2, 1), 16, 32, 3), ((2, 2), (4, 1), 16, 16, 2), ((2, 1), (4, 1), 16, 16, 2),
                 ((4, 2), (4, 1), 16, 32, 5), ((2, 1), (2, 1), 32, 16, 3))
-WINDOW_KERNELS = (((1, 1), (1, 1), 16, 16, 2), ((2, 1), (4, 1), 16, 16, 2),            # any K
-                  ((1, 1), (1, 1), 16, 32, 3), ((4, 1), (2, 1), 16, 32, 3), ((2, 1), (4, 1), 16, 32, 5),
-                  ((4, 2), (4, 1), 16, 32, 3), ((4, 1), (4, 1), 16, 32, 8), ((4, 1), (4, 1), 16, 64, 8),
+WINDOW_KERNELS = (((1, 1), (1, 1), 16, 16, 2), ((2, 1), (4, 1), 16, 16, 2), ((2, 2), (4, 1), 16, 16, 2),
+                  ((2, 1), (2, 1), 32, 16, 3),                                         # any K
+                  ((1, 1), (1, 1), 16, 32, 3), ((2, 1), (2, 1), 16, 32, 3), ((4, 1), (2, 1), 16, 32, 3),
+                  ((2, 1), (4, 1), 16, 32, 5), ((4, 2), (4, 1), 16, 32, 3), ((4, 1), (4, 1), 16, 32, 8),
+                  ((4, 1), (4, 1), 16, 64, 8),
                   ((2, 1), (2, 1), 16, 144, 8), ((2, 1), (2, 1), 32, 72, 8), ((4, 1), (2, 1), 32, 72, 8))
 
 
-def _conv_clocks(view, tiles, m, n, mf, bk, depth, groups):
-    """Predicted clocks (2.38 GHz) of a convolution on the busiest compute unit; see _default_conv."""
+def _conv_clocks(view, tiles, m, n, mf, bk, depth, groups, call=False):
+    """Predicted clocks (2.38 GHz) of a convolution on the busiest compute unit, or of a whole ``call``; see
+    _default_conv. The numbers are fitted, and those of the gather stand for all that a load costs there."""
     (wm, rm), (wn, rn) = m, n
     bm, bn = wm * rm * mf, wn * rn * mf
     steps = ceil_div(view.K, bk * groups)
     nw = wm * wn * groups
     lds = groups * 2 * 4 * (bm + bn) * bk
-    if lds > LDS_BYTES:
+    window = view.conv["CR"] * view.conv["CS"]
+    if lds > LDS_BYTES or bk in (72, 144) and bk % window:              # those K tiles are for the whole windows they hold
         return None
     share = ceil_div(tiles, NUM_CUS)
     turns = ceil_div(share, max(1, min(LDS_BYTES // lds, 32 // nw)))
     step = rm * rn * mf * mf * 2 * bk / 64.0                            # matrix clocks of one wavefront's k step
     gathered = groups * bn * bk / 64.0                                  # loads of a step's gather, all wavefronts
-    window = view.conv["CR"] * view.conv["CS"]
-    stride = 1
     if window == 1:
         latency = {2: 129, 3: 125, 5: 457, 8: 1499}[depth] * (1 + 0.12 * bk / 32) + 33 * nw
         overlap = {2: 0.8, 3: 0.4, 5: 0.3, 8: 0.35}[depth]
-        gather, gather_chain, start, mix, store = 3.7, 0, 3230, 0.47, 3.0
+        gather, gather_chain, start, mix, store, sums = 3.7, 0, 3230, 0.47, 3.0, 82
         rate = 16 if tiles % 8 == 0 else 9                              # as in _f32_clocks
+        operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
     else:
-        latency = {2: 135, 3: 57, 5: 294, 8: 295 if bk > 64 else 63}[depth] * (1 + 0.12 * bk / 32) + 8.4 * nw
-        overlap = {2: 0.56, 3: 0.23, 5: 0.1, 8: 0.17}[depth]
-        # channel and tap: hoisted out of the loop (what is left are the loads), scalars, or lane by lane
-        hoisted = bk % window == 0
-        gather = 41 if hoisted else 50 if bn % 64 else 29
-        gather_chain = 0 if hoisted else 93
-        if window > 31:                                                 # position and predicate for every element
-            gather, gather_chain = gather * 2.5, gather_chain * 2
-        start, mix, store, rate = 1914, 0.88, 1.49, 274
-        stride = 6.1 if view.conv["CSTRW"] > 1 else 1                   # half of a line's pixels are used
+        latency = {2: 144, 3: 49, 5: 138, 8: 236 if bk > 64 else 6}[depth] * (1 + 0.12 * bk / 32) + 19 * nw
+        overlap, mix, store, sums = 0.14, 0.95, 5.0, 54
+        # channel and tap: hoisted out of the loop (what is left are the loads), scalars, or lane by lane; before the
+        # loop, per element of a thread its offset, or per pixel of a thread its padding bits
+        threads = wm * wn * 64
+        elements = ceil_div(bn * bk, threads)
+        pixels = 1 if threads % bn == 0 else elements
+        if bk % window == 0:
+            gather, gather_chain, start = 39, 0, 257 * elements
+        else:
+            gather, gather_chain = (32, 103) if bn % 64 == 0 else (53, 123)
+            start = pixels * 19 * window
+            if window > 31:                                             # position and predicate for every element
+                gather, gather_chain, start = gather * 1.4, gather_chain * 1.4, 257 * pixels
+        if view.conv["CSTRW"] > 1:                                      # a load's lanes lie in more lines
+            gather *= 1.3
+        operands = 0                                                    # nothing that the gather's loads do not show
     compute = ceil_div(share * nw, 4) * step * steps + share * steps * gathered * gather / 4
     chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap + gather_chain * gathered / nw) + start)
-    operands = tiles * (bm + bn * stride) * steps * bk * groups * 4.0 / NUM_CUS / rate
     longest = max(compute, chain, operands)
     return (longest + mix * (compute + chain + operands - longest) + share * bm * bn * 4 * store / 64
-            + 82 * rm * rn * mf * mf / 64 * (groups - 1))
+            + sums * rm * rn * mf * mf / 64 * (groups - 1) + (3720 if call else 0))
 
 
 def _default_conv(view, padded=False, direct=True, by_image=False):
@@ -1128,10 +1139,9 @@ def _default_conv(view, padded=False, direct=True, by_image=False):
     What differs from the plain product is the gathered operand: one float per lane and load, with its own address.
     Where the K tile holds whole windows (or the window is one pixel) the address advances by a constant; else an
     element costs its channel and tap, which are scalars where a wavefront loads from one row of the tile. Windows of
-    several pixels: fitted to 3 000 timings over 69 layers (1 .. 16 images, 16 .. 512 channels, 7 .. 112 rows; 3x3,
-    stride 1 and 2) together with the tiles without LDS; the pick is 7.8 % off the best measured kernel in the geometric
-    mean and 1.34 times for the worst layer (11 % and 1.7 times with the constants and kernels before, fitted when
-    channel, tap and predicate were computed anew for every element).
+    several pixels (2x2 .. 11x11 and single rows and columns, strides 1 .. 4, dilation 1 and 2, 1 .. 4 groups; 3 .. 512
+    channels): fitted to 1 853 timings over 230 layers together with the tiles without LDS; the pick is 4 % off the best
+    measured kernel in the geometric mean and 1.28 times for the worst layer.
     One pixel: 5 % off (1 .. 16 images, 16 .. 512 channels). Pointwise layers whose tiles are no multiple of 8 go at
     the lower rate of grids that were not renumbered by XCD: 4 x 464x49x49 -> 48 stride 2 11.96 -> 7.93 us, 8 x 144x30x30 -> 192
     stride 2 6.84 -> 5.09, 15 x 131x21x21 -> 45 5.42 -> 4.29 (with one rate up to 15 % slower than the rule before).

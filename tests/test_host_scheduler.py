@@ -815,3 +815,39 @@ def test_tiles_without_lds_only_where_they_are_faster(m, k, n, direct):
     from flextensor_amd.te import placeholder
     op = nn.gemm(placeholder((m, k)), placeholder((k, n))).op
     assert (gfx950.untuned_config(op)["reorder"][0][3:] == [1]) == direct
+
+
+@pytest.mark.parametrize("shape,direct,tile", [
+    # images, channels, rows, columns, output channels, window, stride, padding, dilation, groups; wavefronts and MFMA tiles
+    # along M and N, K tile; us before and with these
+    ((2, 22, 40, 40, 48, (5, 5), 1, (2, 2), 1, 2), False, (2, 1, 2, 1, 32)),            # K tile of 144: 10.7, 6.0
+    ((5, 6, 44, 44, 27, (7, 7), 1, (3, 3), 2, 1), False, (2, 1, 2, 1, 32)),             # 32x64 tiles: 9.5, 6.4
+    ((16, 208, 51, 15, 164, (1, 3), 3, (0, 1), 2, 1), False, (4, 1, 2, 1, 32)),         # without LDS: 16.4, 10.9
+    ((16, 26, 83, 83, 45, (3, 1), 1, (1, 0), 2, 1), False, (2, 1, 2, 1, 16)),           # without LDS: 21.2, 16.6
+    ((4, 54, 24, 24, 27, (3, 3), 1, (1, 1), 1, 1), True, (1, 1, 1, 2, 32)),             # with LDS: 7.4, 4.5
+])
+def test_kernels_of_untuned_windows(shape, direct, tile):
+    from flextensor_amd.nn import conv2d_nchw
+    from flextensor_amd.te import placeholder
+    b, c, h, w, o, window, stride, padding, dilation, groups = shape
+    op = conv2d_nchw(placeholder((b, c, h, w)), placeholder((o, c // groups) + window), stride=stride, padding=padding,
+                     dilation=dilation, groups=groups).op
+    cfg = gfx950.untuned_config(op)
+    assert (cfg["reorder"][0][3:] == [1]) == direct
+    assert tuple(cfg["spatial"][0][1:3] + cfg["spatial"][1][1:3] + [cfg["reduce"][0][2]]) == tile
+
+
+def test_k_tiles_of_whole_windows_are_for_windows_they_hold():
+    """72 and 144 are K tiles of 3x3 windows and of what else divides them; a 5x5 window is cut by them like by any other."""
+    from flextensor_amd.nn import conv2d_nchw
+    from flextensor_amd.te import placeholder
+    seen = set()
+    for o in (16, 48, 96, 200):
+        for c in (8, 22, 64):
+            for h in (9, 20, 40):
+                for r in (3, 5, 7):
+                    op = conv2d_nchw(placeholder((2, c, h, h)), placeholder((o, c, r, r)), padding=r // 2).op
+                    bk = gfx950.untuned_config(op)["reduce"][0][2]
+                    assert bk not in (72, 144) or r == 3
+                    seen.add((r, bk))
+    assert {bk for r, bk in seen if r == 3} & {72, 144}
