@@ -115,6 +115,24 @@ def test_benchmark_kernels_have_no_early_accumulator_reads(tmp_path):
     assert checked == 5
 
 
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+@pytest.mark.parametrize("op,sizes,template,define", [
+    ("gemm", (34, 2149, 1917), "direct_f32.hip", "PD"), ("gemm", (108, 896, 1027), "direct_f32.hip", "PD"),
+    ("conv2d", (13, 77, 8, 8, 130, 3, 1, 1, 1, 1), "direct_f32.hip", "CR"),
+    ("conv2d", (4, 54, 24, 24, 27, 3, 1, 1, 1, 1), "direct_f32.hip", "CR"),
+    ("conv2d", (16, 128, 57, 57, 256, 3, 2, 1, 1, 1), "igemm_f32.hip", "CR"),       # tiles that cut windows
+    ("conv2d", (2, 240, 35, 35, 160, 1, 1, 0, 1, 1), "igemm_f32.hip", "IMAGES")])
+def test_untuned_kernels_pass_the_static_checks(op, sizes, template, define):
+    """Default plans of the operators nobody tuned: tiles without LDS, gathered windows, images one at a time."""
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.task import conv2d, gemm
+    ops, bufs = (gemm if op == "gemm" else conv2d)(*sizes)
+    plan, _ = schedule_with_config_ops(ops, bufs, Config([], None))
+    assert plan.specs[-1].template == template and define in plan.specs[-1].defines
+    assert "v_mfma" in isa_hazards.assembly_of(plan.specs[-1])
+    assert isa_hazards.check_plan(plan) == []
+
+
 ARRIVAL = """
 k:
 	global_store_dword v1, v2, s[0:1] sc1
