@@ -152,7 +152,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
     int bid = blockIdx.x;
 #if XCD_REMAP
     const int nblk = TILES_M * TILES_N * CG;
-    bid = (bid % 8) * (nblk / 8) + (bid % 8 < nblk % 8 ? bid % 8 : nblk % 8) + bid / 8;
+    bid = (bid % 8) * (nblk / 8) + (nblk % 8 == 0 ? 0 : bid % 8 < nblk % 8 ? bid % 8 : nblk % 8) + bid / 8;
 #endif
     const int gi = bid / (TILES_M * TILES_N);
     int m0, n0;                         /* of the wavefront's tile */

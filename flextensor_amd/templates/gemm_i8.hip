@@ -252,7 +252,7 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
     int bid = blockIdx.x;
 #if XCD_REMAP
     /* as in igemm_f32.hip: 2752x1120x80, 172 tiles, 4.43 -> 3.77 us for renumbering counts that 8 does not divide too */
-    bid = (bid % 8) * (nblk / 8) + (bid % 8 < nblk % 8 ? bid % 8 : nblk % 8) + bid / 8;
+    bid = (bid % 8) * (nblk / 8) + (nblk % 8 == 0 ? 0 : bid % 8 < nblk % 8 ? bid % 8 : nblk % 8) + bid / 8;
 #endif
 #if SPLITK > 1
     const int kz = bid / (TILES_M * TILES_N);       /* which part of K */

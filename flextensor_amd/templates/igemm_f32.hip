@@ -721,7 +721,9 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
      * whose ragged grid is resident at once: such tiles wait for their loads' latency, not for traffic, and nothing was
      * gained (196 tiles of 1x64x56x56 -> 64 3x3 5.04 us, 5.12 renumbered). Counts 8 does not divide, in order and
      * renumbered: batch 77 x 137x64x87 5.73 -> 4.22 us, GEMM 112x288x1648 4.92 -> 3.76, 7x259x90x90 -> 25 1x1 16.6 -> 14.8. */
-    if (MODE != 1 || nblk > 256 || nblk % 8 == 0)
+    if (nblk % 8 == 0)
+        bid = (bid % 8) * (nblk / 8) + bid / 8;
+    else if (MODE != 1 || nblk > 256)
         bid = (bid % 8) * (nblk / 8) + (bid % 8 < nblk % 8 ? bid % 8 : nblk % 8) + bid / 8;
 #endif
     const int gi = bid / (TILES_M * TILES_N * SPLITK);   /* convolution group */
