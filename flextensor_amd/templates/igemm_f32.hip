@@ -765,7 +765,11 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
     auto gather_offset = [&](int k0, int e) -> unsigned {
 #if TAP_BITS
 #if ROW_SCALAR
+#if BN % NT == 0            /* the same row for all wavefronts, known when compiled */
+        const unsigned k = (unsigned)(k0 + e * NT / BN);
+#else
         const unsigned k = (unsigned)(k0 + (e * NT + gather_wave * 64) / BN);
+#endif
         const unsigned c = k / (unsigned)(CR * CS), t = k % (unsigned)(CR * CS), r = t / CS;
 #else
         const unsigned k = (unsigned)(k0 + b_row[e]);
