@@ -198,10 +198,12 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
         const int nn = n < N ? n : 0, ib = nn / OHW, p = nn % OHW;
         const int h = p / CQ * CSTRH - CPADH, w = p % CQ * CSTRW - CPADW;
         b_off[j] = (unsigned)(((ib * CC + gi * (CC / CG)) * CH + h) * CW + w) * 4u;     /* of tap (0, 0), inside or not */
-        unsigned bad = 0;
+        unsigned cols = 0, bad = 0;     /* rows and columns of the window apart, as in igemm_f32.hip */
 #pragma unroll
-        for (int t = 0; t < CR * CS; ++t)
-            bad |= (((unsigned)(h + t / CS * CDILH) < (unsigned)CH) & ((unsigned)(w + t % CS * CDILW) < (unsigned)CW) ? 0u : OOB) >> t;
+        for (int t = 0; t < CS; ++t) cols = cols << 1 | ((unsigned)(w + t * CDILW) < (unsigned)CW ? 0u : 1u);
+#pragma unroll
+        for (int t = 0; t < CR; ++t) bad = bad << CS | ((unsigned)(h + t * CDILH) < (unsigned)CH ? cols : (1u << CS) - 1u);
+        bad <<= 32 - CR * CS;
         b_bad[j] = n < N ? bad : ~0u;
 #endif
     }

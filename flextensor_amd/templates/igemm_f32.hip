@@ -966,11 +966,12 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
         if (PXE(e) != e) continue;
         const int h0 = (p / CQ) * CSTRH - CPADH, w0 = (p % CQ) * CSTRW - CPADW;
         px_base[e] = (unsigned)((b * CC + gi * (CC / CG)) * (CH * CW) + h0 * CW + w0) * 4u;
-        unsigned bad = 1;               /* the tap of a k behind K */
+        unsigned cols = 0, bad = 0;     /* rows and columns of the window apart: CR + CS compares for CR * CS taps */
 #pragma unroll
-        for (int t = 0; t < CR * CS; ++t)
-            bad |= (((unsigned)(h0 + t / CS * CDILH) < (unsigned)CH) & ((unsigned)(w0 + t % CS * CDILW) < (unsigned)CW)
-                    ? 0u : OOB) >> t;
+        for (int t = 0; t < CS; ++t) cols = cols << 1 | ((unsigned)(w0 + t * CDILW) < (unsigned)CW ? 0u : 1u);
+#pragma unroll
+        for (int t = 0; t < CR; ++t) bad = bad << CS | ((unsigned)(h0 + t * CDILH) < (unsigned)CH ? cols : (1u << CS) - 1u);
+        bad = bad << (32 - CR * CS) | 1u;       /* bit 0: the tap of a k behind K */
         px_bad[e] = inside ? bad : ~0u;
 #else
         px_ok[e] = inside;

@@ -314,3 +314,13 @@ def test_gather_of_a_single_k_tile_has_no_scalar_divisions():
     d = spec.defines
     assert d["KP"] == d["BK"] and d["WAVES_N"] * d["REP_N"] * d["MFMA"] == d["WAVES_M"] * d["WAVES_N"] * 64
     assert sum(line.split()[0].startswith("s_mul") for line in isa_hazards.assembly_of(spec).split("\n") if line.strip()) < 16
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_padding_bits_take_rows_and_columns_apart():
+    """A 5x5 window's 25 bits from 5 + 5 compares a pixel (1x16x28x28 -> 32 5x5: 4.3 us, 4.6 with 25 pairs of compares)."""
+    from flextensor_amd.tuned import lookup
+    key = "conv2d_google7_(1, 16, 28, 28, 32, 5, 1, 2, 1, 1)_rocm(0)"
+    spec = schedule_with_config(key, lookup(key))[0].specs[-1]
+    text = isa_hazards.assembly_of(spec)
+    assert spec.defines["CR"] * spec.defines["CS"] == 25 and text.count("v_cndmask") < 40
