@@ -988,9 +988,9 @@ def _direct_clocks(view, m, n, pd, groups):
     # latency, or the gathered operand's table of offsets and its pixels' padding bits, both once; the table's entries
     # are read anew in every step.
     if view.conv:
-        loads = (2 * m * 25 + 8 * n * 7.5 * (2 if view.conv["CSTRW"] > 1 else 1)) * (1 + 0.05 * (groups - 1))
-        once = 188.0 * view.K / (64 * groups) + 97 * n * view.conv["CR"] * view.conv["CS"]
-        start, mix, store, sums, launch, entries = 0, 0.35, 10.2, 0, 5000, 54
+        loads = (2 * m * 23 + 8 * n * 7.4 * (2 if view.conv["CSTRW"] > 1 else 1)) * (1 + 0.056 * (groups - 1))
+        once = 186.0 * view.K / (64 * groups) + 144 * n * (view.conv["CR"] + view.conv["CS"])
+        start, mix, store, sums, launch, entries = 0, 0.34, 9.7, 0, 4600, 62
     else:
         loads = 2 * m * 50 + 8 * {1: 9.7, 2: 19, 4: 26}[n]
         once, start, mix, store, sums, launch, entries = 0, 1380, 0.23, 7.6, 29, 3930, 0
@@ -1011,10 +1011,10 @@ def _pick_f32(view, kernels, predict, padded, direct):
     LDS kernel's also where tiles without LDS are taken); where the LDS rows are to be padded, among the kernels whose tiles
     pass through registers, with K undivided (the groups' tiles lie beside each other in LDS).
 
-    Against it stand the tiles without LDS, which have to be predicted 8 % faster (windows of several pixels: 3 %). The
+    Against it stand the tiles without LDS, which for GEMMs have to be predicted 8 % faster, for windows faster at all. The
     two predictions of a call are off by 10 % each (one standard deviation), fitted to the LDS picks and to 1 180 timings of
-    the tiles without LDS over 210 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16), for windows to 1 853
-    and 1 242 timings over 230 layers. Of those GEMMs 68 go without LDS; all 210 take 0.975 times the LDS kernels' time in the
+    the tiles without LDS over 210 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16), for windows to 1 887
+    and 1 233 timings over 230 layers. Of those GEMMs 68 go without LDS; all 210 take 0.975 times the LDS kernels' time in the
     geometric mean, nine are more than 3 % slower than those, at most 1.12 times. One rule whatever the rows and their
     alignment: 64x1500x667 6.9 us with LDS and 7.3 without, 32x4096x4096 18.7 and 19.7, 74x3120x1200 22.7 and 14.3,
     64x1610x1067 11.2 and 10.0, 112x4096x4096 36.6 and 50.4.
@@ -1051,7 +1051,7 @@ def _pick_f32(view, kernels, predict, padded, direct):
                 kernel = (tiles, m, n, mf, bk, depth, groups)
     if direct and view.groups == 1 and view.mode != 2 and not view.trans_a and view.K >= 32 \
             and (not view.conv or 1 < window <= 31 and view.K * 8 + 256 < LDS_BYTES and view.conv["CSTRW"] <= 2):
-        limit = predict(view, *kernel, call=True) / (1.03 if view.conv else 1.08)
+        limit = predict(view, *kernel, call=True) / (1 if view.conv else 1.08)
         for m, n, pd in DIRECT_KERNELS:
             if m * 16 >= 2 * max(view.M, 16) or n * 16 >= 2 * max(view.N, 16):
                 continue
@@ -1109,20 +1109,20 @@ def _conv_clocks(view, tiles, m, n, mf, bk, depth, groups, call=False):
         rate = 16 if tiles % 8 == 0 else 9                              # as in _f32_clocks
         operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
     else:
-        latency = {2: 144, 3: 49, 5: 138, 8: 236 if bk > 64 else 6}[depth] * (1 + 0.12 * bk / 32) + 19 * nw
-        overlap, mix, store, sums = 0.14, 0.95, 5.0, 54
+        latency = {2: 132, 3: 31, 5: 117, 8: 166 if bk > 64 else 3}[depth] * (1 + 0.12 * bk / 32) + 18 * nw
+        overlap, mix, store, sums = 0.13, 1.0, 4.7, 45
         # channel and tap: hoisted out of the loop (what is left are the loads), scalars, or lane by lane; before the
         # loop, per element of a thread its offset, or per pixel of a thread its padding bits
         threads = wm * wn * 64
         elements = ceil_div(bn * bk, threads)
         pixels = 1 if threads % bn == 0 else elements
         if bk % window == 0:
-            gather, gather_chain, start = 39, 0, 257 * elements
+            gather, gather_chain, start = 41, 0, 255 * elements
         else:
-            gather, gather_chain = (32, 103) if bn % 64 == 0 else (53, 123)
-            start = pixels * 19 * window
+            gather, gather_chain = (30, 98) if bn % 64 == 0 else (52, 118)
+            start = pixels * 54 * (view.conv["CR"] + view.conv["CS"])
             if window > 31:                                             # position and predicate for every element
-                gather, gather_chain, start = gather * 1.4, gather_chain * 1.4, 257 * pixels
+                gather, gather_chain, start = gather * 1.4, gather_chain * 1.4, 255 * pixels
         if view.conv["CSTRW"] > 1:                                      # a load's lanes lie in more lines
             gather *= 1.3
         operands = 0                                                    # nothing that the gather's loads do not show
@@ -1130,7 +1130,7 @@ def _conv_clocks(view, tiles, m, n, mf, bk, depth, groups, call=False):
     chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap + gather_chain * gathered / nw) + start)
     longest = max(compute, chain, operands)
     return (longest + mix * (compute + chain + operands - longest) + share * bm * bn * 4 * store / 64
-            + sums * rm * rn * mf * mf / 64 * (groups - 1) + (3720 if call else 0))
+            + sums * rm * rn * mf * mf / 64 * (groups - 1) + (3550 if call else 0))
 
 
 def _default_conv(view, padded=False, direct=True, by_image=False):
@@ -1140,8 +1140,8 @@ def _default_conv(view, padded=False, direct=True, by_image=False):
     Where the K tile holds whole windows (or the window is one pixel) the address advances by a constant; else an
     element costs its channel and tap, which are scalars where a wavefront loads from one row of the tile. Windows of
     several pixels (2x2 .. 11x11 and single rows and columns, strides 1 .. 4, dilation 1 and 2, 1 .. 4 groups; 3 .. 512
-    channels): fitted to 1 853 timings over 230 layers together with the tiles without LDS; the pick is 4 % off the best
-    measured kernel in the geometric mean and 1.28 times for the worst layer.
+    channels): fitted to 1 887 timings over 230 layers together with the tiles without LDS; the pick is 4 % off the best
+    measured kernel in the geometric mean and 1.29 times for the worst layer.
     One pixel: 5 % off (1 .. 16 images, 16 .. 512 channels). Pointwise layers whose tiles are no multiple of 8 go at
     the lower rate of grids that were not renumbered by XCD: 4 x 464x49x49 -> 48 stride 2 11.96 -> 7.93 us, 8 x 144x30x30 -> 192
     stride 2 6.84 -> 5.09, 15 x 131x21x21 -> 45 5.42 -> 4.29 (with one rate up to 15 % slower than the rule before).

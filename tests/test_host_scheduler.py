@@ -842,9 +842,9 @@ def test_k_tiles_of_whole_windows_are_for_windows_they_hold():
     from flextensor_amd.nn import conv2d_nchw
     from flextensor_amd.te import placeholder
     seen = set()
-    for o in (16, 48, 96, 200):
-        for c in (8, 22, 64):
-            for h in (9, 20, 40):
+    for o in (16, 48, 96, 256):
+        for c in (8, 22, 64, 128):
+            for h in (9, 20, 56):
                 for r in (3, 5, 7):
                     op = conv2d_nchw(placeholder((2, c, h, h)), placeholder((o, c, r, r)), padding=r // 2).op
                     bk = gfx950.untuned_config(op)["reduce"][0][2]
