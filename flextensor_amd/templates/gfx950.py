@@ -992,8 +992,10 @@ def _direct_clocks(view, m, n, pd, groups):
         once = 186.0 * view.K / (64 * groups) + 144 * n * (view.conv["CR"] + view.conv["CS"])
         start, mix, store, sums, launch, entries = 0, 0.34, 9.7, 0, 4600, 62
     else:
-        loads = 2 * m * 50 + 8 * {1: 9.7, 2: 19, 4: 26}[n]
-        once, start, mix, store, sums, launch, entries = 0, 1380, 0.23, 7.6, 29, 3930, 0
+        # rows of B that are no whole vectors: four neighbouring floats lie across two 16-byte pieces
+        column = {1: 8.2, 2: 17, 4: 23} if view.N % 4 == 0 else {1: 12.8, 2: 18.4, 4: 25.5}
+        loads = (2 * m * 44 + 8 * column[n]) * (1 + 0.025 * (groups - 1))
+        once, start, mix, store, sums, launch, entries = 0, 844, 0.24, 8.9, 9.4, 4380, 0
     # wavefronts of one matrix core; two workgroups of two wavefronts begin on the same two of the four
     wavefronts = 2 if share == groups == 2 else ceil_div(share * groups, 4)
     matrix = wavefronts * steps * step
@@ -1012,12 +1014,12 @@ def _pick_f32(view, kernels, predict, padded, direct):
     pass through registers, with K undivided (the groups' tiles lie beside each other in LDS).
 
     Against it stand the tiles without LDS, which for GEMMs have to be predicted 8 % faster, for windows faster at all. The
-    two predictions of a call are off by 10 % each (one standard deviation), fitted to the LDS picks and to 1 180 timings of
-    the tiles without LDS over 210 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16), for windows to 1 887
-    and 1 233 timings over 230 layers. Of those GEMMs 68 go without LDS; all 210 take 0.975 times the LDS kernels' time in the
-    geometric mean, nine are more than 3 % slower than those, at most 1.12 times. One rule whatever the rows and their
-    alignment: 64x1500x667 6.9 us with LDS and 7.3 without, 32x4096x4096 18.7 and 19.7, 74x3120x1200 22.7 and 14.3,
-    64x1610x1067 11.2 and 10.0, 112x4096x4096 36.6 and 50.4.
+    two predictions of a call are off by 10 % each (one standard deviation), fitted to the LDS picks and to 1 368 timings of
+    the tiles without LDS over 400 GEMMs (8 .. 4096 rows, half of them with K and N multiples of 16), for windows to 1 887
+    and 1 233 timings over 230 layers. Over 357 GEMMs timed on both, the picks take 0.979 times the LDS kernels' time in the
+    geometric mean, ten are more than 3 % slower than those, four more than 8 %. One rule whatever the rows and their
+    alignment: 64x1500x667 6.9 us with LDS and 7.3 without, 32x4096x4096 18.7 and 19.2, 74x3120x1200 22.7 and 14.3,
+    57x1610x1067 11.1 and 8.9, 112x4096x4096 36.6 and 50.4.
     Not for 1x1 windows, whose gathers the LDS kernels do without index arithmetic (7 x 259x90x90 -> 25 16.4 us, 18.4
     without LDS); not for strides of more than 2 along the rows, where the few layers timed took up to 1.5 times the predicted
     time (16x208x51x15 -> 164 1x3 stride 3 10.9 us, 16.4 without LDS); and not for B stored [N][K] nor for batches: with few

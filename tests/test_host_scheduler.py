@@ -808,6 +808,9 @@ def test_a_tuned_operator_is_not_slower_than_an_untuned_one(func, args, variant,
     (74, 3120, 1200, True),         # 22.7, 14.3
     (40, 410, 879, True),           # 3.8, 3.1
     (44, 2110, 1431, True),         # 14.3, 11.9: more tiles than units, rows that are no whole vectors
+    (36, 768, 1006, False),         # 4.1, 5.7: one float a load, from rows that are no whole vectors
+    (158, 1006, 126, False),        # 4.7, 6.1
+    (216, 1236, 278, False),        # 6.0, 7.0
     (9, 815, 1416, True),           # 4.9, 3.6
 ])
 def test_tiles_without_lds_only_where_they_are_faster(m, k, n, direct):
