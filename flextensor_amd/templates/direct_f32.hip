@@ -14,8 +14,10 @@
 // their way at a time. igemm_f32.hip shares every operand between the wavefronts of a tile through LDS and pays a
 // barrier and an LDS round trip per K tile for it; this is the better split where tiles are small or few (few rows,
 // few output channels), or where the LDS kernels compute channel, tap and predicate anew for every gathered element (here
-// they come from a table in LDS, made once per workgroup). Measured, LDS kernel and this one: 4x54x24x24 -> 27 3x3
-// 7.4 -> 4.5 us, 13x77x8x8 -> 130 3x3 11.1 -> 7.3, 34x2149x1917 11.9 -> 9.3, 23x2029x1834 14.3 -> 8.1.
+// they come from a table in LDS, made once per workgroup). Measured, LDS kernel and this one: 4x54x24x24 -> 27 3x3 5.8 and
+// 4.2 us, 13x77x8x8 -> 130 3x3 8.2 and 7.2, 74x3120x1200 22.7 and 14.4 (matrix cores busy 18 and 42 % of the time),
+// 16x119x24x23 -> 74 5x5 90.9 and 68.7; the other way round 112x4096x4096 36.6 and 50.4, 16x128x57x57 -> 256 3x3 stride 2 77.7
+// and 142.
 
 #define MODE FT_MODE
 #define M FT_M
