@@ -996,7 +996,7 @@ def _direct_clocks(view, m, n, pd, groups):
         column = {1: 8.2, 2: 17, 4: 23} if view.N % 4 == 0 else {1: 12.8, 2: 18.4, 4: 25.5}
         loads = (2 * m * 44 + 8 * column[n]) * (1 + 0.025 * (groups - 1))
         once, start, mix, store, sums, launch, entries = 0, 844, 0.24, 8.9, 9.4, 4380, 0
-    # wavefronts of one matrix core; two workgroups of two wavefronts begin on the same two of the four
+    # wavefronts of one matrix core; two workgroups of two wavefronts go as if they shared two of the four (timed, not traced)
     wavefronts = 2 if share == groups == 2 else ceil_div(share * groups, 4)
     matrix = wavefronts * steps * step
     memory = share * groups * steps * loads
