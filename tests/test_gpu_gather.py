@@ -15,6 +15,8 @@ TOL = 1e-5
     ((4, 1, 2, 1, 16), 32, 3, 2),         # two rows, K divided
     ((1, 1, 1, 1, 16), 16, 2, 4),         # four rows, one pixel a thread
     ((2, 1, 2, 1, 16), 32, 5, 1),         # two rows, straight into LDS
+    ((1, 2, 4, 4, 16), 32, 3, 1),         # all wavefronts load from one row: its number is known when compiled
+    ((1, 1, 1, 8, 16), 16, 2, 2),         # rows of two elements a thread
 ])
 @pytest.mark.parametrize("shape,bias", [
     ((2, 24, 9, 7, 19, 3, 1, 1, 1, 1), True),       # columns and rows that end inside the tile
