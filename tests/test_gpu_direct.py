@@ -111,6 +111,7 @@ def test_conv2d(oracle, shape, bias, tile, groups, ahead, variant):
 def test_defaults_take_the_tiles_without_lds(oracle, shape, func):
     """Few rows, few pixels: the default plan is one of these, and right; a call on another stream runs there."""
     import torch
+    from flextensor_amd.plan import build
     from flextensor_amd.measure import seeded_inputs
     from flextensor_amd.scheduler import schedule_with_config_ops
     from flextensor_amd.utils import Config
@@ -120,10 +121,25 @@ def test_defaults_take_the_tiles_without_lds(oracle, shape, func):
     host = seeded_inputs(bufs, seed=3)
     ref = (np.matmul(host[0].astype(np.float64), host[1].astype(np.float64)) if len(shape) == 4
            else oracle.conv2d_nchw_c(host[0], host[1], *shape[6:]))
+    assert rel(run(plan, bufs, host), ref) <= TOL
+    # the stream is busy for milliseconds before it writes the operands: a launch elsewhere would read zeros
+    func = build(plan, bufs, "rocm")
+    busy = torch.randn(2048, 2048, device="cuda")
+    new = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in host]
+    tensors = [torch.zeros_like(a) for a in new] + [torch.zeros(bufs[-1].shape, device="cuda")]
     stream = torch.cuda.Stream()
+    busy @ busy
+    torch.cuda.synchronize()
     with torch.cuda.stream(stream):
-        out = run(plan, bufs, host)
-    assert rel(out, ref) <= TOL
+        for _ in range(20):
+            busy @ busy
+        for a, b in zip(tensors, new):
+            a.copy_(b)
+        func(*tensors)
+        got = tensors[-1].clone()
+    torch.cuda.synchronize()
+    func.close()
+    assert rel(got.cpu().numpy(), ref) <= TOL
 
 
 @pytest.mark.parametrize("xcd", [0, 1])
