@@ -41,11 +41,12 @@ import tempfile
 
 # issue slots before another instruction may read the result, as the compiler's own hazard table
 # for gfx950 enforces them in straight-line code: passes + 2 for the fp32 shapes (16 and 8 passes),
-# passes + 4 for the integer ones (32x32x32: 8 passes, 16x16x64: 4 passes; the distances it leaves
-# between such an MFMA and a v_accvgpr_read of its result are exactly 12 and 8). A larger number
+# passes + 4 for the integer and the bf16 ones (32x32x32, 32x32x16: 8 passes, 16x16x64, 16x16x32: 4 passes; the distances
+# it leaves between such an MFMA and a v_accvgpr_read of its result are exactly 12 and 8). A larger number
 # here would flag the compiler's correct code; the point of the walk is to find the paths on which
 # its padding got lost.
-NEED = {"f32_32x32x2": 18, "f32_16x16x4": 10, "i32_32x32x32": 12, "i32_16x16x64": 8}
+NEED = {"f32_32x32x2": 18, "f32_16x16x4": 10, "i32_32x32x32": 12, "i32_16x16x64": 8,
+        "f32_32x32x16_bf16": 12, "f32_16x16x32_bf16": 8}
 REG = re.compile(r"\b([av])(?:\[(\d+):(\d+)\]|(\d+)\b)")
 BRANCH = re.compile(r"^s_(branch|cbranch_\w+)\s+(\S+)")
 

@@ -12,6 +12,8 @@ Operator kinds and the template each one lowers to:
   conv2d_nchw            igemm_f32.hip  MODE 1 (implicit GEMM, padding folded
                                          into the gather; or PAD=0 over a
                                          materialised padded tensor)
+                         Products in bf16 parts are the second kernel of igemm_f32.hip and of direct_f32.hip: pipeline
+                         depths 9 to 11, chosen by the defaults, not searched
   both and batch_gemm    direct_f32.hip (operands straight into registers, no LDS tiles: fourth number of the
                                          reorder entry 1; chosen by the defaults, not searched)
   conv2d_nchw, 1x1       igemm_f32.hip  MODE 0 per image where the fourth number of the reorder entry is 2 (the same)
@@ -301,6 +303,9 @@ SPECIAL_DEFAULTS = {
 # 8 = 7 with the main loop's instruction order written out (fragment reads and tile loads issued
 # one at a time between the MFMAs);
 # fp32: 6 and 7 = 5 with three and four LDS buffers (two and three tiles requested ahead)
+# fp32: 9 and 10 = products in bf16 parts (the second kernel of igemm_f32.hip), one and two k steps ahead; 11 = the same
+# with every wavefront on its own (the second kernel of direct_f32.hip)
+SPLIT_DEPTHS = {9: ("igemm_f32.hip", 1), 10: ("igemm_f32.hip", 2), 11: ("direct_f32.hip", 0)}
 PIPELINE = {1: (1, 1), 2: (2, 1), 3: (2, 2), 4: (2, 3), 5: (2, 1), 6: (2, 1), 7: (2, 1), 8: (2, 1)}
 
 
@@ -359,9 +364,10 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
     (gm, wm, rm, mfm), (gn, wn, rn, mfn) = [list(map(int, x)) for x in sp]
     splitk, kiters, bk = [int(x) for x in rd[0]]
     depth = int((config.get("unroll") or [[2, 1]])[0][0])
-    if depth not in PIPELINE:
+    split = view.dtype != "int8" and depth in SPLIT_DEPTHS
+    if depth not in PIPELINE and not split:
         raise InvalidConfig("pipeline depth %d is not available" % depth)
-    stages, pd = PIPELINE[depth]
+    stages, pd = PIPELINE.get(depth, (2, 1))
     if view.dtype != "int8" and depth in (6, 7):
         stages = depth - 3        # fp32: 6 and 7 = tiles straight into LDS with three and four buffers
     # fp32 depth 8: as 5 (two buffers), and the first operands of the next tile are read from LDS
@@ -399,7 +405,8 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
     kp = splitk * waves_k * kiters * bk
     # the fewest whole tiles that cover K will do as well (zeros behind it): int8 always, fp32 up to a quarter more;
     # tiles without LDS multiply no zeros but give some groups of wavefronts fewer steps
-    if kp not in view.KP_options and not (view.K <= kp < view.K + splitk * waves_k * bk and (i8 or direct or kp * 4 <= view.K * 5)):
+    if kp not in view.KP_options and not (view.K <= kp < view.K + splitk * waves_k * bk
+                                          and (i8 or direct or split or kp * 4 <= view.K * 5)):
         raise InvalidConfig("reduce split does not multiply to K, nor to the fewest whole tiles that cover it")
     nt = wm * wn * 64          # threads of one k-group
     D = dict(M=view.M, N=view.N, K=view.K, KP=kp, MFMA=mfm, WAVES_M=wm, WAVES_N=wn, REP_M=rm,
@@ -471,6 +478,10 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
                                 [("buf", in_names[0]), ("buf", in_names[1]), ("buf", out_name)], align=align))
         return specs
 
+    if split:
+        if bk != 32 or splitk > 1 or stream_k or direct:
+            raise InvalidConfig("products in bf16 parts: k steps of 32, K divided inside the workgroup only")
+        return _lower_split(op, view, D, depth, special, out_name, in_names, materialized_pad, bias_name, merged_out, waves_k)
     if direct:
         if mfm != 16 or bk != 32 or splitk > 1 or stream_k:
             raise InvalidConfig("operands straight into registers: 16x16 tiles, k steps of 32, K divided inside the "
@@ -658,6 +669,68 @@ def _lower_direct(op, view, D, direct, depth, out_name, in_names, materialized_p
         args.append(("buf", bias_name))
     tiles = ceil_div(view.M, D["WAVES_M"] * rm * 16) * ceil_div(view.N, D["WAVES_N"] * rn * 16)
     return [KernelSpec("direct_f32.hip", "igemm_f32", D, (tiles * view.groups, 1, 1), (waves * 64, 1, 1), args)]
+
+
+def _lower_split(op, view, D, depth, special, out_name, in_names, materialized_pad, bias_name, merged_out, waves_k):
+    """Products in three bf16 parts (the second kernels of igemm_f32.hip and direct_f32.hip)."""
+    template, ahead = SPLIT_DEPTHS[depth]
+    if view.trans_a:
+        raise InvalidConfig("products in bf16 parts need A stored [M][K]")
+    if _special(special, "lds_pad") != SPECIAL_DEFAULTS["lds_pad"]:
+        raise InvalidConfig("products in bf16 parts have an LDS layout of their own")
+    if view.mode == 1 and (view.conv["CR"] * view.conv["CS"] > 31 or view.K > 16384):
+        raise InvalidConfig("a pixel's valid taps are bits of a word, the offsets of the gathered operand's k a table")
+    keys = ["M", "N", "K", "WAVES_M", "WAVES_N", "REP_M", "REP_N", "GROUP_M", "XCD_REMAP"]
+    bm, bn = D["WAVES_M"] * D["REP_M"] * D["MFMA"], D["WAVES_N"] * D["REP_N"] * D["MFMA"]
+    waves, blocks = D["WAVES_M"] * D["WAVES_N"] * waves_k, D["REP_M"] * D["REP_N"]
+    sums = waves_k * bm * bn * 4 if waves_k > 1 else 0
+    if depth == 11:
+        if D["MFMA"] != 32 or blocks > 4 or blocks > 2 and waves_k < 4 or waves > 8 and blocks > 2:
+            raise InvalidConfig("32x32 MFMAs, up to four of them a wavefront, more than two only where K is divided by four")
+        if view.mode == 0 and D["REP_N"] not in (1, 2, 4) or view.mode == 1 and D["REP_N"] > 3:
+            raise InvalidConfig("a lane's neighbouring columns are one load, loads in flight are counted to 63")
+        rows = (D["REP_M"] + (D["REP_N"] if view.mode == 2 else 0)) * 32
+        lds = waves * 2 * rows * 128 + (ceil_div(view.K, 32) * 256 if view.mode == 1 else 0)
+    else:
+        # 2 * blocks * NACC accumulators, the parts of a row of blocks and of a block, a thread's share of the tile
+        regs = 2 * blocks * D["MFMA"] ** 2 // 64 + 12 * (D["REP_N"] + 1) + ceil_div((bm + bn) * 32 * ahead, waves // waves_k * 64) + 40
+        if regs > (512 if waves <= 4 else 256 if waves <= 8 else 128):
+            raise InvalidConfig("the tile and its loads need %d registers per lane" % regs)
+        keys.append("MFMA")
+        lds = waves_k * 2 * 192 * (bm + bn) + 16
+    if max(lds, sums) > LDS_BYTES:
+        raise InvalidConfig("LDS tiles or partial sums need %d bytes" % max(lds, sums))
+    D = {k: D[k] for k in keys}
+    D.update(SPLIT=1, MODE=view.mode, WAVES_K=waves_k)
+    if ahead:
+        D.update(PD=ahead)
+    b_bytes = view.groups * view.K * view.N * 4
+    a_name, b_name = in_names[0], in_names[1]
+    if view.mode == 1:
+        conv = dict(view.conv)
+        if materialized_pad:
+            conv["CH"] += 2 * conv["CPADH"]
+            conv["CW"] += 2 * conv["CPADW"]
+            conv["CPADH"] = conv["CPADW"] = 0
+        D.update(conv)
+        b_bytes = (conv["CB"] * conv["CC"] * conv["CH"] * conv["CW"] + conv["CPADH"] * conv["CW"] + conv["CPADW"]) * 4
+        if op.kind == "col_gemm" and merged_out is None:
+            D.update(COLOUT=1)
+    elif view.images:
+        D.update(IMAGES=view.images)
+    elif view.groups > 1:
+        D.update(CG=view.groups)
+    if op.kind in ("col_gemm", "conv2d_nchw"):
+        a_name, b_name = b_name, a_name          # A = weight, B = the image or the stored columns
+    a_bytes = (1 if view.images else view.groups) * view.M * view.K * 4
+    if max(a_bytes, b_bytes, view.groups * view.M * view.N * 4) >= 2 ** 31:
+        raise InvalidConfig("operands of 2 GiB or more are not addressable by the buffer loads")
+    args = [("buf", a_name), ("buf", b_name), ("buf", out_name)]
+    if bias_name is not None:
+        D.update(HAS_BIAS=1)
+        args.append(("buf", bias_name))
+    tiles = ceil_div(view.M, bm) * ceil_div(view.N, bn)
+    return [KernelSpec(template, "igemm_f32", D, (tiles * view.groups, 1, 1), (waves * 64, 1, 1), args)]
 
 
 def _lower_depthwise(op, config, special, out_name, in_names, materialized_pad=False, bias_name=None):
@@ -933,7 +1006,7 @@ def _f32_clocks(view, tiles, m, n, mf, bk, depth, groups, call=False):
     chain = turns * (steps * (latency + step * ceil_div(nw, 4) * overlap) + 930)
     # the lower rate was fitted when only counts that 8 divides were renumbered by XCD; it still steers to those, which
     # end in whole rounds (one rate for all: 24 drawn batches 1 % faster in the mean, single pointwise layers up to 16 % slower)
-    rate = 31 if view.groups == 1 or tiles % 8 == 0 else 14
+    rate = 31 if call or view.groups == 1 or tiles % 8 == 0 else 14
     operands = tiles * (bm + bn) * steps * bk * groups * 4.0 / NUM_CUS / rate
     longest = max(matrix, chain, operands)
     clocks = (longest + 0.35 * (matrix + chain + operands - longest) + share * bm * bn * 4 * 4.8 / 64
@@ -969,7 +1042,8 @@ def _default_f32(view, padded=False, direct=True):
     114 x 68x110x63 (B^T) 6.38 -> 4.88, 63 x 52x80x274 7.01 -> 5.21. K streaming is left to the search: a plan that owns a
     workspace cannot run on two streams at once, and a default plan can.
     """
-    return _pick_f32(view, F32_KERNELS, _f32_clocks, padded, direct)[0]
+    cfg, _, call = _pick_f32(view, F32_KERNELS, _f32_clocks, padded, direct)
+    return _or_split(view, cfg, call) if direct and not padded else cfg
 
 
 # kernels without LDS tiles that the defaults choose among: MFMA tiles per wavefront along M and N, k steps ahead
@@ -1009,8 +1083,8 @@ def _direct_clocks(view, m, n, pd, groups):
 
 
 def _pick_f32(view, kernels, predict, padded, direct):
-    """The config of the kernel and number of wavefront K groups with the smallest predicted time, and that time (the
-    LDS kernel's also where tiles without LDS are taken); where the LDS rows are to be padded, among the kernels whose tiles
+    """The config of the kernel and number of wavefront K groups with the smallest predicted time, that time (the
+    LDS kernel's also where tiles without LDS are taken), and the predicted time of a call; where the LDS rows are to be padded, among the kernels whose tiles
     pass through registers, with K undivided (the groups' tiles lie beside each other in LDS).
 
     Against it stand the tiles without LDS, which for GEMMs have to be predicted 8 % faster, for windows faster at all. The
@@ -1051,9 +1125,10 @@ def _pick_f32(view, kernels, predict, padded, direct):
             if clocks is not None and (best is None or clocks < best[0]):
                 best = (clocks, [tm, m[0], m[1], mf], [tn, n[0], n[1], mf], [groups, steps, bk], depth)
                 kernel = (tiles, m, n, mf, bk, depth, groups)
+    call = predict(view, *kernel, call=True)
     if direct and view.groups == 1 and view.mode != 2 and not view.trans_a and view.K >= 32 \
             and (not view.conv or 1 < window <= 31 and view.K * 8 + 256 < LDS_BYTES and view.conv["CSTRW"] <= 2):
-        limit = predict(view, *kernel, call=True) / (1 if view.conv else 1.08)
+        limit = call / (1 if view.conv else 1.08)
         for m, n, pd in DIRECT_KERNELS:
             if m * 16 >= 2 * max(view.M, 16) or n * 16 >= 2 * max(view.N, 16):
                 continue
@@ -1066,7 +1141,7 @@ def _pick_f32(view, kernels, predict, padded, direct):
                     continue
                 clocks = _direct_clocks(view, m, n, pd, groups)
                 if clocks < limit:
-                    limit = clocks
+                    limit = call = clocks
                     best = (best[0], [tm, 1, m, 16], [tn, 1, n, 16], [groups, kp // (32 * groups), 32], pd, 1)
     cfg = _empty_config()
     cfg["spatial"] = [best[1], best[2]]
@@ -1074,7 +1149,107 @@ def _pick_f32(view, kernels, predict, padded, direct):
     cfg["unroll"] = [[best[4], 1]]
     cfg["fuse"] = [[4]]
     cfg["reorder"] = [[1, 1 if best[3][0] > 1 else 0, 0] + list(best[5:])]
-    return cfg, best[0]
+    return cfg, best[0], call
+
+
+# kernels of products in bf16 parts that the defaults choose among: (wavefronts, MFMA tiles per wavefront) along M and N,
+# MFMA edge, K groups, pipeline depth; and 32x32 MFMA tiles along M and N of a wavefront on its own, K groups
+SPLIT_KERNELS = (((2, 2), (4, 1), 32, 1, 9), ((4, 1), (2, 1), 32, 1, 9), ((4, 1), (2, 1), 32, 2, 9), ((2, 2), (4, 1), 16, 1, 9),
+                 ((2, 2), (4, 1), 16, 2, 9), ((2, 2), (4, 1), 16, 2, 10), ((2, 1), (4, 1), 16, 1, 9))
+ALONE_KERNELS = ((2, 2, 8), (2, 2, 4), (2, 1, 8), (1, 1, 8), (1, 1, 4))
+
+
+def _split_clocks(view, m, n, mf, groups):
+    """Predicted clocks (2.38 GHz) of a call of the split kernel of igemm_f32.hip; see _or_split."""
+    (wm, rm), (wn, rn) = m, n
+    bm, bn = wm * rm * mf, wn * rn * mf
+    conv, waves = view.conv is not None, wm * wn * groups
+    tiles = ceil_div(view.M, bm) * ceil_div(view.N, bn) * view.groups
+    share, steps = ceil_div(tiles, NUM_CUS), ceil_div(ceil_div(view.K, 32), groups)
+    turns = ceil_div(share, max(1, min(share, LDS_BYTES // (groups * 384 * (bm + bn) + 16), 32 // waves)))
+    # a step of all groups on one unit: instructions (an MFMA keeps the others out for 8 clocks, 10 the large one, another
+    # for 4), LDS (six bytes an element in at 70 bytes a clock, out at 230), loads (rows of whole lines by the kilobyte, a
+    # vector less where rows are no whole ones; the gathered operand by 64 elements)
+    elements = (bm + bn) * 32 / (wm * wn * 64.0)
+    vector = elements * 6 + (bn * 64 / (wm * wn * 64.0) if conv else 0)
+    issue = waves * (6 * rm * rn * (20 if mf == 32 else 8) + 4 * (vector + 1)) / 4
+    lds = groups * ((bm + bn) * 192 / 70.0 + wm * wn * (rm + rn) * mf * 192 / 230.0) * (0.97 if conv else 0.86)
+    loads = groups * bm * 0.125 * 28 * (1.3 if view.K % 4 else 1)
+    if conv:
+        loads += groups * bn * 0.5 * 11.1 * (1.67 if view.conv["CSTRW"] > 1 else 1)
+        latency, start, mix, store, sums, launch = 529 + 478 + 17.2 * waves, 434 + 876, 0.518, 6.45, 139, 4110
+    else:
+        loads += groups * bn * 0.125 * 5.15 * (1.3 if (view.K if view.mode == 2 else view.N) % 4 else 1)
+        latency, start, mix, store, sums, launch = 616 + 4.8 * waves, 412, 0.467, 6.93, 134, 3780
+    longest = max(issue, lds, loads)
+    work = longest + mix * (issue + lds + loads - longest)
+    return (max(share * steps * work, turns * steps * (latency + 0.6 * work)) + turns * start + share * bm * bn * store / 16
+            + sums * bm * bn / 64.0 * (groups - 1) / (wm * wn) + launch)
+
+
+def _alone_clocks(view, rm, rn, groups):
+    """Predicted clocks (2.38 GHz) of a call of the split kernel of direct_f32.hip; see _or_split."""
+    conv = view.conv is not None
+    tiles = ceil_div(view.M, 32 * rm) * ceil_div(view.N, 32 * rn) * view.groups
+    share, steps = ceil_div(tiles, NUM_CUS), ceil_div(ceil_div(view.K, 32), groups)
+    lds = max(groups * (rm + (rn if view.mode == 2 else 0)) * 8192 + (view.K * 8 if conv else 0), groups * rm * rn * 4096)
+    turns = ceil_div(share, max(1, min(share, LDS_BYTES // lds, max(1, (8 if rm * rn > 2 else 12) // groups))))
+    issue = groups * (120 * rm * rn + 4 * ((rm + rn) * 96 + (48 * rn if conv else 0))) / 4.0
+    if conv:
+        loads = groups * (rm * 4 * 4.4 * (1.3 if view.K % 4 else 1) + 16 * rn * 3.5 * (4.43 if view.conv["CSTRW"] > 1 else 1))
+        latency, mix, store, sums, launch = 1020 + 123, 0.394, 20, 263, 4530
+        start = 25 + 38.6 * rn * (view.conv["CR"] + view.conv["CS"]) + 1480.0 * view.K / (groups * 64)
+    else:
+        rows = rm * 4 + (rn * 4 if view.mode == 2 else 0)
+        loads = groups * (rows * 11.8 * (1.3 if view.K % 4 else 1)
+                          + (0 if view.mode == 2 else 16 * 1.49 * (1 if rn == 2 else 0.75) * (1.3 if view.N % 4 else 1)))
+        latency, start, mix, store, sums, launch = 1490, 1180, 1.34, 14.9, 274, 2170
+    longest = max(issue, loads)
+    work = longest + mix * (issue + loads - longest)
+    return (max(share * steps * work, turns * steps * (latency + 0.5 * work)) + turns * start + share * rm * rn * 1024 * store / 16
+            + sums * rm * rn * (groups - 1) + launch)
+
+
+def _or_split(view, cfg, call):
+    """``cfg``, whose call is predicted to take ``call`` clocks, or the best predicted kernel with products in bf16 parts
+    where that is 8 % and 500 clocks faster.
+
+    Both predictions were fitted to 2 427 timings over 150 operators (GEMMs of 8 .. 4096 an axis, batches of 8 .. 128, 3x3 and
+    1x1 layers of 1 .. 16 images, 16 .. 512 channels, stride 1 and 2) and are off by 10 % (one standard deviation), like
+    those of the fp32 kernels. Over these operators the picks take 0.954 times the time without them in the geometric mean
+    (0.937 if every pick were the fastest), four are more than 2 % slower (10.3 us at 1.11), and all of them together 1 866
+    us for 2 149: what is long gains most.
+    Four blocks of a wavefront on its own have one set of accumulators, which rounds 1.3 times as much as the fp32 kernels
+    do with K divided alike: they are for at least twice the groups."""
+    if view.trans_a or view.K < 32 or view.conv and (
+            view.groups > 1 or view.conv["CR"] * view.conv["CS"] > 31 or view.conv["CSTRW"] > 2 or view.K > 4096):
+        return cfg
+    limit, best = (call - 500) / 1.08, None
+    before = cfg["reduce"][0][0]
+    for m, n, mf, groups, depth in SPLIT_KERNELS:
+        if m[0] * m[1] * mf >= 2 * max(view.M, 16) or n[0] * n[1] * mf >= 2 * max(view.N, 16) or depth == 10 and view.K < 192:
+            continue
+        clocks = _split_clocks(view, m, n, mf, groups) * (0.99 if depth == 10 else 1) if view.K >= 64 * groups else limit
+        if clocks < limit:
+            limit, best = clocks, ((m[0], m[1], mf), (n[0], n[1], mf), groups, depth)
+    for rm, rn, groups in ALONE_KERNELS:
+        if rm * 32 >= 2 * max(view.M, 32) or rn * 32 >= 2 * max(view.N, 32) or view.K < 32 * groups \
+                or rm * rn == 4 and groups < 2 * before:
+            continue
+        lds = groups * 8192 * (rm + (rn if view.mode == 2 else 0)) + (ceil_div(view.K, 32) * 256 if view.conv else 0)
+        clocks = _alone_clocks(view, rm, rn, groups) if lds <= LDS_BYTES else limit
+        if clocks < limit:
+            limit, best = clocks, ((1, rm, 32), (1, rn, 32), groups, 11)
+    if best is None:
+        return cfg
+    (wm, rm, mf), (wn, rn, _), groups, depth = best
+    cfg = _empty_config()
+    cfg["spatial"] = [[ceil_div(view.M, wm * rm * mf), wm, rm, mf], [ceil_div(view.N, wn * rn * mf), wn, rn, mf]]
+    cfg["reduce"] = [[groups, ceil_div(view.K, 32 * groups), 32]]
+    cfg["unroll"] = [[depth, 1]]
+    cfg["fuse"] = [[4]]
+    cfg["reorder"] = [[1, 1 if groups > 1 else 0, 0]]
+    return cfg
 
 
 # kernels of the convolution's default, as F32_KERNELS: for windows of one pixel, and for larger ones
@@ -1155,14 +1330,18 @@ def _default_conv(view, padded=False, direct=True, by_image=False):
     their picks took.
     """
     window = view.conv["CR"] * view.conv["CS"]
-    cfg, clocks = _pick_f32(view, WINDOW_KERNELS if window > 1 else CONV_KERNELS, _conv_clocks, padded, direct)
+    cfg, clocks, call = _pick_f32(view, WINDOW_KERNELS if window > 1 else CONV_KERNELS, _conv_clocks, padded, direct)
+    if window == 1:
+        call = 0.78 * clocks + 3660
     # images of few pixels end in tiles that are partly empty, and several of them keep the gather's larger tiles
     if view.pixels is not None and by_image and (view.pixels[0] == 1 or view.pixels[1] >= 512):
-        image, image_clocks = _pick_f32(view.by_image(), F32_KERNELS, _f32_clocks, padded, False)
-        if 0.98 * image_clocks + 4130 < 0.78 * clocks + 3660:
+        image, image_clocks, _ = _pick_f32(view.by_image(), F32_KERNELS, _f32_clocks, padded, False)
+        if 0.98 * image_clocks + 4130 < call:
+            if direct and not padded:
+                image = _or_split(view.by_image(), image, 0.98 * image_clocks + 4130)
             image["reorder"] = [image["reorder"][0] + [2]]
             return image
-    return cfg
+    return _or_split(view, cfg, call) if direct and not padded else cfg
 
 
 def default_config(op, padded=False, direct=False):

@@ -68,6 +68,8 @@
 //                   slot; the workgroup that arrives last at the tile's
 //                   counter sums the slots in a fixed order and stores the
 //                   tile (no waiting, no zero fill, deterministic)
+//   SPLIT           1: the second kernel of this file, products on the bf16 matrix
+//                   cores, which has knobs of its own
 //   GROUP_M         tile-traversal group height (L2 locality)
 //   XCD_REMAP       1: consecutive logical tiles stay on one XCD
 //   APAD / BPAD     LDS row padding in floats; APAD = -1 selects an unpadded
@@ -81,6 +83,7 @@
 // Within a k-block of 4*KL values, lane group g of an MFMA takes
 // k = 4*g + s at step s for both operands, so the sum over k is unchanged.
 
+#ifndef FT_SPLIT
 /* Constants arrive as -DFT_<NAME>=value: single-letter macros on the command line
  * would be visible to (and break) the runtime-compilation built-in headers. */
 #ifdef FT_IMAGES
@@ -1450,3 +1453,641 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 #endif
     CLK_END;
 }
+
+#else  /* FT_SPLIT */
+/* ============ the same operators on the bf16 matrix cores: FT_SPLIT ================================================
+ *
+ * An fp32 number is the sum of three bf16 numbers, x = h + m + l: h is x rounded to bf16, m the remainder rounded, l what
+ * then remains (24 bits of significand are three times eight; both subtractions are exact). Of the nine products of the
+ * parts the six of up to 2^-18 of the largest are summed by v_mfma_f32_*_bf16 in fp32, the other three are below 2^-26.
+ * A 16x16x32 bf16 MFMA takes 16 clocks, the eight fp32 MFMAs of the same block 256, so six of them are 2.7 times as fast.
+ * The five small products have accumulators of their own, so the large sum is rounded once every 32 (16) k where the fp32
+ * MFMA rounds it every four: relative error against float64, fp32 MFMA and this, GEMM 1000x1531x777 7.0e-7 and 1.6e-7,
+ * 3x3 16x128x57x57 -> 256 4.2e-7 and 1.5e-7, batch 96 x 197x64x197 1.4e-7 and 0.5e-7.
+ *
+ * Two kinds of numbers have no such parts: infinities, NaN and what rounds to a bf16 infinity (their remainder is NaN, so
+ * a sum is, and every sum is looked at), and those below 2^-110, whose l is smaller than the least bf16 number. A thread
+ * keeps the largest of what it loads of a row or column; where that is below 2^-100 and not zero, or a sum is no finite
+ * number, the workgroup does its part of K again with fp32 MFMAs, slowly, straight from memory. Otherwise a part that is
+ * lost is below 2^-134, which is 2^-34 of the largest.
+ *
+ * What bounds it: a vector instruction and an MFMA overlap for half of the MFMA's clocks only, the split is twelve
+ * instructions for two numbers, and a wavefront writes LDS at 70 bytes a clock and unit (reads: 230). So operands are
+ * split once per workgroup, on the way from memory to LDS: a tile is three planes of bf16, rows of 32 k, read as one
+ * 16-byte load per lane, part and block. Rows of A (and B^T) are loaded eight lanes a row, whole cache lines: 16 rows of
+ * 64 bytes an instruction, which is what an MFMA's lanes would need, run at 15 bytes a clock and unit, eight rows of 128
+ * at 44. Within a step chunk c of a row holds k = 4c .. 4c + 3 and 16 + 4c .. 19 + 4c, whichever operand.
+ * Measured, LDS tiles of fp32 MFMAs and this: 3x3 stride 2 16x128x57x57 -> 256 77.7 and 52 us, GEMM 1024^3 18.5 and 16.6,
+ * 1000x1531x777 27.4 and 22.9, batch 96 x 197x64x197 (B^T) 10.3 and 8.9.
+ *
+ *   PD         k steps of 32 in registers, or on their way to them
+ *   WAVES_K    wavefront groups that divide K, each with LDS tiles of its own, summed through LDS at the end */
+#define MODE FT_MODE
+#define M FT_M
+#define N FT_N
+#define K FT_K
+#define MFMA FT_MFMA
+#define WAVES_M FT_WAVES_M
+#define WAVES_N FT_WAVES_N
+#define REP_M FT_REP_M
+#define REP_N FT_REP_N
+#define WAVES_K FT_WAVES_K
+#define PD FT_PD                /* k steps in registers or on their way to them */
+#define GROUP_M FT_GROUP_M
+#define XCD_REMAP FT_XCD_REMAP
+#ifdef FT_HAS_BIAS
+#define HAS_BIAS FT_HAS_BIAS
+#else
+#define HAS_BIAS 0
+#endif
+#ifdef FT_COLOUT
+#define COLOUT FT_COLOUT
+#else
+#define COLOUT 0
+#endif
+#ifdef FT_IMAGES
+#define IMAGES FT_IMAGES
+#define CG FT_IMAGES
+#define AGROUP(g) 0               /* one weight and bias for every image */
+#else
+#define IMAGES 0
+#define AGROUP(g) (g)
+#ifdef FT_CG
+#define CG FT_CG
+#else
+#define CG 1
+#endif
+#endif
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+#if MFMA == 32
+typedef f32x16 acc_t;
+#define NACC 16
+#define SPLIT_OP(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16((a), (b), (c), 0, 0, 0)
+#define MFMA_OP(a, b, c) __builtin_amdgcn_mfma_f32_32x32x2f32((a), (b), (c), 0, 0, 0)
+#else
+typedef f32x4 acc_t;
+#define NACC 4
+#define SPLIT_OP(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16((a), (b), (c), 0, 0, 0)
+#define MFMA_OP(a, b, c) __builtin_amdgcn_mfma_f32_16x16x4f32((a), (b), (c), 0, 0, 0)
+#endif
+#define KL (64 / MFMA)                  /* lane groups of an MFMA */
+#define KH (4 / KL)                     /* MFMAs that a step's 32 k take */
+#define BM (WAVES_M * REP_M * MFMA)
+#define BN (WAVES_N * REP_N * MFMA)
+#define NT (WAVES_M * WAVES_N * 64)     /* threads of one k group */
+#define NTW (NT * WAVES_K)
+#define TILES_M ((M + BM - 1) / BM)
+#define TILES_N ((N + BN - 1) / BN)
+#define STEPS ((K + 31) / 32)
+#define GSTEPS ((STEPS + WAVES_K - 1) / WAVES_K)
+#define NBLK (REP_M * REP_N)
+
+#define OOB 0x80000000u
+#if MODE == 1
+#define CB FT_CB
+#define CC FT_CC
+#define CH FT_CH
+#define CW FT_CW
+#define CR FT_CR
+#define CS FT_CS
+#define CSTRH FT_CSTRH
+#define CSTRW FT_CSTRW
+#define CPADH FT_CPADH
+#define CPADW FT_CPADW
+#define CDILH FT_CDILH
+#define CDILW FT_CDILW
+#define CP FT_CP
+#define CQ FT_CQ
+#define OHW (CP * CQ)
+#define PADDED (CPADH > 0 || CPADW > 0)
+#define PAD_BYTES ((CPADH * CW + CPADW) * 4)
+#define B_BYTES (CB * CC * CH * CW * 4)
+#else
+#define B_BYTES (CG * K * N * 4)
+#endif
+#define A_BYTES ((IMAGES ? 1 : CG) * M * K * 4)
+
+/* LDS: three planes of [rows][32] bf16 for A, then for B; a row is four chunks of eight k */
+#define PLANE_A (BM * 64)
+#define PLANE_B (BN * 64)
+#define TILE_BYTES (3 * (PLANE_A + PLANE_B))
+#define GROUP_BYTES (2 * TILE_BYTES)
+#define SUM_BYTES (WAVES_K > 1 ? WAVES_K * BM * BN * 4 : 0)
+#define SMEM_BYTES (WAVES_K * GROUP_BYTES > SUM_BYTES ? WAVES_K * GROUP_BYTES : SUM_BYTES)
+/* chunk c of a row lies at c ^ CHUNK_XOR(row): 16 lanes that read the chunks of an MFMA's rows, or write the same chunk of
+ * 16 rows, are in 16 different groups of four banks (the order in which lanes are served: see SWZ_G above) */
+#define CHUNK_XOR(row) ((((((row) >> 2) ^ ((row) >> 3)) & 1) << 1) | (((row) >> 3) & 1))
+
+/* rows of k-contiguous operands: 16-byte vectors, eight lanes a row */
+#define EA ((BM * 8 + NT - 1) / NT)
+/* B [K][N]: tasks of NV columns, one load for each of four k; the gathered operand: tasks of a column and eight k */
+#if MODE == 2
+#define EB ((BN * 8 + NT - 1) / NT)
+#define NV 1
+#elif MODE == 0
+#if BN % 64 == 0 && 2 * BN >= NT
+#define NV 4
+#elif BN % 32 == 0 && 4 * BN >= NT
+#define NV 2
+#else
+#define NV 1
+#endif
+#define EB ((BN / NV * 8 + NT - 1) / NT)
+#else
+#define NV 1
+#define EB ((BN * 4 + NT - 1) / NT)
+#endif
+/* LDS row -> column of the tile: the NV columns of a task are rows of NV different blocks of 16 */
+#define COLUMN(row) ((row) / (16 * NV) * (16 * NV) + NV * ((row) % 16) + (row) / 16 % NV)
+
+#ifdef FT_CLKPROBE          /* as above */
+#define CLK_PARAM , unsigned long long* __restrict__ ft_clk
+#if FT_CLKPROBE == 2
+#define CLK_BEGIN const unsigned long long ft_r0 = wall_clock64();
+#define CLK_END do { __builtin_amdgcn_s_waitcnt(0x0F70); \
+        if (threadIdx.x == 0) { ft_clk[2 * blockIdx.x] = ft_r0; ft_clk[2 * blockIdx.x + 1] = wall_clock64(); } } while (0)
+#else
+#define CLK_BEGIN const unsigned long long ft_t0 = __builtin_readcyclecounter(), ft_r0 = wall_clock64();
+#define CLK_END do { __builtin_amdgcn_s_waitcnt(0x0F70); \
+        if (threadIdx.x == 0) { ft_clk[2 * blockIdx.x] = __builtin_readcyclecounter() - ft_t0; \
+                                ft_clk[2 * blockIdx.x + 1] = wall_clock64() - ft_r0; } } while (0)
+#endif
+#else
+#define CLK_PARAM
+#define CLK_BEGIN
+#define CLK_END do { } while (0)
+#endif
+
+static __device__ __forceinline__ float ld1(__amdgpu_buffer_rsrc_t r, unsigned vo, int so) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, so, 0));
+}
+static __device__ __forceinline__ f32x2 ld2(__amdgpu_buffer_rsrc_t r, unsigned vo, int so) {
+    return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)vo, so, 0));
+}
+static __device__ __forceinline__ f32x4 ld4(__amdgpu_buffer_rsrc_t r, unsigned vo, int so) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)vo, so, 0));
+}
+
+#if MODE == 1
+struct tap_table { unsigned e[STEPS * 64]; };
+static constexpr tap_table make_taps() {
+    tap_table t = {};
+    for (int k = 0; k < STEPS * 32; ++k) {
+        const int c = k / (CR * CS), w = k % (CR * CS);
+        t.e[2 * k] = k < K ? (unsigned)(c * (CH * CW) + w / CS * CDILH * CW + w % CS * CDILW) * 4u : 0u;
+        t.e[2 * k + 1] = k < K ? (unsigned)w : 31u;
+    }
+    return t;
+}
+static __constant__ const tap_table taps = make_taps();
+#endif
+
+extern "C" __global__ __launch_bounds__(NTW)
+void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C
+#if HAS_BIAS
+               , const float* __restrict__ bias
+#endif
+               CLK_PARAM)
+{
+    CLK_BEGIN
+    __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM_BYTES];
+    __shared__ unsigned redo;
+#if WAVES_K > 1
+    const int kg = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / NT));
+    const int tid = threadIdx.x - kg * NT;
+#else
+    const int kg = 0;
+    const int tid = threadIdx.x;
+#endif
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+    const int li = lane % MFMA, lg = lane / MFMA;
+    unsigned char* const lds = smem + kg * GROUP_BYTES;
+
+    int bid = blockIdx.x;
+    if (XCD_REMAP) {                    /* neighbouring tiles share an XCD; the first count % 8 XCDs have one more */
+        const int count = TILES_M * TILES_N * CG;
+        bid = (bid % 8) * (count / 8) + (bid % 8 < count % 8 ? bid % 8 : count % 8) + bid / 8;
+    }
+    const int gi = bid / (TILES_M * TILES_N);
+    int m0, n0;
+    {
+        const int r = bid % (TILES_M * TILES_N);
+        const int first_m = r / (GROUP_M * TILES_N) * GROUP_M;
+        const int gsz = (TILES_M - first_m) < GROUP_M ? (TILES_M - first_m) : GROUP_M;
+        const int rr = r % (GROUP_M * TILES_N);
+        m0 = (first_m + rr % gsz) * BM;
+        n0 = (rr / gsz) * BN;
+    }
+    const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, A_BYTES, 0x00020000);
+#if MODE == 1
+    const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<char*>(const_cast<float*>(B)) - PAD_BYTES, 0, B_BYTES + PAD_BYTES, 0x00020000);
+#else
+    const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, B_BYTES, 0x00020000);
+#endif
+
+    /* ---- what this thread loads and where it goes in LDS ---------------------------------------------------- */
+    unsigned a_off[EA], a_lds[EA];
+#pragma unroll
+    for (int e = 0; e < EA; ++e) {
+        const int q = tid + e * NT, row = q / 8, v = q % 8, m = m0 + row;
+        const unsigned off = (unsigned)((AGROUP(gi) * M + m) * K + 4 * v) * 4u;
+        a_off[e] = (m < M) & (row < BM) ? off : OOB;
+        a_lds[e] = (unsigned)(row * 64 + ((v & 3) ^ CHUNK_XOR(row)) * 16 + (v >> 2) * 8);
+    }
+    unsigned b_off[EB], b_lds[EB];
+#if MODE == 1
+    unsigned b_bad[EB];
+    /* of column n: byte offset of tap (0, 0), counted from PAD_BYTES before the image, and the word whose bit 31 - t says
+     * that tap t is padding (bit 0, the tap of a k behind K, always) */
+    auto pixel = [&](int n, unsigned& at, unsigned& bad) {
+        const int nn = n < N ? n : 0, ib = nn / OHW, p = nn % OHW;
+        const int h = p / CQ * CSTRH, w = p % CQ * CSTRW;
+        at = (unsigned)(((ib * CC + gi * (CC / CG)) * CH + h) * CW + w) * 4u;
+        unsigned cols = 0, b = 0;       /* rows and columns of the window apart */
+#pragma unroll
+        for (int t = 0; t < CS; ++t) cols = cols << 1 | ((unsigned)(w - CPADW + t * CDILW) < (unsigned)CW ? 0u : 1u);
+#pragma unroll
+        for (int t = 0; t < CR; ++t) b = b << CS | ((unsigned)(h - CPADH + t * CDILH) < (unsigned)CH ? cols : (1u << CS) - 1u);
+        bad = n < N ? b << (32 - CR * CS) | 1u : ~0u;
+    };
+#endif
+#pragma unroll
+    for (int e = 0; e < EB; ++e) {
+        const int q = tid + e * NT;
+#if MODE == 2
+        const int row = q / 8, v = q % 8, n = n0 + row;
+        const unsigned off = (unsigned)((gi * N + n) * K + 4 * v) * 4u;
+        b_off[e] = (n < N) & (row < BN) ? off : OOB;
+        b_lds[e] = (unsigned)(row * 64 + ((v & 3) ^ CHUNK_XOR(row)) * 16 + (v >> 2) * 8);
+#elif MODE == 0
+        /* 16 lanes of NV columns, by four k: quad u is half (u & 1) of chunk u >> 1 */
+        const int g = q / 16 / 8, u = q / 16 % 8, l = q % 16, c0 = g * 16 * NV;
+        const int n = n0 + c0 + NV * l;
+        const unsigned off = (unsigned)((gi * K + 4 * (u >> 1) + 16 * (u & 1)) * N + n) * 4u;
+        b_off[e] = (n < N) & (c0 < BN) ? off : OOB;
+        const int row = c0 + l;       
+        b_lds[e] = (unsigned)(row * 64 + ((u >> 1) ^ CHUNK_XOR(row)) * 16 + (u & 1) * 8);
+#else
+        const int row = q % BN, n = n0 + row;
+        pixel(q < 4 * BN ? n : N, b_off[e], b_bad[e]);
+        b_lds[e] = (unsigned)(row * 64 + ((q / BN) ^ CHUNK_XOR(row)) * 16);
+#endif
+    }
+
+    f32x4 axs[PD][EA];
+#if MODE == 2
+    f32x4 bxs[PD][EB];
+#elif MODE == 0
+    float bxs[PD][EB][4][NV];
+#else
+    float bxs[PD][EB][8];
+#endif
+    auto load = [&](int s, int set) {
+        auto& ax = axs[set];
+        auto& bx = bxs[set];
+        const int k0 = (s < STEPS ? s : STEPS - 1) * 32;
+#pragma unroll
+        for (int e = 0; e < EA; ++e) ax[e] = ld4(rsrc_a, a_off[e], k0 * 4);
+#pragma unroll
+        for (int e = 0; e < EB; ++e) {
+#if MODE == 2
+            bx[e] = ld4(rsrc_b, b_off[e], k0 * 4);
+#elif MODE == 0
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const unsigned vo = b_off[e] + (unsigned)(i * N * 4);
+#if NV == 4
+                const f32x4 y = ld4(rsrc_b, vo, k0 * (N * 4));
+#elif NV == 2
+                const f32x2 y = ld2(rsrc_b, vo, k0 * (N * 4));
+#else
+                const float y[1] = {ld1(rsrc_b, vo, k0 * (N * 4))};
+#endif
+#pragma unroll
+                for (int j = 0; j < NV; ++j) bx[e][i][j] = y[j];
+            }
+#else
+#if BN % 64 == 0
+            const int oct = __builtin_amdgcn_readfirstlane((tid + e * NT) / BN) & 3;
+#else
+            const int oct = (tid + e * NT) / BN & 3;
+#endif
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int k = k0 + 4 * oct + (i & 3) + (i & 4) * 4;
+                const unsigned off = taps.e[2 * k], tap = taps.e[2 * k + 1];
+#if PADDED || K % 32 != 0 || N % BN != 0 || (BN * 4) % NT != 0
+                const unsigned vo = b_off[e] | ((b_bad[e] << tap) & OOB);
+#else
+                const unsigned vo = b_off[e];
+#endif
+#if BN % 64 == 0
+                bx[e][i] = ld1(rsrc_b, vo, (int)off);
+#else
+                bx[e][i] = ld1(rsrc_b, vo + off, 0);
+#endif
+            }
+#endif
+        }
+    };
+    /* zeroes what loads took from behind K, and all of a step behind the last */
+    auto cut = [&](int s, int set) {
+        auto& ax = axs[set];
+        auto& bx = bxs[set];
+#pragma unroll
+        for (int e = 0; e < EA; ++e)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ax[e][i] = s * 32 + 4 * ((tid + e * NT) % 8) + i < K ? ax[e][i] : 0.0f;
+#pragma unroll
+        for (int e = 0; e < EB; ++e) {
+#if MODE == 2
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bx[e][i] = s * 32 + 4 * ((tid + e * NT) % 8) + i < K ? bx[e][i] : 0.0f;
+#elif MODE == 0
+            const int u = (tid + e * NT) / 16 % 8;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < NV; ++j) bx[e][i][j] = s * 32 + 4 * (u >> 1) + 16 * (u & 1) + i < K ? bx[e][i][j] : 0.0f;
+#else
+#pragma unroll
+            for (int i = 0; i < 8; ++i) bx[e][i] = s < STEPS ? bx[e][i] : 0.0f;
+#endif
+        }
+    };
+
+    float a_max[EA], b_max[EB];         /* the largest number of what a task loads, all steps */
+#pragma unroll
+    for (int e = 0; e < EA; ++e) a_max[e] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < EB; ++e) b_max[e] = 0.0f;
+    /* two neighbours along k -> their three parts */
+    auto split2 = [&](float x, float y, unsigned (&p)[3], float& largest) {
+        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(x), "v"(y));
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+            const f32x2 t = {x, y};
+            const bf16x2 r = __builtin_convertvector(t, bf16x2);
+            p[part] = __builtin_bit_cast(unsigned, r);
+            if (part < 2) {
+                x -= __builtin_bit_cast(float, p[part] << 16);
+                y -= __builtin_bit_cast(float, p[part] & 0xffff0000u);
+            }
+        }
+    };
+    auto stage = [&](int s, int buf, int set) {
+        auto& ax = axs[set];
+        auto& bx = bxs[set];
+        unsigned char* const at = lds + buf * TILE_BYTES;
+        unsigned char* const bt = at + 3 * PLANE_A;
+#pragma unroll
+        for (int e = 0; e < EA; ++e) {
+            unsigned p0[3], p1[3];
+            split2(ax[e][0], ax[e][1], p0, a_max[e]);
+            split2(ax[e][2], ax[e][3], p1, a_max[e]);
+            if (BM * 8 % NT == 0 || tid + e * NT < BM * 8)
+#pragma unroll
+                for (int part = 0; part < 3; ++part) {
+                    const u32x2 q = {p0[part], p1[part]};
+                    *reinterpret_cast<u32x2*>(at + part * PLANE_A + a_lds[e]) = q;
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < EB; ++e) {
+#if MODE == 2
+            unsigned p0[3], p1[3];
+            split2(bx[e][0], bx[e][1], p0, b_max[e]);
+            split2(bx[e][2], bx[e][3], p1, b_max[e]);
+            if (BN * 8 % NT == 0 || tid + e * NT < BN * 8)
+#pragma unroll
+                for (int part = 0; part < 3; ++part) {
+                    const u32x2 q = {p0[part], p1[part]};
+                    *reinterpret_cast<u32x2*>(bt + part * PLANE_B + b_lds[e]) = q;
+                }
+#elif MODE == 0
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                unsigned p0[3], p1[3];
+                split2(bx[e][0][j], bx[e][1][j], p0, b_max[e]);
+                split2(bx[e][2][j], bx[e][3][j], p1, b_max[e]);
+                if (BN / NV * 8 % NT == 0 || tid + e * NT < BN / NV * 8)
+#pragma unroll
+                    for (int part = 0; part < 3; ++part) {
+                        const u32x2 q = {p0[part], p1[part]};
+                        *reinterpret_cast<u32x2*>(bt + part * PLANE_B + j * 1024 + (b_lds[e])) = q;
+                    }
+            }
+#else
+            u32x4 q[3];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                unsigned p[3];
+                split2(bx[e][2 * i], bx[e][2 * i + 1], p, b_max[e]);
+#pragma unroll
+                for (int part = 0; part < 3; ++part) q[part][i] = p[part];
+            }
+            if (BN * 4 % NT == 0 || tid + e * NT < BN * 4)
+#pragma unroll
+                for (int part = 0; part < 3; ++part) *reinterpret_cast<u32x4*>(bt + part * PLANE_B + b_lds[e]) = q[part];
+#endif
+        }
+    };
+
+    acc_t acc[REP_M][REP_N], low[REP_M][REP_N];
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < REP_M; ++i)
+#pragma unroll
+            for (int j = 0; j < REP_N; ++j) acc[i][j] = low[i][j] = (acc_t)(0.0f);
+    };
+    clear();
+
+    /* ---- fragments: lane (li, lg) reads chunk lg (MFMA 16), 2 t + lg (MFMA 32) of its row ------------------- */
+    const int a_row = wm * REP_M * MFMA + li, b_row = wn * REP_N * MFMA + li;
+    unsigned a_frag[KH], b_frag[KH];
+#pragma unroll
+    for (int t = 0; t < KH; ++t) {
+        a_frag[t] = (unsigned)(a_row * 64 + ((t * KL + lg) ^ CHUNK_XOR(a_row)) * 16);
+        b_frag[t] = (unsigned)(b_row * 64 + ((t * KL + lg) ^ CHUNK_XOR(b_row)) * 16);
+    }
+    auto multiply = [&](int buf) {
+        const unsigned char* const at = lds + buf * TILE_BYTES;
+        const unsigned char* const bt = at + 3 * PLANE_A;
+#pragma unroll
+        for (int t = 0; t < KH; ++t) {
+            bf16x8 b[REP_N][3];
+#pragma unroll
+            for (int j = 0; j < REP_N; ++j)
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    b[j][p] = *reinterpret_cast<const bf16x8*>(bt + p * PLANE_B + j * MFMA * 64 + (b_frag[t]));
+#pragma unroll
+            for (int i = 0; i < REP_M; ++i) {
+                bf16x8 a[3];
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    a[p] = *reinterpret_cast<const bf16x8*>(at + p * PLANE_A + i * MFMA * 64 + (a_frag[t]));
+                const int pa[5] = {2, 0, 1, 1, 0}, pb[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+                for (int q = 0; q < 5; ++q)
+#pragma unroll
+                    for (int j = 0; j < REP_N; ++j) low[i][j] = SPLIT_OP(a[pa[q]], b[j][pb[q]], low[i][j]);
+#pragma unroll
+                for (int j = 0; j < REP_N; ++j) acc[i][j] = SPLIT_OP(a[0], b[j][0], acc[i][j]);
+            }
+        }
+    };
+
+    /* ---- main loop: step s is multiplied from one buffer while step s + 1 goes from registers to the other --------- */
+    const int first = kg * GSTEPS;
+    if (threadIdx.x == 0) redo = 0;
+#pragma unroll
+    for (int p = 0; p < PD; ++p) load(first + p, p);
+    if ((first + 1) * 32 > K) cut(first, 0);
+    stage(first, 0, 0);
+    load(first + PD, 0);
+    __syncthreads();
+    for (int s0 = 0; s0 + 1 < GSTEPS; s0 += PD) {
+#pragma unroll
+        for (int u = 0; u < PD; ++u) {
+            const int s = s0 + u;
+            if (s + 1 >= GSTEPS) break;
+            const int set = (u + 1) % PD;
+            if ((first + s + 2) * 32 > K) cut(first + s + 1, set);
+            multiply(s & 1);
+            stage(first + s + 1, (s + 1) & 1, set);
+            load(first + s + 1 + PD, set);
+            __syncthreads();
+        }
+    }
+    multiply((GSTEPS - 1) & 1);
+    /* the distance an MFMA's result registers need, made explicit (see above) */
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        bool again = false;
+        float nan = 0.0f;
+#pragma unroll
+        for (int e = 0; e < EA; ++e) again |= (a_max[e] < 0x1p-100f) & (a_max[e] > 0.0f);
+#pragma unroll
+        for (int e = 0; e < EB; ++e) again |= (b_max[e] < 0x1p-100f) & (b_max[e] > 0.0f);
+#pragma unroll
+        for (int i = 0; i < REP_M; ++i)
+#pragma unroll
+            for (int j = 0; j < REP_N; ++j)
+#pragma unroll
+                for (int v = 0; v < NACC; ++v) {
+                    acc[i][j][v] += low[i][j][v];
+                    nan = __builtin_fmaf(acc[i][j][v], 0.0f, nan);
+                }
+        again |= !(nan == 0.0f);
+        if (__any(again) && lane == 0) redo = 1;
+    }
+    __syncthreads();                    /* also the last reads of the tiles, whose LDS the sums take */
+    if (redo) {
+        /* the group's k once more, undivided numbers from memory */
+        clear();
+        const int end = (first + GSTEPS) * 32 < K ? (first + GSTEPS) * 32 : K;
+        int nb[REP_N];
+#if MODE == 1
+        unsigned px[REP_N], bad[REP_N];
+#endif
+#pragma unroll
+        for (int j = 0; j < REP_N; ++j) {
+            nb[j] = n0 + COLUMN((wn * REP_N + j) * MFMA + li);
+#if MODE == 1
+            pixel(nb[j], px[j], bad[j]);
+#endif
+        }
+#pragma unroll 4
+        for (int k0 = first * 32; k0 < end; k0 += KL) {
+            const int k = k0 + lg;
+            float a[REP_M], b[REP_N];
+#pragma unroll
+            for (int i = 0; i < REP_M; ++i) {
+                const int m = m0 + (wm * REP_M + i) * MFMA + li;
+                const unsigned off = (unsigned)((AGROUP(gi) * M + m) * K + k) * 4u;
+                a[i] = ld1(rsrc_a, (m < M) & (k < K) ? off : OOB, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < REP_N; ++j) {
+#if MODE == 1
+                b[j] = ld1(rsrc_b, (px[j] + taps.e[2 * k]) | ((bad[j] << taps.e[2 * k + 1]) & OOB), 0);
+#else
+                const unsigned off = (unsigned)(MODE == 2 ? (gi * N + nb[j]) * K + k : (gi * K + k) * N + nb[j]) * 4u;
+                b[j] = ld1(rsrc_b, (nb[j] < N) & (k < K) ? off : OOB, 0);
+#endif
+            }
+#pragma unroll
+            for (int i = 0; i < REP_M; ++i)
+#pragma unroll
+                for (int j = 0; j < REP_N; ++j) acc[i][j] = MFMA_OP(a[i], b[j], acc[i][j]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+#if WAVES_K > 1
+    /* every group sums and stores a share of each wavefront's blocks */
+#define NOUT ((NBLK + WAVES_K - 1) / WAVES_K)
+    acc_t out[NOUT];
+    {
+        acc_t* const sums = reinterpret_cast<acc_t*>(smem) + wave * (WAVES_K * NBLK * 64);
+#pragma unroll
+        for (int i = 0; i < REP_M; ++i)
+#pragma unroll
+            for (int j = 0; j < REP_N; ++j) sums[(kg * NBLK + i * REP_N + j) * 64 + lane] = acc[i][j];
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NOUT; ++b) {
+            if (NBLK % WAVES_K != 0 && kg * NOUT + b >= NBLK) continue;
+            out[b] = sums[(kg * NOUT + b) * 64 + lane];
+#pragma unroll
+            for (int g = 1; g < WAVES_K; ++g) out[b] += sums[(g * NBLK + kg * NOUT + b) * 64 + lane];
+        }
+    }
+#else
+#define NOUT NBLK
+    acc_t out[NOUT];
+#pragma unroll
+    for (int b = 0; b < NOUT; ++b) out[b] = acc[b / REP_N][b % REP_N];
+#endif
+#pragma unroll
+    for (int b = 0; b < NOUT; ++b) {
+        if (NBLK % WAVES_K != 0 && kg * NOUT + b >= NBLK) continue;
+        const int i = (kg * NOUT + b) / REP_N, j = (kg * NOUT + b) % REP_N;
+        const int n = n0 + COLUMN((wn * REP_N + j) * MFMA + li);
+#if MODE == 1 && !COLOUT
+        float* const col = C + ((size_t)(n / OHW) * (CG * M) + (size_t)gi * M) * OHW + n % OHW;
+        const size_t row = OHW;
+#else
+        float* const col = C + (size_t)gi * M * N + n;
+        const size_t row = N;
+#endif
+#pragma unroll
+        for (int v = 0; v < NACC; ++v) {
+            const int m = m0 + (wm * REP_M + i) * MFMA + (MFMA == 32 ? 8 * (v / 4) : 0) + 4 * lg + v % 4;
+            float val = out[b][v];
+            if ((M % BM == 0 || m < M) & (N % BN == 0 || n < N)) {
+#if HAS_BIAS
+                val += bias[AGROUP(gi) * M + m];
+#endif
+                col[m * row] = val;
+            }
+        }
+    }
+    CLK_END;
+}
+#endif  /* FT_SPLIT */
