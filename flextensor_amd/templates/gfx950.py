@@ -1121,6 +1121,9 @@ def _pick_f32(view, kernels, predict, padded, direct):
             kp = steps * bk * groups
             if kp not in view.KP_options and kp * 4 > view.K * 5:
                 break
+            # its matrix clocks alone are more than the best: not worth a prediction
+            if best is not None and -(-tiles // NUM_CUS) * m[0] * n[0] * groups * m[1] * n[1] * mf * mf * bk * steps > best[0] * 128:
+                continue
             clocks = predict(view, tiles, m, n, mf, bk, depth, groups)
             if clocks is not None and (best is None or clocks < best[0]):
                 best = (clocks, [tm, m[0], m[1], mf], [tn, n[0], n[1], mf], [groups, steps, bk], depth)
@@ -1137,7 +1140,8 @@ def _pick_f32(view, kernels, predict, padded, direct):
                 continue
             for groups in (1, 2, 4, 8):
                 kp = ceil_div(view.K, 32 * groups) * 32 * groups
-                if groups > 1 and tm * tn > 3000 or tm * tn * groups < 128 or kp * 4 > view.K * 5 and kp not in view.KP_options:
+                if groups > 1 and tm * tn > 3000 or tm * tn * groups < 128 \
+                        or -(-tm * tn // NUM_CUS) * groups // 4 * (kp // (32 * groups)) * m * n * 256 > limit or kp * 4 > view.K * 5 and kp not in view.KP_options:
                     continue
                 clocks = _direct_clocks(view, m, n, pd, groups)
                 if clocks < limit:
@@ -1155,36 +1159,45 @@ def _pick_f32(view, kernels, predict, padded, direct):
 # kernels of products in bf16 parts that the defaults choose among: (wavefronts, MFMA tiles per wavefront) along M and N,
 # MFMA edge, K groups, pipeline depth; and 32x32 MFMA tiles along M and N of a wavefront on its own, K groups
 SPLIT_KERNELS = (((2, 2), (4, 1), 32, 1, 9), ((4, 1), (2, 1), 32, 1, 9), ((4, 1), (2, 1), 32, 2, 9), ((2, 2), (4, 1), 16, 1, 9),
-                 ((2, 2), (4, 1), 16, 2, 9), ((2, 2), (4, 1), 16, 2, 10), ((2, 1), (4, 1), 16, 1, 9))
+                 ((2, 2), (4, 1), 16, 2, 10), ((2, 1), (4, 1), 16, 1, 9))
 ALONE_KERNELS = ((2, 2, 8), (2, 2, 4), (2, 1, 8), (1, 1, 8), (1, 1, 4))
+
+
+def _split_step(m, n, mf, groups):
+    """What the step of such a kernel costs one unit whatever the operator: tile, wavefronts, instructions of a thread for
+    its share of the tile's elements and of the gathered ones, of the MFMAs (one keeps the others out for 8 clocks, 10 the
+    large one, another instruction for 4), LDS (six bytes an element in at 70 bytes a clock, out at 230), and the bytes of
+    LDS."""
+    (wm, rm), (wn, rn) = m, n
+    bm, bn, waves = wm * rm * mf, wn * rn * mf, wm * wn
+    return (bm, bn, waves * groups, (bm + bn) * 3.0 / waves, bn * 1.0 / waves, 6 * rm * rn * (20 if mf == 32 else 8),
+            groups * ((bm + bn) * 192 / 70.0 + waves * (rm + rn) * mf * 192 / 230.0), groups * 384 * (bm + bn) + 16)
+
+
+SPLIT_STEPS = {k[:4]: _split_step(*k[:4]) for k in SPLIT_KERNELS}
 
 
 def _split_clocks(view, m, n, mf, groups):
     """Predicted clocks (2.38 GHz) of a call of the split kernel of igemm_f32.hip; see _or_split."""
-    (wm, rm), (wn, rn) = m, n
-    bm, bn = wm * rm * mf, wn * rn * mf
-    conv, waves = view.conv is not None, wm * wn * groups
-    tiles = ceil_div(view.M, bm) * ceil_div(view.N, bn) * view.groups
-    share, steps = ceil_div(tiles, NUM_CUS), ceil_div(ceil_div(view.K, 32), groups)
-    turns = ceil_div(share, max(1, min(share, LDS_BYTES // (groups * 384 * (bm + bn) + 16), 32 // waves)))
-    # a step of all groups on one unit: instructions (an MFMA keeps the others out for 8 clocks, 10 the large one, another
-    # for 4), LDS (six bytes an element in at 70 bytes a clock, out at 230), loads (rows of whole lines by the kilobyte, a
-    # vector less where rows are no whole ones; the gathered operand by 64 elements)
-    elements = (bm + bn) * 32 / (wm * wn * 64.0)
-    vector = elements * 6 + (bn * 64 / (wm * wn * 64.0) if conv else 0)
-    issue = waves * (6 * rm * rn * (20 if mf == 32 else 8) + 4 * (vector + 1)) / 4
-    lds = groups * ((bm + bn) * 192 / 70.0 + wm * wn * (rm + rn) * mf * 192 / 230.0) * (0.97 if conv else 0.86)
-    loads = groups * bm * 0.125 * 28 * (1.3 if view.K % 4 else 1)
-    if conv:
-        loads += groups * bn * 0.5 * 11.1 * (1.67 if view.conv["CSTRW"] > 1 else 1)
-        latency, start, mix, store, sums, launch = 529 + 478 + 17.2 * waves, 434 + 876, 0.518, 6.45, 139, 4110
+    bm, bn, waves, share_ab, share_b, matrix, lds, lds_bytes = SPLIT_STEPS[m, n, mf, groups]
+    share = -(-(-(-view.M // bm) * -(-view.N // bn) * view.groups) // NUM_CUS)
+    steps = -(-view.K // (32 * groups))
+    turns = -(-share // max(1, min(share, LDS_BYTES // lds_bytes, 32 // waves)))
+    # rows of whole lines by the kilobyte, a vector less where rows are no whole ones; the gathered operand by 64 elements
+    loads = groups * bm * (4.55 if view.K % 4 else 3.5)
+    if view.conv:
+        vector = share_ab + share_b
+        loads += groups * bn * (9.27 if view.conv["CSTRW"] > 1 else 5.55)
+        latency, start, mix, store, sums, launch, lds = 1007 + 17.2 * waves, 1310, 0.518, 6.45, 139, 4110, 0.97 * lds
     else:
-        loads += groups * bn * 0.125 * 5.15 * (1.3 if (view.K if view.mode == 2 else view.N) % 4 else 1)
-        latency, start, mix, store, sums, launch = 616 + 4.8 * waves, 412, 0.467, 6.93, 134, 3780
+        vector = share_ab
+        loads += groups * bn * (0.84 if (view.K if view.mode == 2 else view.N) % 4 else 0.64)
+        latency, start, mix, store, sums, launch, lds = 616 + 4.8 * waves, 412, 0.467, 6.93, 134, 3780, 0.86 * lds
+    issue = waves * (matrix + 4 * (vector + 1)) / 4
     longest = max(issue, lds, loads)
     work = longest + mix * (issue + lds + loads - longest)
     return (max(share * steps * work, turns * steps * (latency + 0.6 * work)) + turns * start + share * bm * bn * store / 16
-            + sums * bm * bn / 64.0 * (groups - 1) / (wm * wn) + launch)
+            + sums * bm * bn / 64.0 * (groups - 1) * groups / waves + launch)
 
 
 def _alone_clocks(view, rm, rn, groups):
@@ -1227,14 +1240,18 @@ def _or_split(view, cfg, call):
     limit, best = (call - 500) / 1.08, None
     before = cfg["reduce"][0][0]
     for m, n, mf, groups, depth in SPLIT_KERNELS:
-        if m[0] * m[1] * mf >= 2 * max(view.M, 16) or n[0] * n[1] * mf >= 2 * max(view.N, 16) or depth == 10 and view.K < 192:
+        if m[0] * m[1] * mf >= 2 * max(view.M, 16) or n[0] * n[1] * mf >= 2 * max(view.N, 16):
             continue
-        clocks = _split_clocks(view, m, n, mf, groups) * (0.99 if depth == 10 else 1) if view.K >= 64 * groups else limit
+        # launch, chain of steps, and matrix clocks alone: not worth a prediction
+        steps = -(-view.K // (32 * groups))
+        if view.K < 64 * groups or 3780 + steps * 616 > limit or steps * m[0] * n[0] * groups * m[1] * n[1] * mf * mf * 0.09 > limit:
+            continue
+        clocks = _split_clocks(view, m, n, mf, groups)
         if clocks < limit:
             limit, best = clocks, ((m[0], m[1], mf), (n[0], n[1], mf), groups, depth)
     for rm, rn, groups in ALONE_KERNELS:
         if rm * 32 >= 2 * max(view.M, 32) or rn * 32 >= 2 * max(view.N, 32) or view.K < 32 * groups \
-                or rm * rn == 4 and groups < 2 * before:
+                or rm * rn == 4 and groups < 2 * before or 2170 + -(-view.K // (32 * groups)) * 1020 > limit:
             continue
         lds = groups * 8192 * (rm + (rn if view.mode == 2 else 0)) + (ceil_div(view.K, 32) * 256 if view.conv else 0)
         clocks = _alone_clocks(view, rm, rn, groups) if lds <= LDS_BYTES else limit
