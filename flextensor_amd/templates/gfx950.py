@@ -1246,12 +1246,16 @@ def _or_split(view, cfg, call):
         steps = -(-view.K // (32 * groups))
         if view.K < 64 * groups or 3780 + steps * 616 > limit or steps * m[0] * n[0] * groups * m[1] * n[1] * mf * mf * 0.09 > limit:
             continue
+        if groups > 1 and -(-view.M // (m[0] * m[1] * mf)) * -(-view.N // (n[0] * n[1] * mf)) * view.groups > 2 * NUM_CUS:
+            continue                                # not among the timed: K divided where tiles are many
         clocks = _split_clocks(view, m, n, mf, groups)
         if clocks < limit:
             limit, best = clocks, ((m[0], m[1], mf), (n[0], n[1], mf), groups, depth)
     for rm, rn, groups in ALONE_KERNELS:
         if rm * 32 >= 2 * max(view.M, 32) or rn * 32 >= 2 * max(view.N, 32) or view.K < 32 * groups \
                 or rm * rn == 4 and groups < 2 * before or 2170 + -(-view.K // (32 * groups)) * 1020 > limit:
+            continue
+        if groups > 4 and -(-view.M // (32 * rm)) * -(-view.N // (32 * rn)) * view.groups > 4 * NUM_CUS:
             continue
         lds = groups * 8192 * (rm + (rn if view.mode == 2 else 0)) + (ceil_div(view.K, 32) * 256 if view.conv else 0)
         clocks = _alone_clocks(view, rm, rn, groups) if lds <= LDS_BYTES else limit

@@ -1582,9 +1582,12 @@ typedef f32x4 acc_t;
 #define GROUP_BYTES (2 * TILE_BYTES)
 #define SUM_BYTES (WAVES_K > 1 ? WAVES_K * BM * BN * 4 : 0)
 #define SMEM_BYTES (WAVES_K * GROUP_BYTES > SUM_BYTES ? WAVES_K * GROUP_BYTES : SUM_BYTES)
-/* chunk c of a row lies at c ^ CHUNK_XOR(row): 16 lanes that read the chunks of an MFMA's rows, or write the same chunk of
- * 16 rows, are in 16 different groups of four banks (the order in which lanes are served: see SWZ_G above) */
-#define CHUNK_XOR(row) ((((((row) >> 2) ^ ((row) >> 3)) & 1) << 1) | (((row) >> 3) & 1))
+/* chunk c of a row lies at c ^ CHUNK_XOR(row). Reads serve 16 lanes at a time over 64 banks (in the order that SWZ_G above
+ * speaks of), writes 128 bytes of consecutive lanes over 32 banks: the chunks of 16 rows of an MFMA, or the same chunk of
+ * eight rows, or both halves of it of eight rows (the lanes' order of a task of B [K][N]), are apart in either.
+ * SQ_LDS_BANK_CONFLICT is 0 for all modes; with writes taken to see 64 banks as well it was 0.44 of SQ_ACTIVE_INST_LDS
+ * for B [K][N] and the gathered operand (3x3 stride 2 16x128x57x57 -> 256 52.8 us, 51.4 without). */
+#define CHUNK_XOR(row) ((((row) >> 1) & 3) ^ (((row) >> 4) & 1))
 
 /* rows of k-contiguous operands: 16-byte vectors, eight lanes a row */
 #define EA ((BM * 8 + NT - 1) / NT)
@@ -1730,8 +1733,9 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
         b_off[e] = (n < N) & (row < BN) ? off : OOB;
         b_lds[e] = (unsigned)(row * 64 + ((v & 3) ^ CHUNK_XOR(row)) * 16 + (v >> 2) * 8);
 #elif MODE == 0
-        /* 16 lanes of NV columns, by four k: quad u is half (u & 1) of chunk u >> 1 */
-        const int g = q / 16 / 8, u = q / 16 % 8, l = q % 16, c0 = g * 16 * NV;
+        /* 16 lanes of NV columns, by four k: quad u is half (u & 1) of chunk u >> 1. Eight lanes, then the halves, then
+         * the other eight columns: see CHUNK_XOR */
+        const int g = q / 128, u = q / 32 % 4 * 2 + q / 8 % 2, l = q / 16 % 2 * 8 + q % 8, c0 = g * 16 * NV;
         const int n = n0 + c0 + NV * l;
         const unsigned off = (unsigned)((gi * K + 4 * (u >> 1) + 16 * (u & 1)) * N + n) * 4u;
         b_off[e] = (n < N) & (c0 < BN) ? off : OOB;
@@ -1814,7 +1818,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #pragma unroll
             for (int i = 0; i < 4; ++i) bx[e][i] = s * 32 + 4 * ((tid + e * NT) % 8) + i < K ? bx[e][i] : 0.0f;
 #elif MODE == 0
-            const int u = (tid + e * NT) / 16 % 8;
+            const int u = (tid + e * NT) / 32 % 4 * 2 + (tid + e * NT) / 8 % 2;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1884,7 +1888,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #pragma unroll
                     for (int part = 0; part < 3; ++part) {
                         const u32x2 q = {p0[part], p1[part]};
-                        *reinterpret_cast<u32x2*>(bt + part * PLANE_B + j * 1024 + (b_lds[e])) = q;
+                        *reinterpret_cast<u32x2*>(bt + part * PLANE_B + j * 1024 + (b_lds[e] ^ (j & 1) * 16)) = q;
                     }
             }
 #else
@@ -1930,13 +1934,13 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
             for (int j = 0; j < REP_N; ++j)
 #pragma unroll
                 for (int p = 0; p < 3; ++p)
-                    b[j][p] = *reinterpret_cast<const bf16x8*>(bt + p * PLANE_B + j * MFMA * 64 + (b_frag[t]));
+                    b[j][p] = *reinterpret_cast<const bf16x8*>(bt + p * PLANE_B + j * MFMA * 64 + (b_frag[t] ^ (MFMA == 16 ? (j & 1) * 16 : 0)));
 #pragma unroll
             for (int i = 0; i < REP_M; ++i) {
                 bf16x8 a[3];
 #pragma unroll
                 for (int p = 0; p < 3; ++p)
-                    a[p] = *reinterpret_cast<const bf16x8*>(at + p * PLANE_A + i * MFMA * 64 + (a_frag[t]));
+                    a[p] = *reinterpret_cast<const bf16x8*>(at + p * PLANE_A + i * MFMA * 64 + (a_frag[t] ^ (MFMA == 16 ? (i & 1) * 16 : 0)));
                 const int pa[5] = {2, 0, 1, 1, 0}, pb[5] = {0, 2, 1, 0, 1};
 #pragma unroll
                 for (int q = 0; q < 5; ++q)
