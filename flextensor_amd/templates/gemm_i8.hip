@@ -11,7 +11,7 @@
 //   WAVES_M/N   wavefronts per workgroup along M / N
 //   REP_M/N     MFMA tiles per wavefront along M / N
 //   BK          bytes of K per LDS tile (multiple of the MFMA K)
-//   STAGES      1 or 2 LDS buffers
+//   STAGES      1 or 2 LDS buffers, with DTL 1 also 3
 //   PD          prefetch distance: global loads of tile t+PD are in flight
 //               (in PD register sets) while tile t is multiplied
 //   FRAGPF      1: fragment-prefetch pipeline. Tile t+1 is written to LDS at
@@ -28,7 +28,14 @@
 //   DTL         1: tiles travel global -> LDS directly (buffer loads with the
 //               lds modifier, 16 bytes per lane): no staging registers, no
 //               LDS store instructions; the row swizzle is applied on the
-//               global side, since a wavefront's 64 chunks land contiguously
+//               global side, since a wavefront's 64 chunks land contiguously.
+//               With three buffers two tiles are under way while one is
+//               multiplied, and a step waits for loads that are two steps old.
+//               What bounds a long K on few tiles is that wait: a strip of K is
+//               new to the XCD's L2 in every step, so a step with one tile ahead
+//               lasts as long as a load from behind it (64x64 tiles: 430 ns a
+//               step of 128 with two buffers, 260 with three; 207 tiles at
+//               K = 1900 7.8 -> 5.6 us)
 //               DTL 3: the same data path with the instruction order of the
 //               main loop written out and pinned: the LDS fragment reads of
 //               the next k-step and the direct-to-LDS loads of the tile after
@@ -183,7 +190,7 @@ typedef i32x4 acc_t;
 #define EA ((A_CHUNKS + NT - 1) / NT)
 #define EB ((B_CHUNKS + NT - 1) / NT)
 #if DTL
-#if PAD > 0 || STAGES != 2 || A_CHUNKS % NT != 0 || B_CHUNKS % NT != 0 || K % 16 != 0
+#if PAD > 0 || STAGES < 2 || (STAGES > 2 && DTL != 1) || A_CHUNKS % NT != 0 || B_CHUNKS % NT != 0 || K % 16 != 0
 #error "direct-to-LDS tiles need unpadded rows, two buffers, whole rounds of chunks and K % 16 == 0"
 #endif
 #if DTL == 3 && ((BK / MFMA_K) % 2 != 0 || REP_M * REP_N / 4 + REP_M + REP_N > REP_M * REP_N || REP_M * REP_N / 4 + EA + EB > REP_M * REP_N)
@@ -553,8 +560,16 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
                 dma16(rb, &Bs[buf][(e * NT + wv * 64) * 16], vo, K_AT(k0));
             }
         };
+#if STAGES > 2
+#define AHEAD (STAGES - 2)                     /* tiles under way while the wavefront waits for one */
+        static_assert(AHEAD * (EA + EB) <= 63, "the count of loads under way has six bits");
+#pragma unroll
+        for (int t = 0; t <= AHEAD; ++t)
+            if (t < KT) dma_tile(t, t);
+#else
         dma_tile(0, 0);
-#if DTL != 3
+#endif
+#if DTL != 3 && STAGES == 2
         __builtin_amdgcn_s_waitcnt(0x0F70);     /* vmcnt(0): this wavefront's chunks are in LDS */
         __syncthreads();
 #endif
@@ -719,6 +734,20 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
             }
         }
 #endif
+#elif STAGES > 2
+        int cur = 0, to = STAGES - 1;
+        for (int kt = 0; kt < KT; ++kt) {
+            /* tile kt has landed once the loads of the AHEAD tiles behind it are all that is under way */
+            if (kt + AHEAD < KT)
+                __builtin_amdgcn_s_waitcnt(0x0F70 | ((AHEAD * (EA + EB)) & 15) | (((AHEAD * (EA + EB)) >> 4) << 14));
+            else
+                __builtin_amdgcn_s_waitcnt(0x0F70);
+            __syncthreads();                   /* for everybody, who also has read tile kt - 1: its buffer is free */
+            if (kt + STAGES - 1 < KT) dma_tile(kt + STAGES - 1, to);
+            compute(cur);
+            to = cur;
+            cur = cur + 1 == STAGES ? 0 : cur + 1;
+        }
 #else
         for (int kt = 0; kt < KT; ++kt) {
             const int cur = kt & 1;

@@ -306,6 +306,9 @@ SPECIAL_DEFAULTS = {
 # fp32: 9 and 10 = products in bf16 parts (the second kernel of igemm_f32.hip), one and two k steps ahead; 11 = the same
 # with every wavefront on its own (the second kernel of direct_f32.hip)
 SPLIT_DEPTHS = {9: ("igemm_f32.hip", 1), 10: ("igemm_f32.hip", 2), 11: ("direct_f32.hip", 0)}
+# int8: 9 = 6 with three LDS buffers (two tiles requested ahead). Four and six were timed beside it on 38 sizes: 1.02
+# and 1.12 times its time in the geometric mean, so there are no depths for them.
+I8_BUFFERS = {9: 3}
 PIPELINE = {1: (1, 1), 2: (2, 1), 3: (2, 2), 4: (2, 3), 5: (2, 1), 6: (2, 1), 7: (2, 1), 8: (2, 1)}
 
 
@@ -365,9 +368,10 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
     splitk, kiters, bk = [int(x) for x in rd[0]]
     depth = int((config.get("unroll") or [[2, 1]])[0][0])
     split = view.dtype != "int8" and depth in SPLIT_DEPTHS
-    if depth not in PIPELINE and not split:
+    buffers = I8_BUFFERS.get(depth, 0) if view.dtype == "int8" else 0
+    if depth not in PIPELINE and not split and not buffers:
         raise InvalidConfig("pipeline depth %d is not available" % depth)
-    stages, pd = PIPELINE.get(depth, (2, 1))
+    stages, pd = PIPELINE.get(depth, (buffers or 2, 1))
     if view.dtype != "int8" and depth in (6, 7):
         stages = depth - 3        # fp32: 6 and 7 = tiles straight into LDS with three and four buffers
     # fp32 depth 8: as 5 (two buffers), and the first operands of the next tile are read from LDS
@@ -455,7 +459,7 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
                                 "and an undivided K")
         D.update(PAD=pad, PD=pd, FRAGPF=1 if depth == 5 else 0, NT_STORE=store_mode & 1)
         if depth >= 6:
-            D.update(DTL=depth - 5)
+            D.update(DTL=1 if buffers else depth - 5)
         if store_mode & 2:
             D.update(CVEC=1)
         if store_mode & 4:
@@ -919,7 +923,7 @@ def _empty_config():
 
 
 # tiles of the int8 default: (wavefronts, MFMA tiles per wavefront) along M and along N, 16x16x64 MFMAs
-I8_TILES = (((2, 1), (2, 1)), ((2, 1), (2, 2)), ((2, 2), (2, 2)), ((2, 2), (4, 2)), ((4, 2), (2, 4)),
+I8_TILES = (((2, 1), (2, 1)), ((2, 1), (2, 2)), ((4, 1), (2, 2)), ((2, 2), (4, 2)), ((4, 2), (2, 4)),
             ((4, 4), (4, 4)), ((1, 1), (4, 1)))
 
 
@@ -934,9 +938,9 @@ def _default_i8(view, padded=False):
     faster than its chain of k steps (230 clocks each, a barrier and an LDS round trip) behind the 1750
     clocks until the first operands are there, and only as many tiles run side by side as the LDS holds. The
     factors were fitted to 1 230 timings over 48 sizes (64 .. 4096 an axis, half of them no multiples
-    of 16): what the rule picks is within 6 % of the best of all candidates in the geometric mean, and 1.28
-    times as fast as the rule before it (square-ish power-of-two tiles until every compute unit has one, K tiles of
-    64 through registers): 64x3632x1376 12.0 -> 4.8 us, 1712x1584x2080 21.3 -> 13.6, 3488x176x80 4.2 -> 2.6.
+    of 16) of the kernels with two LDS buffers, among whose candidates the rule's pick was within 6 % of the best in
+    the geometric mean: 64x3632x1376 4.8 us, 1712x1584x2080 13.6, 3488x176x80 2.6. With the third buffer and eight
+    wavefronts on 64x64 tiles it is within 3.8 % of the best of 895 timings over 52 further sizes.
     """
     aligned = view.K % 16 == 0 and not padded        # tiles straight into LDS
     best = None
@@ -949,30 +953,45 @@ def _default_i8(view, padded=False):
         n = ceil_div(tiles, NUM_CUS)
         for bk in (128, 256):
             for groups in (1, 2, 4):
-                if groups > 1 and (tiles > 300 or view.K < bk * groups) or groups * wm * wn > 16:
+                # K of 64x64 tiles divided: 27 of 29 sizes 1.04 .. 1.29 times slower, the others have better tiles
+                if groups > 1 and (tiles > 300 or view.K < bk * groups or bm == bn == 64) or groups * wm * wn > 16:
                     continue
+                steps = ceil_div(view.K, bk * groups)
+                if bm == bn == 64 and steps < 3 and n > 1:
+                    wm, rm, wn, rn = 2, 2, 2, 2                # 297 .. 817 tiles: eight wavefronts 2 .. 7 % slower
                 lds = groups * 2 * (bm + bn) * bk
+                # A third LDS buffer: a tile's loads have two steps to land instead of one, which is what a step waits
+                # for when its operands are not in the L2 yet (144 tiles of 64x64 at K = 3808: 15.8 -> 9.8 us; 216 of
+                # 32x64 at K = 3536: 12.8 -> 8.3). Not where it leaves a compute unit with one workgroup at a time
+                # out of several (425 tiles of 128x128 at 10 steps: 15.7 -> 17.3).
+                third = aligned and steps > 2 and lds * 3 // 2 * min(n, 2) <= LDS_BYTES
+                if third:
+                    lds = lds * 3 // 2
                 if lds > LDS_BYTES or (aligned and ((bm * bk // 16) % (wm * wn * 64) or (bn * bk // 16) % (wm * wn * 64))):
                     continue
                 if not aligned and (ceil_div(bm * bk // 16, wm * wn * 64) + ceil_div(bn * bk // 16, wm * wn * 64)) * 8 > 160:
                     continue          # staging registers
-                steps = ceil_div(view.K, bk * groups)
                 mfma = bm * bn * 2 * 1.12 / 8192.0
-                lds_rw = (wm * wn * (rm + rn) * 16 + (bm + bn) * (0.7 if aligned else 3.7)) * 0.96 / 128.0
+                reads = 16 if bm == bn == 64 else wm * wn * (rm + rn)      # eight wavefronts of 64x64 hide what they read more
+                lds_rw = (reads * 16 + (bm + bn) * (0.7 if aligned else 3.7)) * 0.96 / 128.0
                 l2 = (bm + bn) * 0.68 / 64.0
                 work = n * steps * bk * groups * (max(mfma, lds_rw, l2) + 0.23 * (mfma + lds_rw + l2))
                 beside = max(1, min(LDS_BYTES // lds, 32 // (wm * wn * groups), n))
                 chain = ceil_div(n, beside) * (steps * 230 + 1750 + (220 * rm * rn * (groups - 1)))
                 clocks = max(work, chain) + n * bm * bn * 4 * 2.3 / 64.0
                 if best is None or clocks < best[0]:
-                    best = (clocks, [tm, wm, rm, 16], [tn, wn, rn, 16], [groups, steps, bk])
+                    best = (clocks, [tm, wm, rm, 16], [tn, wn, rn, 16], [groups, steps, bk], third)
     cfg = _empty_config()
-    _, tile_m, tile_n, reduce = best
+    _, tile_m, tile_n, reduce, third = best
     cfg["spatial"] = [tile_m, tile_n]
     cfg["reduce"] = [reduce]
-    # straight into LDS where rows are 16-byte aligned; otherwise two tiles ahead in registers where the tile is
-    # large (2999x4001x1500 49.0 us against 54.6 with the fragment prefetch), fragment prefetch where it is small
-    cfg["unroll"] = [[6 if aligned else (3 if tile_m[1] * tile_m[2] * tile_n[1] * tile_n[2] >= 64 else 5), 1]]
+    # Straight into LDS where rows are 16-byte aligned. Otherwise two tiles ahead in registers (164 tiles of 64x64 at
+    # K = 2050 8.0 -> 7.1 us against the fragment prefetch, 180 of 64x128 15.7 -> 11.5), for tiles of 32x32 from eight
+    # steps on (72 at K = 2800: 5.70 -> 5.32; fewer steps: the same), but not for those of 32x64 (188 at K = 2524:
+    # 4.97 against 5.69).
+    size = tile_m[1] * tile_m[2] * tile_n[1] * tile_n[2]
+    ahead = size >= 16 or (size == 4 and reduce[1] >= 8)
+    cfg["unroll"] = [[(9 if third else 6) if aligned else (3 if ahead else 5), 1]]
     cfg["fuse"] = [[4]]
     cfg["reorder"] = [[1, 1 if reduce[0] > 1 else 0, 0]]
     return cfg
