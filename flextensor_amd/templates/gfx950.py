@@ -231,7 +231,7 @@ def _gemm_space(view):
     if rs.size == 0:
         raise InvalidConfig("K=%d has no admissible LDS tile extent" % view.K)
     space.add_subspace("split_k_0", rs, "reduce")
-    space.add_subspace("unroll", UnrollSpace([1, 2, 3, 4, 5, 6, 7, 8], explicit=True,
+    space.add_subspace("unroll", UnrollSpace([1, 2, 3, 4, 5, 6, 7, 8] + list(I8_BUFFERS if i8 else ()), explicit=True,
                                                extra=() if i8 else [[8, 2], [8, 4], [8, 6], [8, 8]]),
                        "unroll")
     space.add_subspace("group_m", EnumSpace([[1], [2], [4], [8], [16]]), "fuse")
