@@ -426,10 +426,11 @@ def _lower_gemm(op, config, special, out_name, in_names, materialized_pad=False,
         mfma_k = 32 if mfm == 32 else 64
         if bk % mfma_k != 0:
             raise InvalidConfig("BK must be a multiple of the MFMA K extent")
-        if view.K % 16 != 0 and depth >= 6:
+        if depth >= 6 and view.K % (4 if buffers else 16) != 0:
             # a row's last chunk runs into the next row, and for K % 4 != 0 every chunk is cut out of five
-            # dwords: both happen in registers, which the loads that write LDS directly pass by
-            raise InvalidConfig("int8 tiles straight into LDS need K to be a multiple of 16")
+            # dwords: both happen in registers, which the loads that write LDS directly pass by (three buffers:
+            # a row's end is cut out of the fragments)
+            raise InvalidConfig("int8 tiles straight into LDS need K to be a multiple of 16, of 4 with three buffers")
         pad = int(_special(special, "lds_pad")[0])
         pad = -1 if pad < 0 else pad * 4
         if pad >= 0 and pad % 16 != 0:
@@ -943,6 +944,7 @@ def _default_i8(view, padded=False):
     wavefronts on 64x64 tiles it is within 3.8 % of the best of 895 timings over 52 further sizes.
     """
     aligned = view.K % 16 == 0 and not padded        # tiles straight into LDS
+    dwords = view.K % 4 == 0 and not padded          # into three buffers of it
     best = None
     for (wm, rm), (wn, rn) in I8_TILES:
         bm, bn = wm * rm * 16, wn * rn * 16
@@ -964,12 +966,14 @@ def _default_i8(view, padded=False):
                 # for when its operands are not in the L2 yet (144 tiles of 64x64 at K = 3808: 15.8 -> 9.8 us; 216 of
                 # 32x64 at K = 3536: 12.8 -> 8.3). Not where it leaves a compute unit with one workgroup at a time
                 # out of several (425 tiles of 128x128 at 10 steps: 15.7 -> 17.3).
-                third = aligned and steps > 2 and lds * 3 // 2 * min(n, 2) <= LDS_BYTES
+                third = dwords and steps > 2 and lds * 3 // 2 * min(n, 2) <= LDS_BYTES
                 if third:
                     lds = lds * 3 // 2
-                if lds > LDS_BYTES or (aligned and ((bm * bk // 16) % (wm * wn * 64) or (bn * bk // 16) % (wm * wn * 64))):
+                if lds > LDS_BYTES or ((aligned or third) and ((bm * bk // 16) % (wm * wn * 64)
+                                                               or (bn * bk // 16) % (wm * wn * 64))):
                     continue
-                if not aligned and (ceil_div(bm * bk // 16, wm * wn * 64) + ceil_div(bn * bk // 16, wm * wn * 64)) * 8 > 160:
+                if not (aligned or third) and (ceil_div(bm * bk // 16, wm * wn * 64)
+                                               + ceil_div(bn * bk // 16, wm * wn * 64)) * 8 > 160:
                     continue          # staging registers
                 mfma = bm * bn * 2 * 1.12 / 8192.0
                 reads = 16 if bm == bn == 64 else wm * wn * (rm + rn)      # eight wavefronts of 64x64 hide what they read more
@@ -985,13 +989,14 @@ def _default_i8(view, padded=False):
     _, tile_m, tile_n, reduce, third = best
     cfg["spatial"] = [tile_m, tile_n]
     cfg["reduce"] = [reduce]
-    # Straight into LDS where rows are 16-byte aligned. Otherwise two tiles ahead in registers (164 tiles of 64x64 at
+    # Straight into LDS where rows are 16-byte aligned, with three buffers where they are whole dwords (1063x1844x486
+    # 5.78 -> 4.69 us, 318x3700x534 5.56 -> 4.94). Otherwise two tiles ahead in registers (164 tiles of 64x64 at
     # K = 2050 8.0 -> 7.1 us against the fragment prefetch, 180 of 64x128 15.7 -> 11.5), for tiles of 32x32 from eight
     # steps on (72 at K = 2800: 5.70 -> 5.32; fewer steps: the same), but not for those of 32x64 (188 at K = 2524:
     # 4.97 against 5.69).
     size = tile_m[1] * tile_m[2] * tile_n[1] * tile_n[2]
     ahead = size >= 16 or (size == 4 and reduce[1] >= 8)
-    cfg["unroll"] = [[(9 if third else 6) if aligned else (3 if ahead else 5), 1]]
+    cfg["unroll"] = [[9 if third else 6 if aligned else 3 if ahead else 5, 1]]
     cfg["fuse"] = [[4]]
     cfg["reorder"] = [[1, 1 if reduce[0] > 1 else 0, 0]]
     return cfg

@@ -5,7 +5,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def run(m, k, n, tile_m, tile_n, bk, depth, parts=1, in_wg=1):
+def run(m, k, n, tile_m, tile_n, bk, depth, parts=1, in_wg=1, shift=0):
     import torch
     from flextensor_amd import nn
     from flextensor_amd.plan import build
@@ -25,7 +25,13 @@ def run(m, k, n, tile_m, tile_n, bk, depth, parts=1, in_wg=1):
     x, y = [rng.integers(-128, 128, shape, dtype=np.int8) for shape in ((m, k), (n, k))]
     func = build(plan, bufs, "rocm")
     out = torch.full((m, n), -77, dtype=torch.int32, device="cuda")
-    func(torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda(), out)
+
+    def at(host, byte):
+        """The operand ``byte`` bytes into an allocation, with ones around it."""
+        room = torch.ones(host.size + 64, dtype=torch.int8, device="cuda")
+        room[byte:byte + host.size] = torch.from_numpy(host).cuda().reshape(-1)
+        return room[byte:byte + host.size].reshape(host.shape)
+    func(at(x, shift), at(y, 3 * shift), out)
     torch.cuda.synchronize()
     func.close()
     # |sums| <= 4096 * 2^14 < 2^53: exact in float64
@@ -43,6 +49,21 @@ def test_three_buffers(tile_m, tile_n, bk, parts, in_wg, steps):
     assert plan.specs[-1].defines["STAGES"] == 3 and plan.specs[-1].defines["DTL"] == 1
 
 
+@pytest.mark.parametrize("tile_m,tile_n,bk", [((2, 1), (2, 1), 128), ((2, 1), (2, 1), 256), ((2, 1), (2, 2), 128), ((1, 1), (4, 1), 256),
+                                              ((4, 1), (2, 2), 128), ((2, 2), (4, 2), 128), ((4, 2), (2, 4), 128)])
+@pytest.mark.parametrize("k,shift", [(124, 0), (260, 4), (380, 0), (388, 8), (516, 12), (1276, 4)])
+def test_rows_of_whole_dwords_in_three_buffers(tile_m, tile_n, bk, k, shift):
+    """K ends after one, two or three dwords of a chunk; operands begin at any dword."""
+    m, n = tile_m[0] * tile_m[1] * 32 - 3, tile_n[0] * tile_n[1] * 16 + 5
+    assert run(m, k, n, tile_m, tile_n, bk, 9, shift=shift).specs[-1].defines["STAGES"] == 3
+
+
+@pytest.mark.parametrize("k", [516, 900, 1276])
+@pytest.mark.parametrize("in_wg", [0, 1])
+def test_rows_of_whole_dwords_with_k_divided(k, in_wg):
+    run(61, k, 69, (2, 1), (2, 1), 128, 9, 2, in_wg)
+
+
 @pytest.mark.parametrize("k", [1, 127, 129, 258, 1531])
 @pytest.mark.parametrize("depth", [3, 4])
 def test_eight_wavefronts_through_registers(k, depth):
@@ -58,4 +79,4 @@ def test_default_takes_the_third_buffer():
     def depth(m, k, n):
         a, b = placeholder((m, k), dtype="int8"), placeholder((n, k), dtype="int8")
         return gfx950.untuned_config(nn.gemm_int8(a, b).op)["unroll"][0][0]
-    assert depth(1152, 3808, 512) == 9 and depth(1152, 112, 512) == 6 and depth(1152, 3801, 512) == 3
+    assert depth(1152, 3808, 512) == 9 and depth(1152, 3804, 512) == 9 and depth(1152, 112, 512) == 6 and depth(1152, 3801, 512) == 3
