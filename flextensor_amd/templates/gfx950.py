@@ -992,11 +992,15 @@ def _default_i8(view, padded=False):
     # Straight into LDS where rows are 16-byte aligned, with three buffers where they are whole dwords (1063x1844x486
     # 5.78 -> 4.69 us, 318x3700x534 5.56 -> 4.94). Otherwise two tiles ahead in registers (164 tiles of 64x64 at
     # K = 2050 8.0 -> 7.1 us against the fragment prefetch, 180 of 64x128 15.7 -> 11.5), for tiles of 32x32 from eight
-    # steps on (72 at K = 2800: 5.70 -> 5.32; fewer steps: the same), but not for those of 32x64 (188 at K = 2524:
-    # 4.97 against 5.69).
+    # steps on (72 at K = 2800: 5.70 -> 5.32; fewer steps: the same). Those of 32x64 keep the prefetch (188 at K = 2524:
+    # 4.97 against 5.69) up to 25 steps; from about there on its steps take 370 ns instead of 250 at most sizes (why is
+    # not known), and three tiles ahead is faster: of 47 sizes at K = 2800 .. 4057 the 14 of up to 25 steps take
+    # 0.77 .. 1.05 of its time, half of them above 1, the 33 of more 0.75 .. 1.05, one above 1.02, 0.80 in the geometric
+    # mean (1251x4045x361 14.1 -> 10.5 us).
     size = tile_m[1] * tile_m[2] * tile_n[1] * tile_n[2]
     ahead = size >= 16 or (size == 4 and reduce[1] >= 8)
-    cfg["unroll"] = [[9 if third else 6 if aligned else 3 if ahead else 5, 1]]
+    long = size == 8 and reduce[1] > 25
+    cfg["unroll"] = [[9 if third else 6 if aligned else 3 if ahead else 4 if long else 5, 1]]
     cfg["fuse"] = [[4]]
     cfg["reorder"] = [[1, 1 if reduce[0] > 1 else 0, 0]]
     return cfg

@@ -70,6 +70,11 @@ def test_eight_wavefronts_through_registers(k, depth):
     run(70, k, 131, (4, 1), (2, 2), 128, depth)
 
 
+@pytest.mark.parametrize("k", [3329, 3455, 3458])
+def test_small_tiles_three_ahead(k):
+    run(35, k, 131, (2, 1), (2, 2), 128, 4)
+
+
 def test_default_takes_the_third_buffer():
     """Where K is long and a unit holds the larger workgroups; not where they would run one at a time."""
     from flextensor_amd import nn
@@ -80,3 +85,4 @@ def test_default_takes_the_third_buffer():
         a, b = placeholder((m, k), dtype="int8"), placeholder((n, k), dtype="int8")
         return gfx950.untuned_config(nn.gemm_int8(a, b).op)["unroll"][0][0]
     assert depth(1152, 3808, 512) == 9 and depth(1152, 3804, 512) == 9 and depth(1152, 112, 512) == 6 and depth(1152, 3801, 512) == 3
+    assert depth(1251, 4045, 361) == 4 and depth(1086, 2893, 290) == 5
