@@ -185,6 +185,28 @@ def test_k_streaming_arrivals_wait_for_the_slot_stores(tmp_path):
         assert found == [], [(insts[i], insts[j]) for i, j in found[:3]]
 
 
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+@pytest.mark.parametrize("args,tile,groups", [
+    ((5, 32, 3, 3, 17, 3, 1, 0, 1, 1), (1, 1, 1, 3), 4),        # five pixels: two of three blocks of columns behind the last one
+    ((5, 32, 3, 3, 17, 3, 1, 0, 1, 1), (1, 1, 1, 2), 1),
+    ((2, 20, 13, 11, 70, 3, 1, 1, 1, 1), (1, 2, 1, 2), 4), ((2, 64, 14, 14, 70, 1, 2, 0, 1, 1), (1, 1, 1, 1), 1),
+    ((1, 100, 150, 90), (1, 2, 1, 2), 4), ((1, 20, 300, 5), (1, 1, 1, 4), 4)])
+def test_loads_that_a_wait_counts_are_all_there(args, tile, groups):
+    """A wavefront of direct_f32.hip's second kernel waits for its rows in LDS by the number of loads behind them, the
+    second half of a step's B: each step, both times the products can be made, has all of them, none merged with another
+    or dropped because nothing is stored from it."""
+    from test_gpu_direct import conv_of, gemm_of
+    from test_gpu_split import split_plan
+    plan, _ = split_plan(conv_of(False) if len(args) == 10 else gemm_of(False), args, tile, 32, groups, 11)
+    (spec,) = [s for s in plan.specs if s.template == "direct_f32.hip"]
+    loads = 16 if len(args) == 4 else 16 * tile[3]
+    text = isa_hazards.assembly_of(spec)
+    found = [l for l in text.split("\n") if re.match(r"\s+buffer_load_dword", l) and not l.rstrip().endswith(" lds")]
+    waits = re.findall(r"s_waitcnt vmcnt\((\d+)\)", text)
+    assert waits.count(str(loads // 2)) >= 2, waits
+    assert len(found) == 4 * loads, (len(found), loads)         # before the loop and in it, split and whole products
+
+
 MASKED = """k:
 \tv_cmp_ne_u32_e32 vcc, 0, v12
 \tv_mov_b32_e32 v23, 0
