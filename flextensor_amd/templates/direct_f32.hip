@@ -378,14 +378,14 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #else  /* FT_SPLIT */
 /* ============ the same operators on the bf16 matrix cores: FT_SPLIT ================================================
  *
- * Numbers in three bf16 parts, six products, the sums looked at, as the second kernel of igemm_f32.hip explains them; here
+ * Numbers (2^23 times each) in three bf16 parts, six products, the sums looked at, as the second kernel of igemm_f32.hip explains them; here
  * a wavefront works alone: it multiplies REP_M x REP_N blocks of 32 x 32 over its share of K, splits what it needs itself
  * and waits for no barrier before the sum over the groups. Rows of A (and B^T) go through LDS, which is the wavefront's
  * own, because eight lanes a row load at three times the rate of four (44 and 15 bytes a clock and unit) and the loads
  * need no registers on their way; B [K][N] and gathered elements are loaded by the lane that multiplies them, whole lines
  * already. Two steps of A are in LDS or on their way, of B one.
  *
- * What bounds it: twelve vector instructions for two numbers beside an MFMA that hides two for every eight clocks of its
+ * What bounds it: thirteen vector instructions for two numbers beside an MFMA that hides two for every eight clocks of its
  * own, 2 000 clocks a step of 64 x 64 x 32 where the MFMAs are 1 536, and the operands of a 64 x 64 tile, 1 900 clocks from
  * L2. LDS tiles of several wavefronts (igemm_f32.hip) split and gather every element once, this kernel once for each
  * wavefront's tile, but a gathered tile of theirs waits for its slowest wavefront at every barrier: 3x3 8x256x14x14 -> 512
@@ -702,19 +702,11 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #endif
     };
 
-    float a_max[REP_M], b_max[REP_N];
-#pragma unroll
-    for (int i = 0; i < REP_M; ++i) a_max[i] = 0.0f;
-#pragma unroll
-    for (int j = 0; j < REP_N; ++j) b_max[j] = 0.0f;
-    auto split = [&](const float (&x)[8], bf16x8 (&p)[3], float& largest) {
+    auto split = [&](const float (&x)[8], bf16x8 (&p)[3]) {         /* of 2^23 x */
         u32x4 q[3];
         float y[8];
 #pragma unroll
-        for (int h = 0; h < 8; ++h) y[h] = x[h];
-#pragma unroll
-        for (int h = 0; h < 4; ++h)
-            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(y[2 * h]), "v"(y[2 * h + 1]));
+        for (int h = 0; h < 8; ++h) y[h] = x[h] * 0x1p23f;
 #pragma unroll
         for (int part = 0; part < 3; ++part) {
 #pragma unroll
@@ -785,11 +777,11 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
                 } else {
                     bf16x8 a[REP_M][3], b[REP_N][3];
 #pragma unroll
-                    for (int j = 0; j < REP_N; ++j) split(bx[t][j], b[j], b_max[j]);
+                    for (int j = 0; j < REP_N; ++j) split(bx[t][j], b[j]);
                     if (t == 1) load_rows(next, buf ^ 1);
                     load_b(next, t);
 #pragma unroll
-                    for (int i = 0; i < REP_M; ++i) split(ax[i], a[i], a_max[i]);
+                    for (int i = 0; i < REP_M; ++i) split(ax[i], a[i]);
                     const int pa[5] = {2, 0, 1, 1, 0}, pb[5] = {0, 2, 1, 0, 1};
 #pragma unroll
                     for (int q = 0; q < 5; ++q)
@@ -813,12 +805,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
     };
     run(parts());
     {
-        bool again = false;
         float nan = 0.0f;
-#pragma unroll
-        for (int i = 0; i < REP_M; ++i) again |= (a_max[i] < 0x1p-100f) & (a_max[i] > 0.0f);
-#pragma unroll
-        for (int j = 0; j < REP_N; ++j) again |= (b_max[j] < 0x1p-100f) & (b_max[j] > 0.0f);
 #pragma unroll
         for (int i = 0; i < REP_M; ++i)
 #pragma unroll
@@ -828,9 +815,10 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #if LOW
                     acc[i][j][v] += low[i][j][v];
 #endif
+                    acc[i][j][v] *= 0x1p-46f;
                     nan = __builtin_fmaf(acc[i][j][v], 0.0f, nan);
                 }
-        if (__any(again | !(nan == 0.0f))) run(whole());
+        if (__any(!(nan == 0.0f))) run(whole());
     }
 
     /* ---- sum over the k groups and stores: a group takes every WAVES_K-th set of four rows a lane ------------- */

@@ -1458,20 +1458,23 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
 /* ============ the same operators on the bf16 matrix cores: FT_SPLIT ================================================
  *
  * An fp32 number is the sum of three bf16 numbers, x = h + m + l: h is x rounded to bf16, m the remainder rounded, l what
- * then remains (24 bits of significand are three times eight; both subtractions are exact). Of the nine products of the
- * parts the six of up to 2^-18 of the largest are summed by v_mfma_f32_*_bf16 in fp32, the other three are below 2^-26.
+ * then remains (24 bits of significand are three times eight; both subtractions are exact). |m| is up to 2^-8 of |x| and
+ * |l| up to 2^-17. Of the nine products of the parts the six from 2^-17 up are summed by v_mfma_f32_*_bf16 in fp32; ml, lm
+ * and ll are left out: each up to 2^-25 of the product, together up to 2^-24 (2^-27.5 in the root mean square over all
+ * significands), where an fp32 sum is rounded by up to 2^-24 each time.
  * A 16x16x32 bf16 MFMA takes 16 clocks, the eight fp32 MFMAs of the same block 256, so six of them are 2.7 times as fast.
  * The five small products have accumulators of their own, so the large sum is rounded once every 32 (16) k where the fp32
  * MFMA rounds it every four: relative error against float64, fp32 MFMA and this, GEMM 1000x1531x777 7.0e-7 and 1.6e-7,
  * 3x3 16x128x57x57 -> 256 4.2e-7 and 1.5e-7, batch 96 x 197x64x197 1.4e-7 and 0.5e-7.
  *
- * Two kinds of numbers have no such parts: infinities, NaN and what rounds to a bf16 infinity (their remainder is NaN, so
- * a sum is, and every sum is looked at), and those below 2^-110, whose l is smaller than the least bf16 number. A thread
- * keeps the largest of what it loads of a row or column; where that is below 2^-100 and not zero, or a sum is no finite
- * number, the workgroup does its part of K again with fp32 MFMAs, slowly, straight from memory. Otherwise a part that is
- * lost is below 2^-134, which is 2^-34 of the largest.
+ * The parts are those of 2^23 x, which is a multiple of 2^-126 whatever x is, so every part is zero or a normal number and
+ * nothing of a small x is lost, whatever stands beside it; the sums are multiplied by 2^-46 at the end. (Parts of x itself lose bits below
+ * 2^-110. To look for the largest number of a row, an instruction for two numbers less, misses a small one beside it: GEMM
+ * 1024^3 16.75 us and 16.91 with the factor, 1000x1531x777 22.8 and 23.2.) Infinities, NaN and numbers from 2^105 on have no
+ * such parts, their remainder is NaN, and sums from 2^82 on are infinite: every sum is looked at, and where one is no
+ * finite number the workgroup does its part of K again with fp32 MFMAs, slowly, straight from memory.
  *
- * What bounds it: a vector instruction and an MFMA overlap for half of the MFMA's clocks only, the split is twelve
+ * What bounds it: a vector instruction and an MFMA overlap for half of the MFMA's clocks only, the split is thirteen
  * instructions for two numbers, and a wavefront writes LDS at 70 bytes a clock and unit (reads: 230). So operands are
  * split once per workgroup, on the way from memory to LDS: a tile is three planes of bf16, rows of 32 k, read as one
  * 16-byte load per lane, part and block. Rows of A (and B^T) are loaded eight lanes a row, whole cache lines: 16 rows of
@@ -1830,14 +1833,10 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
         }
     };
 
-    float a_max[EA], b_max[EB];         /* the largest number of what a task loads, all steps */
-#pragma unroll
-    for (int e = 0; e < EA; ++e) a_max[e] = 0.0f;
-#pragma unroll
-    for (int e = 0; e < EB; ++e) b_max[e] = 0.0f;
-    /* two neighbours along k -> their three parts */
-    auto split2 = [&](float x, float y, unsigned (&p)[3], float& largest) {
-        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(x), "v"(y));
+    /* two neighbours along k -> the three parts of 2^23 times each */
+    auto split2 = [&](float x, float y, unsigned (&p)[3]) {
+        x *= 0x1p23f;
+        y *= 0x1p23f;
 #pragma unroll
         for (int part = 0; part < 3; ++part) {
             const f32x2 t = {x, y};
@@ -1857,8 +1856,8 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #pragma unroll
         for (int e = 0; e < EA; ++e) {
             unsigned p0[3], p1[3];
-            split2(ax[e][0], ax[e][1], p0, a_max[e]);
-            split2(ax[e][2], ax[e][3], p1, a_max[e]);
+            split2(ax[e][0], ax[e][1], p0);
+            split2(ax[e][2], ax[e][3], p1);
             if (BM * 8 % NT == 0 || tid + e * NT < BM * 8)
 #pragma unroll
                 for (int part = 0; part < 3; ++part) {
@@ -1870,8 +1869,8 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
         for (int e = 0; e < EB; ++e) {
 #if MODE == 2
             unsigned p0[3], p1[3];
-            split2(bx[e][0], bx[e][1], p0, b_max[e]);
-            split2(bx[e][2], bx[e][3], p1, b_max[e]);
+            split2(bx[e][0], bx[e][1], p0);
+            split2(bx[e][2], bx[e][3], p1);
             if (BN * 8 % NT == 0 || tid + e * NT < BN * 8)
 #pragma unroll
                 for (int part = 0; part < 3; ++part) {
@@ -1882,8 +1881,8 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #pragma unroll
             for (int j = 0; j < NV; ++j) {
                 unsigned p0[3], p1[3];
-                split2(bx[e][0][j], bx[e][1][j], p0, b_max[e]);
-                split2(bx[e][2][j], bx[e][3][j], p1, b_max[e]);
+                split2(bx[e][0][j], bx[e][1][j], p0);
+                split2(bx[e][2][j], bx[e][3][j], p1);
                 if (BN / NV * 8 % NT == 0 || tid + e * NT < BN / NV * 8)
 #pragma unroll
                     for (int part = 0; part < 3; ++part) {
@@ -1896,7 +1895,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 unsigned p[3];
-                split2(bx[e][2 * i], bx[e][2 * i + 1], p, b_max[e]);
+                split2(bx[e][2 * i], bx[e][2 * i + 1], p);
 #pragma unroll
                 for (int part = 0; part < 3; ++part) q[part][i] = p[part];
             }
@@ -1980,23 +1979,17 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
     asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     {
-        bool again = false;
         float nan = 0.0f;
-#pragma unroll
-        for (int e = 0; e < EA; ++e) again |= (a_max[e] < 0x1p-100f) & (a_max[e] > 0.0f);
-#pragma unroll
-        for (int e = 0; e < EB; ++e) again |= (b_max[e] < 0x1p-100f) & (b_max[e] > 0.0f);
 #pragma unroll
         for (int i = 0; i < REP_M; ++i)
 #pragma unroll
             for (int j = 0; j < REP_N; ++j)
 #pragma unroll
                 for (int v = 0; v < NACC; ++v) {
-                    acc[i][j][v] += low[i][j][v];
+                    acc[i][j][v] = (acc[i][j][v] + low[i][j][v]) * 0x1p-46f;
                     nan = __builtin_fmaf(acc[i][j][v], 0.0f, nan);
                 }
-        again |= !(nan == 0.0f);
-        if (__any(again) && lane == 0) redo = 1;
+        if (__any(!(nan == 0.0f)) && lane == 0) redo = 1;
     }
     __syncthreads();                    /* also the last reads of the tiles, whose LDS the sums take */
     if (redo) {

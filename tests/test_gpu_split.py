@@ -1,7 +1,7 @@
 """Products in bf16 parts (pipeline depths 9 to 11) at the sizes where their parts have edges, against sums in float64, and
 the numbers that have no such parts.
 
-Bound: a product of two numbers in three parts is off by less than 2^-24 of itself, the large sum is rounded once for every
+Bound: a product of two numbers in three parts is off by up to 2^-24 of itself, the large sum is rounded once for every
 16 or 32 of K (six times for every 16 where a wavefront has four blocks), each time by up to 2^-24 of what it holds;
 for the K of these cases (up to 1023) that is below 1e-5 of the largest result whatever the order."""
 import numpy as np
@@ -84,54 +84,84 @@ def test_image_by_image_and_order_of_the_workgroups(oracle, kernel, xcd):
     assert rel(run(plan, bufs, host), ref) <= TOL
 
 
-NUMBERS = {"small": (1e-34, 1e10), "denormal": (1e-41, 1e38), "large": (7e37, 1e-3), "zero": (0.0, 1.0)}
+# factors of the two operands: numbers of every size that float32 holds, results that no sum of scaled parts holds
+NUMBERS = {"small": (1e-34, 1e10), "denormal": (1e-41, 1e38), "large": (7e37, 1e-3), "large sums": (1e15, 1e15), "zero": (0.0, 1.0)}
+# factors along k of (weights or A, columns of B), and along the columns: an ordinary number hides none that is below 2^-110
+MIXED = {"columns": ((1e20, 1e20), (1.0, 1.0), (1.0, 2.0 ** -120)), "small terms": ((1.0, 2.0 ** -120), (0.0, 2.0 ** 100), (1.0, 1.0)),
+         "terms of two sizes": ((2.0 ** -118, 2.0 ** 60), (2.0 ** 70, 2.0 ** -124), (1.0, 1.0)),
+         "denormal terms": ((2.0 ** 90, 1.0), (2.0 ** -140, 2.0 ** -45), (1.0, 1.0))}
+
+
+def in_turn(factors, count):
+    return np.resize(np.asarray(factors), count)
 
 
 @pytest.mark.parametrize("kernel", [((2, 2, 4, 1), 16, 2, 10), ((2, 1, 2, 1), 32, 1, 9), ((1, 2, 1, 2), 32, 4, 11), ((1, 1, 1, 1), 32, 2, 11)])
-@pytest.mark.parametrize("what", sorted(NUMBERS) + ["infinite", "nan", "scattered"])
+@pytest.mark.parametrize("what", sorted(NUMBERS) + sorted(MIXED) + ["infinite", "nan", "scattered"])
 @pytest.mark.parametrize("func,args", [(gemm_of(False), (1, 100, 150, 90)), (gemm_of(True), (1, 100, 150, 90)),
                                        (conv_of(False), (2, 20, 13, 11, 70, 3, 1, 1, 1, 1))])
 def test_numbers_without_three_parts(func, args, what, kernel):
-    """Operands of one size, at both ends of the range; single infinities and NaNs; rows and columns in which numbers below
-    2^-110 and of 2^100 stand among others. Results that float32 holds are off by no more than they are elsewhere, the
-    others are the infinities and NaNs that the products give."""
+    """Operands of one size, at both ends of the range; ordinary numbers beside those whose low parts bf16 does not hold, in
+    neighbouring columns, along k where the other operand is zero, and scattered; single infinities and NaNs. Every result that float32
+    holds is off by no more than TOL of the sum of its own products' magnitudes, the others are the infinities and NaNs
+    that the products give."""
     import torch
     from flextensor_amd.measure import seeded_inputs
     plan, bufs = split_plan(func, args, *kernel)
-    host = [x * np.float32(1.0) for x in seeded_inputs(bufs, seed=11)]
+    conv, trans_b = len(args) == 10, bool(func(*args)[0][0].attrs.get("transposeB"))
+    host = [x.astype(np.float64) for x in seeded_inputs(bufs, seed=11)]
     if what in NUMBERS:
-        host = [(x.astype(np.float64) * s).astype(np.float32) for x, s in zip(host, NUMBERS[what])]
+        host = [x * s for x, s in zip(host, NUMBERS[what])]
+    elif what in MIXED:
+        fa, fb, fn = MIXED[what]
+        if conv:            # the weights' k are channels, columns are pixels: every other one of a row of the image
+            host[1] *= in_turn(fa, 20)[:, None, None]
+            host[0] *= in_turn(fb, 20)[:, None, None] * in_turn(fn, 11)
+        else:
+            host[0] *= in_turn(fa, 150)
+            host[1] *= (in_turn(fb, 150)[:, None] * in_turn(fn, 90)).T if trans_b else in_turn(fb, 150)[:, None] * in_turn(fn, 90)
     elif what == "scattered":
-        host[0].ravel()[::7] *= np.float32(1e-36)
-        host[1].ravel()[::5] *= np.float32(1e30)
-    else:
+        host[0].ravel()[::7] *= 1e-36
+        host[1].ravel()[::11] *= 1e30           # 11 divides no row: every column has them at k of its own
+    host = [x.astype(np.float32) for x in host]
+    if what in ("infinite", "nan"):
         host[0].ravel()[host[0].size // 2] = np.inf if what == "infinite" else np.nan
     x, y = [torch.from_numpy(h).double() for h in host]
+
+    def product(x, y):
+        if conv:
+            return torch.stack([y.reshape(70, -1) @ c for c in torch.nn.functional.unfold(x, 3, padding=1)]).reshape(bufs[-1].shape).numpy()
+        return (x @ (y.T if trans_b else y)).numpy()
+
     with np.errstate(all="ignore"):
-        if len(args) == 10:
-            cols = torch.nn.functional.unfold(x, 3, padding=1)
-            ref = torch.stack([y.reshape(70, -1) @ c for c in cols]).reshape(bufs[-1].shape).numpy()
-        else:
-            ref = (x @ (y.T if func(*args)[0][0].attrs.get("transposeB") else y)).numpy()
-        held = ref.astype(np.float32).astype(np.float64)
+        held, most = product(x, y).astype(np.float32).astype(np.float64), product(x.abs(), y.abs())
     out = run(plan, bufs, host).astype(np.float64)
     finite = np.isfinite(held)
     assert np.array_equal(out[~finite], held[~finite], equal_nan=True)
-    # rows apart (a row of one operand is of one size): 1e-5 of the row's largest, and the least float32 number
-    axis = 1 if len(args) == 10 else -1
-    d, r = np.abs(np.where(finite, out, 0) - np.where(finite, held, 0)), np.abs(np.where(finite, held, 0))
-    assert np.all(d <= TOL * r.max(axis=axis, keepdims=True) + 2.0 ** -148)
+    # and half of the least float32 number for each group of K that is rounded to one
+    assert np.all(np.abs(out[finite] - held[finite]) <= TOL * most[finite] + 2.0 ** -147)
 
 
-def test_more_exact_than_fp32_products():
-    """K of 2304 undivided: nearer to float64 than the kernels whose products are fp32."""
-    from flextensor_amd.measure import seeded_inputs
-    from test_gpu_grid_order import plan_of
-    shape = (1, 128, 2304, 128)
-    plan, bufs = split_plan(gemm_of(False), shape, (2, 2, 4, 1), 16, 1, 9)
-    other, _, _ = plan_of(gemm_of(False)(*shape), "gemm", 16, 16)
-    a, b = seeded_inputs(bufs, seed=5)
-    ref = a.astype(np.float64) @ b.astype(np.float64)
+@pytest.mark.parametrize("shape,trans_b,kernel", [
+    ((1, 128, 2304, 128), False, ((2, 2, 4, 1), 16, 1, 9)), ((1, 300, 1300, 200), True, ((2, 2, 4, 1), 32, 1, 9)),
+    # four blocks of a wavefront share one set of accumulators: with K divided by at least twice the default's groups
+    ((1, 1000, 1531, 777), False, ((1, 2, 1, 2), 32, 4, 11)), ((1, 700, 2000, 900), True, ((1, 2, 1, 2), 32, 4, 11)),
+    ((1, 1024, 1024, 1024), False, ((1, 2, 1, 2), 32, 8, 11)), ((1, 320, 4096, 520), False, ((1, 1, 1, 2), 32, 8, 11))])
+def test_more_exact_than_fp32_products(shape, trans_b, kernel, monkeypatch):
+    """Nearer to float64 than the kernel the default takes where products are fp32; bell-shaped operands of both signs."""
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.templates import gfx950
+    from flextensor_amd.utils import Config
+    func = gemm_of(trans_b)
+    plan, bufs = split_plan(func, shape, *kernel)
+    monkeypatch.setattr(gfx950, "_or_split", lambda view, cfg, call: cfg)
+    other, _ = schedule_with_config_ops(*func(*shape), Config([], None))
+    spec = other.specs[-1]
+    assert "SPLIT" not in spec.defines and (kernel[0] != (1, 2, 1, 2) or kernel[2] >= 2 * spec.defines.get("WAVES_K", 1))
+    rng = np.random.default_rng(5)
+    a, b = (rng.standard_normal([int(e) for e in x.shape]).astype(np.float32) for x in bufs[:2])
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    ref = a64 @ (b64.T if trans_b else b64)
     mine, theirs = (np.linalg.norm(run(p, bufs, [a, b]) - ref) for p in (plan, other))
     assert mine < theirs
 
