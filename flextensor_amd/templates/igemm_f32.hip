@@ -1468,11 +1468,12 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
  * 3x3 16x128x57x57 -> 256 4.2e-7 and 1.5e-7, batch 96 x 197x64x197 1.4e-7 and 0.5e-7.
  *
  * The parts are those of 2^23 x, which is a multiple of 2^-126 whatever x is, so every part is zero or a normal number and
- * nothing of a small x is lost, whatever stands beside it; the sums are multiplied by 2^-46 at the end. (Parts of x itself lose bits below
- * 2^-110. To look for the largest number of a row, an instruction for two numbers less, misses a small one beside it: GEMM
- * 1024^3 16.75 us and 16.91 with the factor, 1000x1531x777 22.8 and 23.2.) Infinities, NaN and numbers from 2^105 on have no
- * such parts, their remainder is NaN, and sums from 2^82 on are infinite: every sum is looked at, and where one is no
- * finite number the workgroup does its part of K again with fp32 MFMAs, slowly, straight from memory.
+ * nothing of a small x is lost, whatever stands beside it; the sums are multiplied by 2^-46 at the end. (Parts of x itself
+ * lose bits below 2^-110. To look for the largest number of a row, an instruction for two numbers less, misses a small one
+ * beside it: GEMM 1024^3 16.75 us and 16.91 with the factor, 1000x1531x777 22.8 and 23.2.) Infinities, NaN and numbers from
+ * 2^105 on have no such parts, their remainder is NaN, and sums from 2^82 on are infinite: every sum is looked at, and
+ * where one is no finite number the workgroup does its part of K again with fp32 MFMAs (a call whose rows all hold an
+ * infinity takes 1.5 to 2.6 times an ordinary one, 1.3 to 2.5 times the kernel of fp32 products).
  *
  * What bounds it: a vector instruction and an MFMA overlap for half of the MFMA's clocks only, the split is thirteen
  * instructions for two numbers, and a wavefront writes LDS at 70 bytes a clock and unit (reads: 230). So operands are
@@ -1991,49 +1992,68 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
                 }
         if (__any(!(nan == 0.0f)) && lane == 0) redo = 1;
     }
-    __syncthreads();                    /* also the last reads of the tiles, whose LDS the sums take */
+    __syncthreads();                    /* also the last reads of the tiles, whose LDS the sums or other tiles take */
     if (redo) {
-        /* the group's k once more, undivided numbers from memory */
+        /* the group's k once more: tiles of undivided numbers, rows of 32 floats, at twice the places of their parts. A load
+         * for each number straight from memory took 3 to 9 times an ordinary call (1500x1000x3001 714 us for 81). */
         clear();
-        const int end = (first + GSTEPS) * 32 < K ? (first + GSTEPS) * 32 : K;
-        int nb[REP_N];
-#if MODE == 1
-        unsigned px[REP_N], bad[REP_N];
-#endif
+        load(first, 0);
+        for (int s = 0; s < GSTEPS; ++s) {
+            auto& ax = axs[0];
+            auto& bx = bxs[0];
+            unsigned char* const at = lds + (s & 1) * (128 * (BM + BN));
+            unsigned char* const bt = at + 128 * BM;
+            if ((first + s + 1) * 32 > K) cut(first + s, 0);
 #pragma unroll
-        for (int j = 0; j < REP_N; ++j) {
-            nb[j] = n0 + COLUMN((wn * REP_N + j) * MFMA + li);
-#if MODE == 1
-            pixel(nb[j], px[j], bad[j]);
-#endif
-        }
-#pragma unroll 4
-        for (int k0 = first * 32; k0 < end; k0 += KL) {
-            const int k = k0 + lg;
-            float a[REP_M], b[REP_N];
+            for (int e = 0; e < EA; ++e)
+                if (BM * 8 % NT == 0 || tid + e * NT < BM * 8) *reinterpret_cast<f32x4*>(at + 2 * a_lds[e]) = ax[e];
 #pragma unroll
-            for (int i = 0; i < REP_M; ++i) {
-                const int m = m0 + (wm * REP_M + i) * MFMA + li;
-                const unsigned off = (unsigned)((AGROUP(gi) * M + m) * K + k) * 4u;
-                a[i] = ld1(rsrc_a, (m < M) & (k < K) ? off : OOB, 0);
-            }
+            for (int e = 0; e < EB; ++e) {
+#if MODE == 2
+                if (BN * 8 % NT == 0 || tid + e * NT < BN * 8) *reinterpret_cast<f32x4*>(bt + 2 * b_lds[e]) = bx[e];
+#elif MODE == 0
+                if (BN / NV * 8 % NT == 0 || tid + e * NT < BN / NV * 8)
 #pragma unroll
-            for (int j = 0; j < REP_N; ++j) {
-#if MODE == 1
-                b[j] = ld1(rsrc_b, (px[j] + taps.e[2 * k]) | ((bad[j] << taps.e[2 * k + 1]) & OOB), 0);
+                    for (int j = 0; j < NV; ++j) {
+                        const f32x4 y = {bx[e][0][j], bx[e][1][j], bx[e][2][j], bx[e][3][j]};
+                        *reinterpret_cast<f32x4*>(bt + 2 * (j * 1024 + (b_lds[e] ^ (j & 1) * 16))) = y;
+                    }
 #else
-                const unsigned off = (unsigned)(MODE == 2 ? (gi * N + nb[j]) * K + k : (gi * K + k) * N + nb[j]) * 4u;
-                b[j] = ld1(rsrc_b, (nb[j] < N) & (k < K) ? off : OOB, 0);
+                if (BN * 4 % NT == 0 || tid + e * NT < BN * 4)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const f32x4 y = {bx[e][4 * h], bx[e][4 * h + 1], bx[e][4 * h + 2], bx[e][4 * h + 3]};
+                        *reinterpret_cast<f32x4*>(bt + 2 * b_lds[e] + 16 * h) = y;
+                    }
 #endif
             }
+            __syncthreads();            /* for everybody, who also has read the step before: its buffer is the next one's */
+            load(first + s + 1, 0);
 #pragma unroll
-            for (int i = 0; i < REP_M; ++i)
+            for (int t = 0; t < KH; ++t) {
+                f32x4 b[REP_N][2];
 #pragma unroll
-                for (int j = 0; j < REP_N; ++j) acc[i][j] = MFMA_OP(a[i], b[j], acc[i][j]);
+                for (int j = 0; j < REP_N; ++j)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        b[j][h] = *reinterpret_cast<const f32x4*>(bt + 2 * (j * MFMA * 64 + (b_frag[t] ^ (MFMA == 16 ? (j & 1) * 16 : 0))) + 16 * h);
+#pragma unroll
+                for (int i = 0; i < REP_M; ++i) {
+                    f32x4 a[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        a[h] = *reinterpret_cast<const f32x4*>(at + 2 * (i * MFMA * 64 + (a_frag[t] ^ (MFMA == 16 ? (i & 1) * 16 : 0))) + 16 * h);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+#pragma unroll
+                        for (int j = 0; j < REP_N; ++j) acc[i][j] = MFMA_OP(a[q / 4][q % 4], b[j][q / 4][q % 4], acc[i][j]);
+                }
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();                /* the last reads of these tiles */
     }
 
 #if WAVES_K > 1
