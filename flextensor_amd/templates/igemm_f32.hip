@@ -1644,16 +1644,22 @@ static __device__ __forceinline__ f32x4 ld4(__amdgpu_buffer_rsrc_t r, unsigned v
 }
 
 #if MODE == 1
+/* of every k: byte offset and tap. The offset is the scalar one of its loads, which must not reach beyond the buffer (see
+ * K_AT in the first kernel): one that does, the last rows of a window that is wider than the image and its padding on one side
+ * (10x10, 3x3 with dilation and padding 12), is of padding for every pixel, like a k behind K. */
 struct tap_table { unsigned e[STEPS * 64]; };
 static constexpr tap_table make_taps() {
     tap_table t = {};
     for (int k = 0; k < STEPS * 32; ++k) {
         const int c = k / (CR * CS), w = k % (CR * CS);
-        t.e[2 * k] = k < K ? (unsigned)(c * (CH * CW) + w / CS * CDILH * CW + w % CS * CDILW) * 4u : 0u;
-        t.e[2 * k + 1] = k < K ? (unsigned)w : 31u;
+        const long long off = 4ll * (c * (CH * CW) + w / CS * CDILH * CW + w % CS * CDILW);
+        const bool inside = k < K && off < 1ll * B_BYTES + PAD_BYTES;
+        t.e[2 * k] = inside ? (unsigned)off : 0u;
+        t.e[2 * k + 1] = inside ? (unsigned)w : 31u;
     }
     return t;
 }
+/* end of the table */
 static __constant__ const tap_table taps = make_taps();
 #endif
 

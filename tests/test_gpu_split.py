@@ -61,7 +61,9 @@ def test_gemm(shape, trans_b, kernel):
     # padding on every side, windows of 1 to 25 taps, strides, dilation, channel groups, a window that covers the image
     ((2, 5, 9, 7, 19, 3, 1, 1, 1, 1), True), ((1, 16, 14, 14, 33, 3, 2, 1, 1, 1), False), ((3, 37, 8, 11, 20, 1, 1, 0, 1, 1), True),
     ((2, 24, 13, 13, 24, 3, 1, 2, 2, 2), False), ((1, 3, 15, 15, 40, 5, 1, 2, 1, 1), True), ((5, 32, 3, 3, 17, 3, 1, 0, 1, 1), True),
-    ((2, 64, 7, 7, 70, 1, 2, 0, 1, 1), False), ((3, 32, 8, 8, 64, 1, 1, 0, 1, 1), False)])
+    ((2, 64, 7, 7, 70, 1, 2, 0, 1, 1), False), ((3, 32, 8, 8, 64, 1, 1, 0, 1, 1), False),
+    # windows whose last rows are padding for every pixel, and lie behind the image's end
+    ((1, 8, 5, 5, 40, 3, 1, 6, 6, 1), False), ((1, 20, 10, 10, 33, 3, 1, 12, 12, 1), True), ((1, 40, 1, 1, 70, 5, 1, 2, 1, 1), False)])
 def test_conv2d(oracle, shape, bias, kernel):
     from flextensor_amd.measure import seeded_inputs
     plan, bufs = split_plan(conv_of(bias), shape, *kernel)

@@ -207,6 +207,53 @@ def test_loads_that_a_wait_counts_are_all_there(args, tile, groups):
     assert len(found) == 4 * loads, (len(found), loads)         # before the loop and in it, split and whole products
 
 
+TAPS_CPP = """
+%s
+%s
+extern "C" const unsigned* table() { static const tap_table t = make_taps(); return t.e; }
+"""
+
+
+@pytest.mark.parametrize("image,conv", [
+    ((1, 8, 5, 5), (3, 3, 1, 6, 6)), ((1, 16, 10, 10), (3, 3, 1, 12, 12)), ((1, 40, 1, 1), (5, 5, 1, 2, 1)), ((1, 3, 4, 4), (5, 5, 1, 8, 3)),
+    ((2, 20, 13, 11), (3, 3, 1, 1, 1)), ((1, 16, 14, 14), (3, 3, 2, 1, 1)), ((3, 7, 8, 9), (1, 1, 1, 0, 1)), ((2, 5, 9, 7), (1, 7, 2, 3, 1))])
+def test_scalar_offsets_of_taps_stay_inside_the_buffer(tmp_path, image, conv):
+    """The table of igemm_f32.hip's second kernel, compiled for the host: no offset reaches beyond image and padding, where
+    the range check of the loads would wrap; entries say the tap and its offset, or 31, padding for every pixel, and
+    those are only taps that no pixel has inside the image."""
+    import ctypes
+    from flextensor_amd.templates import gfx950
+    (cb, cc, ch, cw), (cr, cs, stride, pad, dil) = image, conv
+    k = cc * cr * cs
+    text = gfx950.template_source("igemm_f32.hip")
+    body = re.search(r"(struct tap_table \{.*?)(static __constant__|/\* end of the table \*/)", text, re.S).group(1)
+    values = dict(CB=cb, CC=cc, CH=ch, CW=cw, CR=cr, CS=cs, CDILH=dil, CDILW=dil, CPADH=pad, CPADW=pad, K=k, STEPS=ceil_div(k, 32))
+    defines = ["#define %s %d" % x for x in values.items()] + re.findall(r"#define (?:PAD_BYTES|B_BYTES) .*CW.*", text[text.index("#else  /* FT_SPLIT"):])
+    assert len(defines) == len(values) + 2
+    (tmp_path / "taps.cpp").write_text(TAPS_CPP % ("\n".join(defines), body))
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-o", str(tmp_path / "taps.so"), str(tmp_path / "taps.cpp")])
+    table = ctypes.CDLL(str(tmp_path / "taps.so")).table
+    table.restype = ctypes.POINTER(ctypes.c_uint32)
+    entries = table()
+    size = 4 * (cb * cc * ch * cw + pad * cw + pad)
+
+    def some_pixel_inside(n, extent, window):
+        at = [o * stride - pad + n * dil for o in range((extent + 2 * pad - dil * (window - 1) - 1) // stride + 1)]
+        return any(0 <= x < extent for x in at)
+
+    for i in range(values["STEPS"] * 32):
+        off, tap = entries[2 * i], entries[2 * i + 1]
+        assert off < size, (i, off, size)
+        if i < k and tap != 31:
+            assert tap == i % (cr * cs)
+            assert off == 4 * (i // (cr * cs) * ch * cw + tap // cs * dil * cw + tap % cs * dil)
+        elif i < k:
+            t = i % (cr * cs)
+            assert not (some_pixel_inside(t // cs, ch, cr) and some_pixel_inside(t % cs, cw, cs))
+        else:
+            assert (off, tap) == (0, 31)
+
+
 MASKED = """k:
 \tv_cmp_ne_u32_e32 vcc, 0, v12
 \tv_mov_b32_e32 v23, 0
