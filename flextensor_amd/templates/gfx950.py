@@ -676,6 +676,11 @@ def _lower_direct(op, view, D, direct, depth, out_name, in_names, materialized_p
     return [KernelSpec("direct_f32.hip", "igemm_f32", D, (tiles * view.groups, 1, 1), (waves * 64, 1, 1), args)]
 
 
+def _gathered_bytes(conv, ahead):
+    """Bytes that the offsets of the gathered operand span: with LDS tiles (``ahead``) they count from before the padding."""
+    return 4 * (conv["CB"] * conv["CC"] * conv["CH"] * conv["CW"] + (conv["CPADH"] * conv["CW"] + conv["CPADW"] if ahead else 0))
+
+
 def _lower_split(op, view, D, depth, special, out_name, in_names, materialized_pad, bias_name, merged_out, waves_k):
     """Products in three bf16 parts (the second kernels of igemm_f32.hip and direct_f32.hip)."""
     template, ahead = SPLIT_DEPTHS[depth]
@@ -718,7 +723,7 @@ def _lower_split(op, view, D, depth, special, out_name, in_names, materialized_p
             conv["CW"] += 2 * conv["CPADW"]
             conv["CPADH"] = conv["CPADW"] = 0
         D.update(conv)
-        b_bytes = (conv["CB"] * conv["CC"] * conv["CH"] * conv["CW"] + conv["CPADH"] * conv["CW"] + conv["CPADW"]) * 4
+        b_bytes = _gathered_bytes(conv, ahead)
         if op.kind == "col_gemm" and merged_out is None:
             D.update(COLOUT=1)
     elif view.images:
@@ -1268,7 +1273,8 @@ def _or_split(view, cfg, call):
     limit, best = (call - 500) / 1.08, None
     before = cfg["reduce"][0][0]
     for m, n, mf, groups, depth in SPLIT_KERNELS:
-        if m[0] * m[1] * mf >= 2 * max(view.M, 16) or n[0] * n[1] * mf >= 2 * max(view.N, 16):
+        if m[0] * m[1] * mf >= 2 * max(view.M, 16) or n[0] * n[1] * mf >= 2 * max(view.N, 16) \
+                or view.conv and _gathered_bytes(view.conv, 1) >= 2 ** 31:
             continue
         # launch, chain of steps, and matrix clocks alone: not worth a prediction
         steps = -(-view.K // (32 * groups))

@@ -854,3 +854,17 @@ def test_k_tiles_of_whole_windows_are_for_windows_they_hold():
                     assert bk not in (72, 144) or r == 3
                     seen.add((r, bk))
     assert {bk for r, bk in seen if r == 3} & {72, 144}
+
+
+@pytest.mark.parametrize("shape", [(1, 32, 1000, 16777, 64, 5, 2, 2), (1, 64, 1000, 8388, 128, 3, 2, 1), (2, 32, 2896, 2896, 24, 5, 2, 2)])
+def test_default_of_an_image_just_below_2_gib(shape):
+    """Offsets that count from before the padding go beyond 2 GiB where those of the image do not: the default is a kernel
+    that takes the image."""
+    from flextensor_amd import nn
+    from flextensor_amd.scheduler import schedule_with_config_ops
+    from flextensor_amd.te import placeholder
+    b, c, h, w, o, r, stride, pad = shape
+    x, wt = placeholder((b, c, h, w), name="X"), placeholder((o, c, r, r), name="W")
+    y = nn.conv2d_nchw(x, wt, stride=stride, padding=pad)
+    plan, _ = schedule_with_config_ops([y.op], [x, wt, y], Config([], None))
+    assert plan.specs
