@@ -30,6 +30,8 @@ if ROOT not in sys.path:
 # published MI355X peaks (dense)
 PEAK_F32_TFLOPS = 157.3
 PEAK_I8_TOPS = 5000.0
+PEAK_BF16_TFLOPS = 2500.0
+BF16_PRODUCTS = 6       # bf16 products that make one of two fp32 numbers in three parts
 PEAK_HBM_GBS = 8000.0
 
 WORKLOADS = [
@@ -94,7 +96,9 @@ def roofline(name, bound, dtype, ops, nbytes, ms, plan, clock=None):
         out = {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                "frac": achieved / PEAK_HBM_GBS, "traffic": traffic, "traffic_provenance": prov}
     else:
-        peak = PEAK_I8_TOPS if dtype == "i8" else PEAK_F32_TFLOPS
+        # a kernel whose fp32 products are made of bf16 ones is not bound by the fp32 matrix rate
+        parts = plan.specs[-1].defines.get("SPLIT")
+        peak = PEAK_I8_TOPS if dtype == "i8" else PEAK_BF16_TFLOPS / BF16_PRODUCTS if parts else PEAK_F32_TFLOPS
         achieved = ops / (ms * 1e-3) / 1e12
         out = {"bound": "mfma", "achieved": achieved, "peak": peak,
                "unit": "TOP/s" if dtype == "i8" else "TFLOP/s", "frac": achieved / peak,

@@ -868,3 +868,16 @@ def test_default_of_an_image_just_below_2_gib(shape):
     y = nn.conv2d_nchw(x, wt, stride=stride, padding=pad)
     plan, _ = schedule_with_config_ops([y.op], [x, wt, y], Config([], None))
     assert plan.specs
+
+
+def test_roofline_of_products_in_bf16_parts():
+    """bench.py holds a kernel to the matrix rate it uses: a sixth of the bf16 one where products are made of bf16 parts."""
+    import bench
+    from flextensor_amd.tuned import lookup
+    key = "gemm_gemm_(1024, 1024, 1024)_rocm(0)"
+    parts, _ = schedule_with_config(key, lookup(key))
+    assert parts.specs[-1].defines["SPLIT"] == 1
+    whole, _ = schedule_with_config("conv2d_baseline0_(1, 64, 56, 56, 64, 3, 1, 1, 1, 1)_rocm(0)", Config([], None))
+    assert "SPLIT" not in whole.specs[-1].defines
+    peak = [bench.roofline("gemm_f32_1024", "mfma", "f32", 2 * 1024 ** 3, 12582912, 0.016, p)["peak"] for p in (parts, whole)]
+    assert peak == [2500.0 / 6, 157.3]
