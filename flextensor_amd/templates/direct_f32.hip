@@ -385,11 +385,14 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
  * need no registers on their way; B [K][N] and gathered elements are loaded by the lane that multiplies them, whole lines
  * already. Two steps of A are in LDS or on their way, of B one.
  *
- * What bounds it: thirteen vector instructions for two numbers beside an MFMA that hides two for every eight clocks of its
- * own, 2 000 clocks a step of 64 x 64 x 32 where the MFMAs are 1 536, and the operands of a 64 x 64 tile, 1 900 clocks from
- * L2. LDS tiles of several wavefronts (igemm_f32.hip) split and gather every element once, this kernel once for each
- * wavefront's tile, but a gathered tile of theirs waits for its slowest wavefront at every barrier: 3x3 8x256x14x14 -> 512
- * 39 us there and 31 here (34.9 fp32 MFMAs), 1x289x63x63 -> 90 40 and 25 (32.5); but stride 2 16x128x57x57 -> 256 52 and 67.
+ * What bounds it: thirteen vector instructions for two numbers, 1 664 clocks a step of 64 x 64 x 32 where the MFMAs are
+ * 1 536, and the operands of a 64 x 64 tile, 1 900 clocks from L2. Of GEMM 1024^3 (two wavefronts a SIMD) vector
+ * instructions and MFMAs are 16.7 k and 12.3 k clocks, the whole life of a workgroup, first loads and sums included, 29.0 k:
+ * they overlap by little. LDS tiles of several wavefronts (igemm_f32.hip) split and gather every element once, this kernel
+ * once for each wavefront's tile, but a gathered tile of theirs waits for its slowest wavefront at every barrier: us a
+ * call, best tile there and here, and the default's kernel of fp32 products, 3x3 8x256x14x14 -> 512 44.9, 32.1 and 47.0 (the
+ * shipped one, with K streaming, 34.9), 1x289x63x63 -> 90 48.6, 25.4 and 32.6; but stride 2 16x128x57x57 -> 256 56.0, 74.4 and
+ * 77.8.
  *
  * Up to two blocks a wavefront have accumulators of their own for the five small products; with four there are no registers
  * for them and every product rounds the sum, so K has to be divided by four or more: error against float64 of

@@ -540,9 +540,11 @@ void gemm_i8(const signed char* __restrict__ A, const signed char* __restrict__ 
         const int wv = __builtin_amdgcn_readfirstlane(wave);
         /* The load is written as an instruction, not through the builtin: the
          * compiler makes every later LDS read wait for a direct-to-LDS load it
-         * knows of (it cannot tell the two buffers apart), which would undo the
-         * overlap. Completion is tracked by hand: vmcnt(0) and a barrier at
-         * the end of every iteration. */
+         * knows of (it cannot tell the buffers apart), which would undo the
+         * overlap. Completion is tracked by hand. Two buffers: vmcnt(0) and a
+         * barrier at the end of every iteration. Three: a count of the loads
+         * of the tile behind and a barrier at its start, and none behind the
+         * last tile, so whatever uses the LDS next needs a barrier of its own. */
         auto descriptor = [](const signed char* base, unsigned bytes) {
             const unsigned long long p = (unsigned long long)base;
             i32x4 d;                         /* raw buffer: base, stride 0, size in bytes, untyped dwords */

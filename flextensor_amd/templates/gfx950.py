@@ -1264,7 +1264,10 @@ def _or_split(view, cfg, call):
     1x1 layers of 1 .. 16 images, 16 .. 512 channels, stride 1 and 2) and are off by 10 % (one standard deviation), like
     those of the fp32 kernels. Over these operators the picks take 0.954 times the time without them in the geometric mean
     (0.937 if every pick were the fastest), four are more than 2 % slower (10.3 us at 1.11), and all of them together 1 866
-    us for 2 149: what is long gains most.
+    us for 2 149: what is long gains most. These timings are of parts of x itself; parts of 2^23 x take the kernel of
+    direct_f32.hip 3 % longer in the mean, 5 .. 9 % with one block a wavefront. 94 operators drawn since that it changes: 0.866,
+    13 more than 2 % slower, one at 1.14 (0.852, ten and 1.10 with parts of x). With the factor in the prediction six of
+    them go back, three of which were at 0.80 .. 0.89 and two above 1, so it is left out.
     Four blocks of a wavefront on its own have one set of accumulators, which rounds 1.3 times as much as the fp32 kernels
     do with K divided alike: they are for at least twice the groups."""
     if view.trans_a or view.K < 32 or view.conv and (

@@ -1475,14 +1475,15 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
  * where one is no finite number the workgroup does its part of K again with fp32 MFMAs (a call whose rows all hold an
  * infinity takes 1.5 to 2.6 times an ordinary one, 1.3 to 2.5 times the kernel of fp32 products).
  *
- * What bounds it: a vector instruction and an MFMA overlap for half of the MFMA's clocks only, the split is thirteen
- * instructions for two numbers, and a wavefront writes LDS at 70 bytes a clock and unit (reads: 230). So operands are
+ * What bounds it: an MFMA hides two vector instructions at most (16x16x32 alone 16 clocks, with two 17, with four 25), the
+ * split is thirteen for two numbers, and a wavefront writes LDS at 70 bytes a clock and unit (reads: 230). So operands are
  * split once per workgroup, on the way from memory to LDS: a tile is three planes of bf16, rows of 32 k, read as one
  * 16-byte load per lane, part and block. Rows of A (and B^T) are loaded eight lanes a row, whole cache lines: 16 rows of
  * 64 bytes an instruction, which is what an MFMA's lanes would need, run at 15 bytes a clock and unit, eight rows of 128
  * at 44. Within a step chunk c of a row holds k = 4c .. 4c + 3 and 16 + 4c .. 19 + 4c, whichever operand.
- * Measured, LDS tiles of fp32 MFMAs and this: 3x3 stride 2 16x128x57x57 -> 256 77.7 and 52 us, GEMM 1024^3 18.5 and 16.6,
- * 1000x1531x777 27.4 and 22.9, batch 96 x 197x64x197 (B^T) 10.3 and 8.9.
+ * Measured in one lease, the default's kernel of fp32 products and the best tile of this, us a call: 3x3 stride 2
+ * 16x128x57x57 -> 256 77.8 and 56.0, GEMM 1024^3 20.8 and 17.6, 1000x1531x777 28.2 and 24.2, batch 96 x 197x64x197 (B^T)
+ * 10.6 and 9.2.
  *
  *   PD         k steps of 32 in registers, or on their way to them
  *   WAVES_K    wavefront groups that divide K, each with LDS tiles of its own, summed through LDS at the end */
