@@ -567,7 +567,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
         m0 = (first_m + rr % gsz) * BM + wm * REP_M * 32;
         n0 = (rr / gsz) * BN + wn * REP_N * 32;
     }
-    /* The wait for rows in LDS counts the loads behind them, so none may go missing: where one tile holds all columns the
+    /* The wait for rows in LDS counts the loads behind them, so none may go missing (see load_b as well): where one tile holds all columns the
      * compiler would know blocks that lie behind the last, make one load of two that both miss the buffer and drop those
      * nothing is stored from (5 columns in three blocks: 32 loads a step instead of 48, and products of what the LDS held
      * before the rows arrived). */
@@ -673,12 +673,14 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
 #if K % 32 == 0
-            const unsigned vo = b_off;
+            unsigned vo = b_off;
             const int so = (k0 + 16 * t + i) * (N * 4);
 #else
-            const unsigned vo = b_off + (unsigned)((16 * t + i) * N * 4);
+            unsigned vo = b_off + (unsigned)((16 * t + i) * N * 4);
             const int so = k0 * (N * 4);
 #endif
+            /* as many columns as a load takes: the loads of two rows are neighbours, which the compiler would make one */
+            if (N == REP_N) asm volatile("" : "+v"(vo));
 #if REP_N == 4
             const f32x4 y = ld4(rsrc_b, vo, so);
 #elif REP_N == 2

@@ -45,6 +45,7 @@ GEMM_KERNELS = [((2, 2, 4, 1), 16, 1, 9), ((4, 1, 2, 2), 16, 2, 10), ((2, 1, 2, 
     ((1, 16, 1, 16), False), ((1, 17, 33, 19), False),              # one k; K that ends inside a vector
     ((1, 130, 321, 135), False), ((1, 65, 96, 129), True),          # edges along M and N; whole steps, rows of B^T
     ((1, 70, 90, 45), True), ((1, 64, 1023, 64), False),            # groups with fewer steps than others
+    ((6, 23, 651, 1), False), ((1, 70, 330, 2), False), ((3, 100, 320, 1), False),      # rows of B of one load and less
     ((3, 40, 70, 37), False), ((2, 37, 100, 41), True),             # batches, whose rows end where the next product's begin
 ])
 def test_gemm(shape, trans_b, kernel):

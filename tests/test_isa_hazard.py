@@ -190,7 +190,10 @@ def test_k_streaming_arrivals_wait_for_the_slot_stores(tmp_path):
     ((5, 32, 3, 3, 17, 3, 1, 0, 1, 1), (1, 1, 1, 3), 4),        # five pixels: two of three blocks of columns behind the last one
     ((5, 32, 3, 3, 17, 3, 1, 0, 1, 1), (1, 1, 1, 2), 1),
     ((2, 20, 13, 11, 70, 3, 1, 1, 1, 1), (1, 2, 1, 2), 4), ((2, 64, 14, 14, 70, 1, 2, 0, 1, 1), (1, 1, 1, 1), 1),
-    ((1, 100, 150, 90), (1, 2, 1, 2), 4), ((1, 20, 300, 5), (1, 1, 1, 4), 4)])
+    ((1, 100, 150, 90), (1, 2, 1, 2), 4), ((1, 20, 300, 5), (1, 1, 1, 4), 4),
+    # a lane's loads of neighbouring rows of B are neighbours in memory: as many columns as blocks
+    ((6, 23, 651, 1), (2, 1, 1, 1), 2), ((1, 100, 320, 1), (1, 1, 1, 1), 2), ((1, 70, 330, 2), (1, 1, 1, 2), 2), ((1, 70, 320, 2), (1, 2, 1, 2), 4),
+    ((1, 70, 330, 4), (1, 1, 1, 4), 4), ((1, 70, 330, 3), (1, 1, 1, 1), 2)])
 def test_loads_that_a_wait_counts_are_all_there(args, tile, groups):
     """A wavefront of direct_f32.hip's second kernel waits for its rows in LDS by the number of loads behind them, the
     second half of a step's B: each step, both times the products can be made, has all of them, none merged with another
