@@ -567,10 +567,10 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* 
         m0 = (first_m + rr % gsz) * BM + wm * REP_M * 32;
         n0 = (rr / gsz) * BN + wn * REP_N * 32;
     }
-    /* The wait for rows in LDS counts the loads behind them, so none may go missing (see load_b as well): where one tile holds all columns the
-     * compiler would know blocks that lie behind the last, make one load of two that both miss the buffer and drop those
-     * nothing is stored from (5 columns in three blocks: 32 loads a step instead of 48, and products of what the LDS held
-     * before the rows arrived). */
+    /* The wait for rows in LDS counts the loads behind them, so none may go missing (see load_b as well): where one tile
+     * holds all columns the compiler would know blocks that lie behind the last, make one load of two that both miss the
+     * buffer and drop those nothing is stored from (5 columns in three blocks: 32 loads a step instead of 48, and products
+     * of what the LDS held before the rows arrived). */
     asm volatile("" : "+s"(n0));
 
     auto descriptor = [](const float* base, unsigned bytes) {

@@ -1481,7 +1481,7 @@ void igemm_f32(const float* __restrict__ A, const float* __restrict__ B,
  * 16-byte load per lane, part and block. Rows of A (and B^T) are loaded eight lanes a row, whole cache lines: 16 rows of
  * 64 bytes an instruction, which is what an MFMA's lanes would need, run at 15 bytes a clock and unit, eight rows of 128
  * at 44. Within a step chunk c of a row holds k = 4c .. 4c + 3 and 16 + 4c .. 19 + 4c, whichever operand.
- * Measured in one lease, the default's kernel of fp32 products and the best tile of this, us a call: 3x3 stride 2
+ * Measured side by side, the default's kernel of fp32 products and the best tile of this, us a call: 3x3 stride 2
  * 16x128x57x57 -> 256 77.8 and 56.0, GEMM 1024^3 20.8 and 17.6, 1000x1531x777 28.2 and 24.2, batch 96 x 197x64x197 (B^T)
  * 10.6 and 9.2.
  *
